@@ -6,24 +6,26 @@
 // scenes.  Each lane handles one particle; a wavefront whose particles belong
 // to several scenes runs once per distinct scene (readfirstlane loop), so the
 // scene's parameters are wave-uniform and read through the scalar cache.
+#include <type_traits>
+
 #include "fg_batch_bodies.hpp"
 #include "fg_internal.hpp"
 #include "fg_sph_fast.hpp"
 
 namespace fg {
 
-// Calls f(scene) with a wave-uniform scene index for every lane whose scene
-// is below nscenes.
+// Calls f(scene, whole) for every lane whose scene is below nscenes: with a
+// wave-uniform scene index and whole = true for a wavefront whose 64 lanes
+// are all of one scene (all but the few at the scenes' boundaries), whose
+// parameters then are scalar loads, else with each lane's own index.
 template <class F>
 __device__ __forceinline__ void for_each_scene(uint32_t sc, uint32_t nscenes, F&& f) {
-    if (sc >= nscenes) return;
-    for (;;) {
-        const uint32_t s0 = __builtin_amdgcn_readfirstlane(sc);
-        if (sc == s0) {
-            f(s0);
-            return;
-        }
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)sc);
+    if (__ballot(sc == s0 && sc < nscenes) == ~0ull) {
+        f(s0, std::true_type{});
+        return;
     }
+    if (sc < nscenes) f(sc, std::false_type{});
 }
 
 __device__ __forceinline__ GridDesc scene_grid(const fg_common_fluid_params& cp) {
@@ -49,7 +51,7 @@ __global__ void __launch_bounds__(256) k_batch_hash(const fg_scene_desc* __restr
         return;
     }
     const float4 p = pos[i];
-    for_each_scene(sc, nscenes, [&](uint32_t s) {
+    for_each_scene(sc, nscenes, [&](uint32_t s, auto whole) {
         const GridDesc g = scene_grid(scenes[s].common);
         const CellXYZ c = grid_cell(p.x, p.y, p.z, g);
         key[i] = scenes[s].keyBase + grid_linear_key(c.x, c.y, c.z, g);
@@ -117,18 +119,19 @@ __global__ void __launch_bounds__(BS)
                     unsigned long long* __restrict__ masks, uint32_t n, WorkQueue q) {
     __shared__ uint32_t s_rb[FLAT ? 9 * BS : 1];
     __shared__ uint32_t s_re[FLAT ? 9 * BS : 1];
-    __shared__ float4 s_stage[FLAT ? 1 : (BS / 64) * kStagePos];
-    float4* stage = FLAT ? nullptr : s_stage + (threadIdx.x / 64) * kStagePos;
-    FlatRanges fr{s_rb, s_re, (uint32_t)BS, (uint32_t)threadIdx.x};
+    __shared__ WaveCells s_cells[FLAT ? BS / 64 : 1];
+    __shared__ DensityStage s_stage[FLAT ? 1 : BS / 64];
+    DensityStage* stage = FLAT ? nullptr : &s_stage[threadIdx.x / 64];
+    FlatRanges fr{s_rb, s_re, (uint32_t)BS, (uint32_t)threadIdx.x, &s_cells[FLAT ? threadIdx.x / 64 : 0]};
     for_each_particle<BS, PERSIST>(q, n, [&](uint32_t i) {
-        for_each_scene(scene_of[i], nscenes, [&](uint32_t s) {
+        for_each_scene(scene_of[i], nscenes, [&](uint32_t s, auto whole) {
             const fg_scene_desc& d = scenes[s];
             if (!scene_stencil_covers_h(d.common)) {
                 rho_p[i] = make_float2(__builtin_nanf(""), __builtin_nanf(""));
                 return;
             }
             density_particle<true>(i, sp, sv, rho_p, start, end, n, d.gasConstant, d.restDensity, d.mass, d.common,
-                                   d.kernels, d.keyBase, masks, FLAT ? &fr : nullptr, stage);
+                                   d.kernels, d.keyBase, masks, FLAT ? &fr : nullptr, whole ? stage : nullptr);
         });
     });
 }
@@ -143,15 +146,16 @@ __global__ void __launch_bounds__(BS)
     __shared__ uint32_t s_rb[FLAT ? 9 * BS : 1];
     __shared__ uint32_t s_mm[FLAT ? 9 * BS : 1];
     __shared__ float4 s_stage[FLAT ? 1 : (BS / 64) * 2 * kStageRecs];
-    float4* stage = FLAT ? nullptr : s_stage + (threadIdx.x / 64) * 2 * kStageRecs;
+    float4* stage = FLAT || !q.runs ? nullptr : s_stage + (threadIdx.x / 64) * 2 * kStageRecs;
     const Contacts none{};
     FlatRows fr{s_rb, s_mm, (uint32_t)BS, (uint32_t)threadIdx.x};
     for_each_particle<BS, PERSIST>(q, n, [&](uint32_t i) {
-        for_each_scene(scene_of[i], nscenes, [&](uint32_t s) {
+        for_each_scene(scene_of[i], nscenes, [&](uint32_t s, auto whole) {
             const fg_scene_desc& d = scenes[s];
             if (!scene_stencil_covers_h(d.common)) return refuse_scene_particle(i, id, n, vout);
-            forces_particle<true>(i, sp, sv, rho_p, start, end, vout, pout, id, n, d.mass, d.viscosity, d.common,
-                                  d.kernels, d.keyBase, masks, none, FLAT ? &fr : nullptr, nullptr, stage);
+            forces_particle<true, false, false, decltype(whole)::value>(
+                i, sp, sv, rho_p, start, end, vout, pout, id, n, d.mass, d.viscosity, d.common, d.kernels, d.keyBase,
+                masks, none, FLAT ? &fr : nullptr, nullptr, whole ? stage : nullptr);
         });
     });
 }
@@ -172,28 +176,28 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(5)))
     __shared__ uint32_t s_rb[FLAT ? 9 * BS : 1];
     __shared__ uint32_t s_mm[FLAT ? 9 * BS : 1];
     __shared__ float4 s_stage[FLAT ? 1 : (BS / 64) * 2 * kStageRecs];
-    float4* stage = FLAT ? nullptr : s_stage + (threadIdx.x / 64) * 2 * kStageRecs;
+    float4* stage = FLAT || !q.runs ? nullptr : s_stage + (threadIdx.x / 64) * 2 * kStageRecs;
     FlatRows fr{s_rb, s_mm, (uint32_t)BS, (uint32_t)threadIdx.x};
     for_each_particle<BS, PERSIST>(q, n, [&](uint32_t i) {
-        for_each_scene(scene_of[i], nscenes, [&](uint32_t s) {
+        for_each_scene(scene_of[i], nscenes, [&](uint32_t s, auto whole) {
             const fg_scene_desc& d = scenes[s];
             if (!scene_stencil_covers_h(d.common)) return refuse_scene_particle(i, id, n, vout);
             Contacts c{};
             c.dyn = bodies[s].dyn;
             c.coupled = c.dyn.enabled;
-            forces_particle<true, true>(i, sp, sv, rho_p, start, end, vout, pout, id, n, d.mass, d.viscosity,
-                                        d.common, d.kernels, d.keyBase, masks, c, FLAT ? &fr : nullptr, nullptr,
-                                        stage);
+            forces_particle<true, true, false, decltype(whole)::value>(
+                i, sp, sv, rho_p, start, end, vout, pout, id, n, d.mass, d.viscosity, d.common, d.kernels, d.keyBase,
+                masks, c, FLAT ? &fr : nullptr, nullptr, whole ? stage : nullptr);
         });
     });
 }
 
 // The coupled force pass with body contact deferred (forces_particle with
 // DEFER): without the contact walk it needs fewer registers than
-// k_batch_forces_coupled.  amdgpu_waves_per_eu(7): 72 VGPRs without
-// scratch (73 and occupancy 6 without the hint; 8 waves spill to scratch).
+// k_batch_forces_coupled.  amdgpu_waves_per_eu(6): fitted to 7 waves it
+// spills 36 bytes to scratch.
 template <int BS, bool FLAT, bool PERSIST>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6)))
     k_batch_forces_deferred(const fg_scene_desc* __restrict__ scenes, uint32_t nscenes,
                             const uint32_t* __restrict__ scene_of, const float4* __restrict__ sp,
                             const float4* __restrict__ sv, const float2* __restrict__ rho_p,
@@ -204,18 +208,18 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
     __shared__ uint32_t s_rb[FLAT ? 9 * BS : 1];
     __shared__ uint32_t s_mm[FLAT ? 9 * BS : 1];
     __shared__ float4 s_stage[FLAT ? 1 : (BS / 64) * 2 * kStageRecs];
-    float4* stage = FLAT ? nullptr : s_stage + (threadIdx.x / 64) * 2 * kStageRecs;
+    float4* stage = FLAT || !q.runs ? nullptr : s_stage + (threadIdx.x / 64) * 2 * kStageRecs;
     FlatRows fr{s_rb, s_mm, (uint32_t)BS, (uint32_t)threadIdx.x};
     for_each_particle<BS, PERSIST>(q, n, [&](uint32_t i) {
-        for_each_scene(scene_of[i], nscenes, [&](uint32_t s) {
+        for_each_scene(scene_of[i], nscenes, [&](uint32_t s, auto whole) {
             const fg_scene_desc& d = scenes[s];
             if (!scene_stencil_covers_h(d.common)) return refuse_scene_particle(i, id, n, vout);
             Contacts c{};
             c.dyn = bodies[s].dyn;
             c.coupled = c.dyn.enabled;
-            forces_particle<true, true, true>(i, sp, sv, rho_p, start, end, vout, pout, id, n, d.mass, d.viscosity,
-                                              d.common, d.kernels, d.keyBase, masks, c, FLAT ? &fr : nullptr, &dc,
-                                              stage);
+            forces_particle<true, true, true, decltype(whole)::value>(
+                i, sp, sv, rho_p, start, end, vout, pout, id, n, d.mass, d.viscosity, d.common, d.kernels, d.keyBase,
+                masks, c, FLAT ? &fr : nullptr, &dc, whole ? stage : nullptr);
         });
     });
 }
@@ -241,7 +245,7 @@ __global__ void __launch_bounds__(256)
     // k is the same on every lane of a group, so a group is active or idle as a whole
     for (uint32_t k = (blockIdx.x * blockDim.x + threadIdx.x) / kContactLanes; k < cnt; k += groups) {
         const uint32_t i = dc.list[k];
-        for_each_scene(scene_of[i], nscenes, [&](uint32_t s) {
+        for_each_scene(scene_of[i], nscenes, [&](uint32_t s, auto whole) {
             const BodyContact& dyn = bodies[s].dyn;
             const float4 pos = sp[i], vel = sv[i];
             // fluid_external with the dynamic grid only: +0 + its contact sum
@@ -315,6 +319,7 @@ int batch_density(const fg_scene_desc* scenes, uint32_t nscenes, const uint32_t*
         return FG_ERR_INVALID_ARGUMENT;
     }
     if (!queue_ok(q, "fg_batch_density_nbr")) return FG_ERR_INVALID_ARGUMENT;
+    note_nbr_format(masks, n, false);
     if (state().flat_density)
         FG_BATCH_LAUNCH2(k_batch_density, true, n, q, scenes, nscenes, scene_of, (const float4*)sp, sv, rho_p,
                          (const uint32_t*)start, (const uint32_t*)end, masks, n);
@@ -337,6 +342,7 @@ int batch_forces(const fg_scene_desc* scenes, uint32_t nscenes, const uint32_t* 
         return FG_ERR_INVALID_ARGUMENT;
     }
     if (!queue_ok(q, "fg_batch_forces_integrate_nbr")) return FG_ERR_INVALID_ARGUMENT;
+    q.runs = nbr_has_runs(masks, n) ? 1u : 0u;
     if (state().flat_forces)
         FG_BATCH_LAUNCH2(k_batch_forces, true, n, q, scenes, nscenes, scene_of, (const float4*)sp, (const float4*)sv,
                          (const float2*)rho_p, (const uint32_t*)start, (const uint32_t*)end, masks, vel, pos,
@@ -359,6 +365,7 @@ int batch_forces_coupled(const fg_scene_desc* scenes, uint32_t nscenes, const ui
         return FG_ERR_INVALID_ARGUMENT;
     }
     if (!queue_ok(q, "batch_forces_coupled")) return FG_ERR_INVALID_ARGUMENT;
+    q.runs = nbr_has_runs(masks, n) ? 1u : 0u;
     if (state().flat_forces)
         FG_BATCH_LAUNCH2(k_batch_forces_coupled, true, n, q, scenes, nscenes, scene_of, (const float4*)sp,
                          (const float4*)sv, (const float2*)rho_p, (const uint32_t*)start, (const uint32_t*)end, masks,
@@ -381,6 +388,7 @@ int batch_forces_deferred(const fg_scene_desc* scenes, uint32_t nscenes, const u
         return FG_ERR_INVALID_ARGUMENT;
     }
     if (!queue_ok(q, "batch_forces_deferred")) return FG_ERR_INVALID_ARGUMENT;
+    q.runs = nbr_has_runs(masks, n) ? 1u : 0u;
     hipStream_t st = state().stream;
     launch_fill_u32(dc.count, 0u, 1, st);
     if (state().flat_forces)
@@ -423,7 +431,7 @@ int fg_batch_density_nbr(const fg_scene_desc* scenes, unsigned int numScenes, co
                          unsigned int numParticles) {
     return batch_density(scenes, numScenes, sceneOf, FG_F4(orderedPositions),
                          reinterpret_cast<const float4*>(orderedVelocity), FG_F2(mass_pressure), gridStart, gridEnd,
-                         neighborMasks, numParticles, WorkQueue{nullptr, 1});
+                         neighborMasks, numParticles, WorkQueue{nullptr, 1, 0});
 }
 
 int fg_batch_forces_integrate_nbr(const fg_scene_desc* scenes, unsigned int numScenes, const unsigned int* sceneOf,
@@ -433,7 +441,7 @@ int fg_batch_forces_integrate_nbr(const fg_scene_desc* scenes, unsigned int numS
                                   unsigned int* particleId, unsigned int numParticles) {
     return batch_forces(scenes, numScenes, sceneOf, FG_F4(orderedPositions), FG_F4(orderedVelocity),
                         FG_F2(density_pressure), gridStart, gridEnd, neighborMasks, FG_F4(vel),
-                        pos ? FG_F4(pos) : nullptr, particleId, numParticles, WorkQueue{nullptr, 1});
+                        pos ? FG_F4(pos) : nullptr, particleId, numParticles, WorkQueue{nullptr, 1, 0});
 }
 
 }  // extern "C"

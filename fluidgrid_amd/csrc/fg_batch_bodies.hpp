@@ -39,6 +39,7 @@ constexpr uint32_t kQueueStride = 16;  // one 64-byte line per counter
 struct WorkQueue {
     uint32_t* counters;
     uint32_t per_item;
+    uint32_t runs;  // (force passes) the neighbour buffer holds the wavefronts' row runs
 };
 
 // fg_batch_density_nbr / fg_batch_forces_integrate_nbr, optionally persistent.

@@ -190,12 +190,11 @@ __global__ void __launch_bounds__(BS)
                    const uint32_t* __restrict__ start,
                    const uint32_t* __restrict__ end, uint32_t n, float k, float rho0, float m,
                    fg_common_fluid_params cp, fg_kernels_cache kc, unsigned long long* __restrict__ masks) {
-    // one LDS slice of kStagePos positions per wavefront (staged row loop)
-    __shared__ float4 s_stage[(BS / 64) * kStagePos];
+    __shared__ DensityStage s_stage[BS / 64];  // one LDS slice per wavefront (staged row loop)
     const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * BS + threadIdx.x;
-    if (i >= n) return;
+    if ((i & ~63u) >= n) return;  // whole wavefronts; lanes past the last particle take part idle
     density_particle<MASKS>(i, sp, sv, rho_p, start, end, n, k, rho0, m, cp, kc, 0u, masks, nullptr,
-                            s_stage + (threadIdx.x / 64) * kStagePos);
+                            &s_stage[threadIdx.x / 64]);
 }
 
 // Flat schedule (row table in LDS); same results as k_density_fast<MASKS>.
@@ -207,32 +206,27 @@ __global__ void __launch_bounds__(BS)
                    fg_common_fluid_params cp, fg_kernels_cache kc, unsigned long long* __restrict__ masks) {
     __shared__ uint32_t s_rb[9 * BS];
     __shared__ uint32_t s_re[9 * BS];
+    __shared__ WaveCells s_cells[BS / 64];
     const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * BS + threadIdx.x;
-    if (i >= n) return;
-    FlatRanges fr{s_rb, s_re, (uint32_t)BS, (uint32_t)threadIdx.x};
+    if ((i & ~63u) >= n) return;
+    FlatRanges fr{s_rb, s_re, (uint32_t)BS, (uint32_t)threadIdx.x, &s_cells[threadIdx.x / 64]};
     density_particle<MASKS>(i, sp, sv, rho_p, start, end, n, k, rho0, m, cp, kc, 0u, masks, &fr);
 }
 
-// amdgpu_waves_per_eu(7): the masked kernels load each stencil row's cell
-// bounds and mask a row ahead (forces_rows_staged<true>), which needs about
-// 70 registers: at 8 waves per SIMD that spills to scratch and the pass is
-// 25% slower, at 7 it is 4-7% faster than the row-by-row loads at 8.  The
-// hint also holds the coupled variant, whose two body-grid descriptors take
-// scalar registers (106 SGPRs without it), to 7 waves.
 template <bool MASKS, bool COUPLED, int BS>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
     k_forces_fast(const float4* __restrict__ sp, const float4* __restrict__ sv, const float2* __restrict__ rho_p,
                   const uint32_t* __restrict__ start, const uint32_t* __restrict__ end, float4* __restrict__ vout,
                   float4* __restrict__ pout, const uint32_t* __restrict__ id, uint32_t n, float m, float mu,
                   fg_common_fluid_params cp, fg_kernels_cache kc, const unsigned long long* __restrict__ masks,
-                  Contacts bc) {
+                  Contacts bc, int runs) {
     // one LDS slice of kStageRecs neighbour records per wavefront (staged row loop)
     __shared__ float4 s_stage[MASKS ? (BS / 64) * 2 * kStageRecs : 1];
     const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * BS + threadIdx.x;
-    if (i >= n) return;
-    forces_particle<MASKS, COUPLED, false, true>(i, sp, sv, rho_p, start, end, vout, pout, id, n, m, mu, cp, kc, 0u,
-                                                 masks, bc, nullptr, nullptr,
-                                                 MASKS ? s_stage + (threadIdx.x / 64) * 2 * kStageRecs : nullptr);
+    if ((i & ~63u) >= n) return;  // whole wavefronts; lanes past the last particle take part idle
+    forces_particle<MASKS, COUPLED>(i, sp, sv, rho_p, start, end, vout, pout, id, n, m, mu, cp, kc, 0u, masks, bc,
+                                    nullptr, nullptr,
+                                    MASKS && runs ? s_stage + (threadIdx.x / 64) * 2 * kStageRecs : nullptr);
 }
 
 // Flat schedule (row table in LDS); same results as k_forces_fast<true, COUPLED>.
@@ -265,12 +259,12 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
                       const uint32_t* __restrict__ start, const uint32_t* __restrict__ end,
                       float4* __restrict__ vout, float4* __restrict__ pout, const uint32_t* __restrict__ id,
                       uint32_t n, float m, float mu, fg_common_fluid_params cp, fg_kernels_cache kc,
-                      const unsigned long long* __restrict__ masks, Contacts bc, DeferredContact dc) {
+                      const unsigned long long* __restrict__ masks, Contacts bc, DeferredContact dc, int runs) {
     __shared__ float4 s_stage[(BS / 64) * 2 * kStageRecs];
     const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * BS + threadIdx.x;
-    if (i >= n) return;
-    forces_particle<true, true, true, true>(i, sp, sv, rho_p, start, end, vout, pout, id, n, m, mu, cp, kc, 0u, masks,
-                                            bc, nullptr, &dc, s_stage + (threadIdx.x / 64) * 2 * kStageRecs);
+    if ((i & ~63u) >= n) return;
+    forces_particle<true, true, true>(i, sp, sv, rho_p, start, end, vout, pout, id, n, m, mu, cp, kc, 0u, masks,
+                                   bc, nullptr, &dc, runs ? s_stage + (threadIdx.x / 64) * 2 * kStageRecs : nullptr);
 }
 
 // Second pass of the deferred form: body contact (fluid_external: the
@@ -308,12 +302,10 @@ __global__ void __launch_bounds__(BS)
                     const uint32_t* __restrict__ start, const uint32_t* __restrict__ end, uint32_t n, float k,
                     float rho0, float m, fg_common_fluid_params cp, fg_kernels_cache kc,
                     unsigned long long* __restrict__ masks) {
-    // per wavefront: kMixedStage + 4 pair records, then kMixedStage positions
-    __shared__ float4 s_stage[(BS / 64) * (2 * kMixedStage + 4)];
+    __shared__ MixedStage s_stage[BS / 64];
     const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * BS + threadIdx.x;
-    if (i >= n) return;
-    density_particle_mixed(i, sp, sv, rho_p, start, end, n, k, rho0, m, cp, kc, masks,
-                           s_stage + (threadIdx.x / 64) * (2 * kMixedStage + 4));
+    if ((i & ~63u) >= n) return;  // whole wavefronts; lanes past the last particle take part idle
+    density_particle_mixed(i, sp, sv, rho_p, start, end, n, k, rho0, m, cp, kc, masks, s_stage[threadIdx.x / 64]);
 }
 
 // LDS-tiled passes (fg_sph_tile.hpp).  Tile b of the grid is the sorted
@@ -430,22 +422,33 @@ __global__ void __launch_bounds__(kTileLanes)
 // Launch helpers
 // ---------------------------------------------------------------------------
 
-// Which form the last density pass wrote into a neighbour buffer: lists (the
-// tiled pass) or row masks only.  The force pass follows it, whatever the
-// schedule is when it runs, so the two passes always agree on the format.
+// Which form the last density pass wrote into a neighbour buffer, and for how
+// many particles: lists (the tiled pass) or row masks with the wavefronts'
+// runs.  The force pass follows it, whatever the schedule is when it runs, so
+// the two passes always agree on the format; a buffer that no density pass of
+// this process wrote for that many particles is read by its row masks alone.
+struct NbrFormat {
+    uint32_t n;
+    bool tiled;
+};
 static std::mutex g_nbr_mu;
-static std::unordered_map<const void*, bool>& nbr_tiled() {
-    static std::unordered_map<const void*, bool> m;
+static std::unordered_map<const void*, NbrFormat>& nbr_formats() {
+    static std::unordered_map<const void*, NbrFormat> m;
     return m;
 }
-static void note_nbr_format(const void* masks, bool tiled) {
+void note_nbr_format(const void* masks, uint32_t n, bool tiled) {
     std::lock_guard<std::mutex> lock(g_nbr_mu);
-    nbr_tiled()[masks] = tiled;
+    nbr_formats()[masks] = NbrFormat{n, tiled};
 }
 static bool nbr_format_tiled(const void* masks) {
     std::lock_guard<std::mutex> lock(g_nbr_mu);
-    auto it = nbr_tiled().find(masks);
-    return it != nbr_tiled().end() && it->second;
+    auto it = nbr_formats().find(masks);
+    return it != nbr_formats().end() && it->second.tiled;
+}
+bool nbr_has_runs(const void* masks, uint32_t n) {
+    std::lock_guard<std::mutex> lock(g_nbr_mu);
+    auto it = nbr_formats().find(masks);
+    return n >= kRunMinParticles && it != nbr_formats().end() && !it->second.tiled && it->second.n == n;
 }
 // Neighbour buffers whose FP16 pair records a cell pass has written, with
 // the particle count it wrote them for (the records' place depends on it).
@@ -524,7 +527,7 @@ int launch_density(float4* sp, float2* rho_p, uint32_t* start, uint32_t* end, ui
                   "for %u particles into this neighbour buffer (fg_cell_offsets_pos_vel with neighborBuffer)", n);
         return FG_ERR_NOT_INITIALIZED;
     }
-    if (masks) note_nbr_format(masks, use_fast() && st.tiled && !mixed);
+    if (masks && use_fast()) note_nbr_format(masks, n, st.tiled && !mixed);
     if (mixed)
         FG_SPH_LAUNCH_BS(k_density_mixed<256>, 256, n, sp, sv, rho_p, start, end, n, k, rho0, m, st.common,
                          st.kernels, masks);
@@ -572,6 +575,7 @@ int launch_forces(float4* sp, float4* sv, float2* rho_p, uint32_t* start, uint32
                           st.kernels, masks, bc);
     } else if (use_fast()) {
         const unsigned long long* mk = masks;
+        const int runs = mk && nbr_has_runs(mk, n) ? 1 : 0;
         if (coupled && mk && st.defer_contact) {
             // The deferred particles' pair sums and list live in the neighbour
             // buffer's list area (used otherwise only by the tiled passes) and
@@ -584,13 +588,13 @@ int launch_forces(float4* sp, float4* sv, float2* rho_p, uint32_t* start, uint32
             launch_fill_u32(dc.count, 0u, 1, st.stream);
             switch (st.sph_block) {
                 case 64: FG_SPH_LAUNCH_BS(k_forces_deferred<64>, 64, n, sp, sv, rho_p, start, end, vout, pout, id, n,
-                                          m, mu, st.common, st.kernels, mk, bc, dc); break;
+                                          m, mu, st.common, st.kernels, mk, bc, dc, runs); break;
                 case 128: FG_SPH_LAUNCH_BS(k_forces_deferred<128>, 128, n, sp, sv, rho_p, start, end, vout, pout, id,
-                                           n, m, mu, st.common, st.kernels, mk, bc, dc); break;
+                                           n, m, mu, st.common, st.kernels, mk, bc, dc, runs); break;
                 case 512: FG_SPH_LAUNCH_BS(k_forces_deferred<512>, 512, n, sp, sv, rho_p, start, end, vout, pout, id,
-                                           n, m, mu, st.common, st.kernels, mk, bc, dc); break;
+                                           n, m, mu, st.common, st.kernels, mk, bc, dc, runs); break;
                 default: FG_SPH_LAUNCH_BS(k_forces_deferred<256>, 256, n, sp, sv, rho_p, start, end, vout, pout, id,
-                                          n, m, mu, st.common, st.kernels, mk, bc, dc);
+                                          n, m, mu, st.common, st.kernels, mk, bc, dc, runs);
             }
             // up to one lane pair per particle (the count is known only on the device)
             unsigned blocks = grid_for((uint64_t)n * kFinishLanes, 256);
@@ -599,16 +603,16 @@ int launch_forces(float4* sp, float4* sv, float2* rho_p, uint32_t* start, uint32
                                st.common, bc, dc);
         } else if (coupled && mk)
             FG_SPH_LAUNCH2(k_forces_fast, true, true, n, sp, sv, rho_p, start, end, vout, pout, id, n, m, mu,
-                           st.common, st.kernels, mk, bc);
+                           st.common, st.kernels, mk, bc, runs);
         else if (coupled)
             FG_SPH_LAUNCH2(k_forces_fast, false, true, n, sp, sv, rho_p, start, end, vout, pout, id, n, m, mu,
-                           st.common, st.kernels, mk, bc);
+                           st.common, st.kernels, mk, bc, runs);
         else if (mk)
             FG_SPH_LAUNCH2(k_forces_fast, true, false, n, sp, sv, rho_p, start, end, vout, pout, id, n, m, mu,
-                           st.common, st.kernels, mk, bc);
+                           st.common, st.kernels, mk, bc, runs);
         else
             FG_SPH_LAUNCH2(k_forces_fast, false, false, n, sp, sv, rho_p, start, end, vout, pout, id, n, m, mu,
-                           st.common, st.kernels, mk, bc);
+                           st.common, st.kernels, mk, bc, runs);
     } else if (st.key_mode == FG_KEY_LINEAR) {
         if (coupled)
             hipLaunchKernelGGL((k_forces_ref<FG_KEY_LINEAR, true>), grid, block, 0, st.stream, sp, sv, rho_p, start,

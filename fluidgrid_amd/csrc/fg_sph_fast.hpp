@@ -4,6 +4,8 @@
 //    velocity/position write-back (reference arithmetic, contraction off);
 //  * the fast LINEAR density and force passes over the 9 stencil rows.
 #pragma once
+#include <cstddef>
+
 #include "fg_contact.hpp"
 #include "fg_internal.hpp"
 #include "fg_walls.hpp"
@@ -246,6 +248,62 @@ __device__ __forceinline__ const float4* nbr_records(const unsigned long long* m
     return reinterpret_cast<const float4*>(reinterpret_cast<const char*>(masks) + nbr_record_offset(n));
 }
 
+// Then, from 256-byte boundaries, a u16 list count per particle and the lists
+// of the tiled passes (kListMax u16 per particle, in 16-byte groups).
+constexpr uint32_t kListMax = 64;
+__host__ __device__ __forceinline__ size_t nbr_align256(size_t x) { return (x + 255) & ~(size_t)255; }
+__host__ __device__ __forceinline__ size_t nbr_count_offset(uint32_t n) {
+    return nbr_align256(nbr_record_offset(n) + 2 * 16 * (size_t)n);
+}
+__host__ __device__ __forceinline__ size_t nbr_list_offset(uint32_t n) {
+    return nbr_align256(nbr_count_offset(n) + 2 * (size_t)n);
+}
+
+// The untiled passes use the list area for the deferred-contact list (its
+// first 20 bytes per particle) and, after it, for the row runs that the
+// density pass leaves for the force pass.  The lanes of a wavefront are 64
+// consecutive sorted particles, so for each stencil row the union of their
+// candidate ranges is one short run of sorted indices:
+//   runs[18 w + row]     first sorted index of wavefront w's run in the row
+//   runs[18 w + 9 + row] its length (kRunLength; 0 when no lane has the row),
+//                        with kRunWide when a lane has more than 32
+//                        candidates, and kRunGeneric when the force pass
+//                        cannot use it: a lane has more than 64 candidates,
+//                        or the density pass found no runs
+//   offs[64 (9 w + row) + lane]  the lane's first candidate, from the run's first
+// A force pass that has them looks up no cells.  Both passes agree on the
+// wavefronts: sorted particles 64 w .. 64 w + 63, all present (the last one
+// padded by inactive lanes in a single fluid).  About 19 bytes per particle,
+// which the list area holds from 64 particles on.
+constexpr uint32_t kRunWords = 18;
+constexpr uint32_t kRunLength = 0xFFFFu;
+constexpr uint32_t kRunMax = 2047u;  // longest run
+constexpr uint32_t kRunWide = 0x10000u;
+constexpr uint32_t kRunGeneric = 0x20000u;
+constexpr uint32_t kRunMinParticles = 64;
+__host__ __device__ __forceinline__ size_t nbr_runs_offset(uint32_t n) {
+    return nbr_align256(nbr_list_offset(n) + 20 * (size_t)n);
+}
+__host__ __device__ __forceinline__ size_t nbr_offs_offset(uint32_t n) {
+    return nbr_runs_offset(n) + sizeof(uint32_t) * kRunWords * (((size_t)n + 63) / 64);
+}
+__device__ __forceinline__ uint32_t* nbr_runs(unsigned long long* masks, uint32_t n) {
+    return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(masks) + nbr_runs_offset(n));
+}
+__device__ __forceinline__ const uint32_t* nbr_runs(const unsigned long long* masks, uint32_t n) {
+    return reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(masks) + nbr_runs_offset(n));
+}
+__device__ __forceinline__ uint16_t* nbr_offs(unsigned long long* masks, uint32_t n) {
+    return reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(masks) + nbr_offs_offset(n));
+}
+__device__ __forceinline__ const uint16_t* nbr_offs(const unsigned long long* masks, uint32_t n) {
+    return reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(masks) + nbr_offs_offset(n));
+}
+
+// The host's note of what a neighbour buffer holds (fg_sph.hip).
+void note_nbr_format(const void* masks, uint32_t n, bool tiled);
+bool nbr_has_runs(const void* masks, uint32_t n);
+
 // xyz of a float4 array element as one 12-byte load (the w of a neighbour
 // is not used by the pair terms).
 __device__ __forceinline__ float3 ld_xyz(const float4* p) {
@@ -253,17 +311,47 @@ __device__ __forceinline__ float3 ld_xyz(const float4* p) {
     return make_float3(f[0], f[1], f[2]);
 }
 
-// LDS staging of neighbour rows, per wavefront.  The lanes of a wavefront
-// are consecutive sorted particles, so for each of the 9 stencil rows the
-// union of their candidate ranges is one short run of sorted indices
-// [lo, hi): the wavefront loads it once, coalesced, into its own LDS slice
-// and the lanes read their candidates from there instead of gathering them
-// from memory, where the lanes of a row touch the same particles many
-// times.  A row whose run does not fit its slice is read from memory.  The
-// density pass stages positions (kStagePos float4 per wavefront), the force
-// pass neighbour records (kStageRecs records of two float4).
-constexpr uint32_t kStagePos = 256;
-constexpr uint32_t kStageRecs = 128;
+// LDS staging of neighbour rows, per wavefront: the wavefront loads each
+// stencil row's run once, coalesced, into its own LDS slice and the lanes
+// read their candidates from there instead of gathering them from memory,
+// where the lanes of a row touch the same particles many times.  The density
+// pass stages positions, kStagePos at a time, the force pass neighbour
+// records (two float4), kStageRecs at a time; a run is about 80 to 100
+// particles, more only where few particles of a wavefront lie in each cell
+// beside full ones, as in the outermost layer of a fluid.
+constexpr uint32_t kStagePos = 252;
+constexpr uint32_t kStageRecs = 160;  // 5 KB a wavefront: 32 wavefronts in a CU's LDS
+
+// The cells of a wavefront's particles (the lanes are consecutive sorted
+// particles, so about eight to twelve distinct ones in the bulk of a fluid
+// and up to 64 at its edges), and what each of the nine stencil rows holds
+// around them.  Entry (row, c) is the first sorted index B0 of cells
+// cx-1..cx+1 of the row at the c-th cell, from the row's run's first (11
+// bits), and, in 7 bits each, the distances from B0 to the end of cell cx-1,
+// the start of cell cx+1 and the end of cell cx+1 (0 in the last: the row is
+// empty there).
+struct WaveCells {
+    uint32_t row[9][64];
+    uint32_t key[64], sides[64];  // a cell's key, and kSide* of the grid around it
+    uint32_t lo[9], hi[9];        // the rows' runs
+};
+constexpr uint32_t kWaveCellsTemp = 9 * 64;  // words that wave_cells needs besides
+constexpr uint32_t kSideLowY = 1u, kSideHighY = 2u, kSideLowZ = 4u, kSideHighZ = 8u, kSideLeft = 16u,
+                   kSideRight = 32u;
+
+// A wavefront's slice in the density pass: the positions of the current run
+// as (x, y) pairs and z (the lanes of one cell read the same candidate and
+// those of the next cell one about eight further: 8- and 4-byte reads of
+// such addresses are free of bank conflicts, where 12- and 16-byte reads of
+// whole positions cost 1.5 times as much per candidate, the test and the sum
+// included: 33 against 21 SIMD cycles).
+struct DensityStage {
+    float2 xy[kStagePos + 4];
+    float z[kStagePos + 4];
+    WaveCells cells;
+    __device__ __forceinline__ uint32_t* temp() { return reinterpret_cast<uint32_t*>(xy); }
+};
+static_assert(offsetof(DensityStage, cells) >= sizeof(uint32_t) * kWaveCellsTemp, "wave_cells' temporary words");
 
 // Orders a wavefront's LDS stores before its other lanes' loads (and loads
 // before the next stores): the lanes of one wavefront need no workgroup
@@ -274,39 +362,144 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Whether one row is staged for the wavefront, and its run [lo, hi).  The
-// sorted ranges of consecutive lanes are ordered (a later lane's cell has a
-// key no lower), so the run is the start of the first lane with the row and
-// the end of the last one: two lane reads, where a min/max reduction over 64
-// lanes is six dependent cross-lane steps.  A lane whose range falls outside
-// that run sends the whole row to memory, so the result never depends on
-// the ordering.  Every lane of the wavefront must call it.
-__device__ __forceinline__ bool wave_run(bool has, uint32_t rb, uint32_t re, uint32_t cap, uint32_t& lo,
-                                         uint32_t& hi) {
-    const unsigned long long hm = __ballot(has);
-    lo = hi = 0u;
-    if (hm == 0ull) return false;
-    lo = (uint32_t)__builtin_amdgcn_readlane((int)rb, __builtin_ctzll(hm));
-    hi = (uint32_t)__builtin_amdgcn_readlane((int)re, 63 - __builtin_clzll(hm));
-    const bool inside = !has || (rb >= lo && re <= hi);
-    return __ballot(!inside) == 0ull && hi - lo <= cap;
+// The runs of a wavefront's nine rows: row r's first index and length word
+// (as in the runs table), in lane r.
+struct WaveRuns {
+    uint32_t lo = 0u, info = 0u;
+    __device__ __forceinline__ uint32_t first(int row) const {
+        return (uint32_t)__builtin_amdgcn_readlane((int)lo, row);
+    }
+    __device__ __forceinline__ uint32_t word(int row) const {
+        return (uint32_t)__builtin_amdgcn_readlane((int)info, row);
+    }
+};
+
+// Fills wc for the wavefront (every lane calls it) and gives each lane the
+// index of its cell there, and the wavefront its runs: row r's run goes from
+// the smallest B0 to the largest end of the row's entries.  False, and
+// nothing of use, when a run is longer than kRunMax or three cells hold more
+// than 127 particles; the caller then reads the rows from memory.
+// `temp`: nine times 64 words of LDS, `stride` words apart, free again afterwards.
+//
+// The nine rows of the cells are looked up by (cell, row) pairs, a pair a
+// lane and two a round: one round of twelve loads for the 64 particles in the
+// bulk of a fluid, where every lane looking up its own nine rows takes 54
+// loads of addresses that mostly coincide.
+__device__ __forceinline__ bool wave_cells(WaveCells& wc, uint32_t* __restrict__ temp, uint32_t stride, const RowWalker& w,
+                                           const fg_common_fluid_params& cp, uint32_t key_base,
+                                           const uint32_t* __restrict__ start, const uint32_t* __restrict__ end,
+                                           uint32_t n, uint32_t& cell, WaveRuns& runs) {
+    const uint32_t lane = __lane_id();
+    const uint32_t key = key_base + linear_key(w.cx, w.cy, w.cz, cp);
+    const uint32_t before = (uint32_t)__shfl_up((int)key, 1);
+    const bool head = lane == 0u || key != before;
+    const uint64_t heads = __ballot(head);
+    const uint32_t pairs = 9u * (uint32_t)__popcll(heads);
+    cell = __builtin_amdgcn_mbcnt_hi((uint32_t)(heads >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)heads, 0u)) -
+           (head ? 0u : 1u);
+    if (head) {
+        wc.key[cell] = key;
+        wc.sides[cell] = (w.cy > 0 ? kSideLowY : 0u) | (w.cy + 1 < cp.bucket_size.y ? kSideHighY : 0u) |
+                         (w.cz > 0 ? kSideLowZ : 0u) | (w.cz + 1 < cp.bucket_size.z ? kSideHighZ : 0u) |
+                         (w.cx > 0 ? kSideLeft : 0u) | (w.cx + 1 < cp.bucket_size.x ? kSideRight : 0u);
+    }
+    if (lane < 9u) {
+        wc.lo[lane] = kEmpty;
+        wc.hi[lane] = 0u;
+    }
+    wave_lds_sync();
+    const uint32_t by = (uint32_t)cp.bucket_size.x, bz = by * (uint32_t)cp.bucket_size.y;
+    bool bad = false;
+    for (uint32_t q0 = lane; q0 < pairs; q0 += 128u) {
+        uint32_t s[2][3], e[2][3];
+        bool valid[2];
+#pragma unroll
+        for (uint32_t u = 0; u < 2u; u++) {
+            const uint32_t q = q0 + 64u * u < pairs ? q0 + 64u * u : q0;  // (the second may be the first again)
+            const uint32_t c = q / 9u, row = q - 9u * c, z3 = row / 3u, y3 = row - 3u * z3;  // dy + 1, dz + 1
+            const uint32_t k = wc.key[c], sides = wc.sides[c];
+            const uint32_t need = (y3 == 0u ? kSideLowY : 0u) | (y3 == 2u ? kSideHighY : 0u) |
+                                  (z3 == 0u ? kSideLowZ : 0u) | (z3 == 2u ? kSideHighZ : 0u);
+            const bool left = (sides & kSideLeft) != 0u, right = (sides & kSideRight) != 0u;
+            valid[u] = (sides & need) == need;
+            // (a row outside the grid reads the cell's own)
+            const uint32_t m = valid[u] ? k + y3 * by + z3 * bz - (by + bz) : k;
+            const uint32_t l = left ? m - 1u : m, r = right ? m + 1u : m;
+            s[u][0] = start[l];
+            s[u][1] = start[m];
+            s[u][2] = start[r];
+            e[u][0] = end[l];
+            e[u][1] = end[m];
+            e[u][2] = end[r];
+            if (!left) s[u][0] = kEmpty;
+            if (!right) s[u][2] = kEmpty;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 2u; u++) {
+            const uint32_t q = q0 + 64u * u < pairs ? q0 + 64u * u : q0;
+            const uint32_t c = q / 9u, row = q - 9u * c;
+            // an empty cell's start is the largest value, its end is stale
+            const uint32_t e0 = s[u][0] != kEmpty ? min(e[u][0], n) : 0u, e1 = s[u][1] != kEmpty ? min(e[u][1], n) : 0u;
+            const uint32_t e2 = s[u][2] != kEmpty ? min(e[u][2], n) : 0u;
+            const uint32_t b0 = min(min(s[u][0], s[u][1]), s[u][2]), b3 = max(max(e0, e1), e2);
+            uint32_t d = 0u;
+            if (valid[u] && b0 < b3) {
+                const uint32_t d1 = s[u][0] != kEmpty ? e0 - b0 : 0u, d2 = s[u][2] != kEmpty ? s[u][2] - b0 : b3 - b0;
+                bad |= b3 - b0 > 127u;
+                d = ((d1 & 127u) << 11) | ((d2 & 127u) << 18) | ((b3 - b0) << 25);
+                atomicMin(&wc.lo[row], b0);
+                atomicMax(&wc.hi[row], b3);
+            }
+            wc.row[row][c] = b0;
+            temp[stride * row + c] = d;
+        }
+    }
+    wave_lds_sync();
+    for (uint32_t q = lane; q < pairs; q += 64u) {  // the first indices from the runs' firsts
+        const uint32_t c = q / 9u, row = q - 9u * c, d = temp[stride * row + c];
+        wc.row[row][c] = d ? ((wc.row[row][c] - wc.lo[row]) & kRunMax) | d : 0u;
+    }
+    uint32_t len = 0u;
+    if (lane < 9u && wc.hi[lane] != 0u) {
+        runs.lo = wc.lo[lane];
+        len = wc.hi[lane] - runs.lo;
+    }
+    runs.info = len;
+    wave_lds_sync();
+    return __ballot(bad || len > kRunMax) == 0ull;
 }
 
-// The same run as a min/max reduction over the 64 lanes (six dependent
-// cross-lane steps, no lane order assumed).  The force pass uses it: with
-// the two lane reads above it measured 7% slower (0.88 against 0.82 ms at
-// 8,388,608 particles, same bits), and at 8 waves per SIMD they also cost a
-// register spill reloaded at every row.
-__device__ __forceinline__ bool wave_run_minmax(bool has, uint32_t rb, uint32_t re, uint32_t cap, uint32_t& lo,
-                                                uint32_t& hi) {
-    lo = has ? rb : 0xFFFFFFFFu;
-    hi = has ? re : 0u;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        lo = min(lo, (uint32_t)__shfl_xor((int)lo, o));
-        hi = max(hi, (uint32_t)__shfl_xor((int)hi, o));
+// A lane's range in a row, from its run's first index: the row's cells after
+// culling by distance (row_keys).
+struct LaneRow {
+    uint32_t off, len;  // len 0: no candidates
+};
+__device__ __forceinline__ LaneRow lane_row(const WaveCells& wc, int row, uint32_t cell, bool active,
+                                            const RowWalker& w, float cut) {
+    const int dz = row / 3 - 1, dy = row % 3 - 1;
+    const float gy = dy < 0 ? w.gy_lo : (dy > 0 ? w.gy_hi : 0.0f);
+    const float gz = dz < 0 ? w.gz_lo : (dz > 0 ? w.gz_hi : 0.0f);
+    const float gyz = gy + gz;
+    const uint32_t c = wc.row[row][cell];
+    const uint32_t first = gyz + w.gx_lo < cut ? 0u : (c >> 11) & 127u;
+    const uint32_t last = gyz + w.gx_hi < cut ? c >> 25 : (c >> 18) & 127u;
+    return LaneRow{(c & kRunMax) + first, active && gyz < cut && last > first ? last - first : 0u};
+}
+
+// A run's length word, from its length and the lanes' candidates in it.
+__device__ __forceinline__ uint32_t run_word(uint32_t run, uint32_t len) {
+    if (__ballot(len > 32u) != 0ull) run |= kRunWide;
+    if (__ballot(len > kRowMaskBits) != 0ull) run |= kRunGeneric;
+    return run;
+}
+
+// Wavefront w's runs and its lanes' offsets (off(row)), for the force pass.
+__device__ __forceinline__ void store_runs(const WaveRuns& runs, uint32_t w, unsigned long long* masks, uint32_t n) {
+    if (__lane_id() < 9u) {
+        uint32_t* t = nbr_runs(masks, n) + (size_t)kRunWords * w + __lane_id();
+        t[0] = runs.lo;
+        t[9] = runs.info;
     }
-    return hi > lo && hi - lo <= cap;
 }
 
 // Poly6 sum over four candidates; bit u of the returned nibble is set when
@@ -357,32 +550,23 @@ __device__ __forceinline__ float3 ld_xyz_lds(const float4* p) {
     return make_float3(q.x, q.y, q.z);
 }
 
-// One stencil row of the density pass: the len candidates src[0, len) in
-// groups of four in sorted order (a short last group padded with far
-// points) added to acc, and the row's mask (0 for rows longer than 64
-// candidates, which are never read through their mask).  src is the sorted
-// positions from the row's first particle, in memory or (LDS) staged.
-template <bool MASKS, bool LDS>
+// One stencil row of the density pass: the len candidates pp[0, len) of the
+// sorted positions, in groups of four in sorted order (a short last group
+// padded with far points) added to acc, and the row's mask (0 for rows
+// longer than 64 candidates, which are never read through their mask).
+template <bool MASKS>
 __device__ __forceinline__ unsigned long long density_row(const float4& p, const float4* __restrict__ pp,
                                                           uint32_t len, float h2u, float hhu, float& acc) {
-    auto ld = [](const float4* q) { return LDS ? ld_xyz_lds(q) : ld_xyz(q); };
     unsigned long long msk = 0ull;
     const uint32_t n4 = len & ~3u;
     uint32_t kk = 0;
-    if (LDS) {
-        // From LDS the loads return quickly: no pipelining, whose register
-        // copies cost a quarter of the loop's instructions.
-        for (; kk < n4; kk += 4, pp += 4) {
-            const uint32_t nib = density4(p, ld(pp), ld(pp + 1), ld(pp + 2), ld(pp + 3), h2u, hhu, acc);
-            if (MASKS) msk |= (unsigned long long)nib << (kk & 63u);
-        }
-    } else if (n4) {
+    if (n4) {
         // Software-pipelined groups of four: the next group's loads are
         // in flight while the current group is evaluated.
-        float3 a0 = ld(pp), a1 = ld(pp + 1), a2 = ld(pp + 2), a3 = ld(pp + 3);
+        float3 a0 = ld_xyz(pp), a1 = ld_xyz(pp + 1), a2 = ld_xyz(pp + 2), a3 = ld_xyz(pp + 3);
         for (; kk + 4 < n4; kk += 4) {
             pp += 4;
-            const float3 b0 = ld(pp), b1 = ld(pp + 1), b2 = ld(pp + 2), b3 = ld(pp + 3);
+            const float3 b0 = ld_xyz(pp), b1 = ld_xyz(pp + 1), b2 = ld_xyz(pp + 2), b3 = ld_xyz(pp + 3);
             const uint32_t nib = density4(p, a0, a1, a2, a3, h2u, hhu, acc);
             if (MASKS) msk |= (unsigned long long)nib << (kk & 63u);
             a0 = b0; a1 = b1; a2 = b2; a3 = b3;
@@ -395,56 +579,211 @@ __device__ __forceinline__ unsigned long long density_row(const float4& p, const
     if (kk < len) {  // 1-3 remaining candidates; the others are masked out
         const uint32_t rest = len - kk;
         const float3 far = make_float3(3.0e38f, 3.0e38f, 3.0e38f);
-        const float3 t0 = ld(pp);
-        const float3 t1 = rest > 1 ? ld(pp + 1) : far;
-        const float3 t2 = rest > 2 ? ld(pp + 2) : far;
+        const float3 t0 = ld_xyz(pp);
+        const float3 t1 = rest > 1 ? ld_xyz(pp + 1) : far;
+        const float3 t2 = rest > 2 ? ld_xyz(pp + 2) : far;
         const uint32_t nib = density4(p, t0, t1, t2, far, h2u, hhu, acc);
         if (MASKS) msk |= (unsigned long long)nib << (kk & 63u);
     }
     return len <= kRowMaskBits ? msk : 0ull;
 }
 
-// The row loop of the density pass with each row's candidate positions
-// staged in the wavefront's LDS slice `stage` (kStagePos positions), for a
-// whole wavefront (every lane present; a lane of an inactive particle takes
-// part with no rows and writes no masks).  Same candidates, same order,
-// same sums and masks as the row loop of density_particle.
+// density4 on four candidates of the staged run, with the same operations, a
+// miss adding +0 (acc starts at +0 and never becomes -0, so that changes no
+// bit), and the hit bits shifted into `bits` from below, the first candidate
+// first.  Candidates from `rest` on are no hits.
+//
+// SAME: h2u and hhu are the same value (always so at simulation scale 1), and
+// no r2 is NaN (stage_finite, own_finite).  Then h2u - r2 is positive exactly
+// for the hits, the sum takes its positive part, and the hit bit is the sign
+// of r2 - hhu: 11 instructions a candidate.
+// Otherwise the compares, selects and shifts are written out: as selects of 0
+// and 1 the mask would cost two instructions a candidate more.  A compare's
+// result is read three instructions after it at the earliest (two must lie
+// between).
+#pragma clang fp contract(off)
+template <bool SAME, bool ALL>
+__device__ __forceinline__ void density_group(const float4& p, const float2* __restrict__ xy,
+                                              const float* __restrict__ z, uint32_t rest, float h2u, float hhu,
+                                              float& acc, uint32_t& bits) {
+    float r2[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const float dx = p.x - xy[u].x, dy = p.y - xy[u].y, dz = p.z - z[u];
+        r2[u] = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+    }
+    if constexpr (SAME) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            float d = r2[u] - hhu;
+            if (!ALL && u > 0u) d = u < rest ? d : 1.0f;
+            bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d), 31);
+            const float t = __builtin_fmaxf(-d, 0.0f);
+            acc = __builtin_fmaf(t * t, t, acc);
+        }
+        return;
+    }
+    float t[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) t[u] = h2u - r2[u];
+    const float l1 = ALL || rest > 1u ? hhu : -1.0f, l2 = ALL || rest > 2u ? hhu : -1.0f;
+    const float l3 = ALL ? hhu : -1.0f;
+    uint64_t c0, c1, c2, c3;
+    asm("v_cmp_lt_f32_e64 %[c0], %[a0], %[m0]\n\t"
+        "v_cmp_lt_f32_e64 %[c1], %[a1], %[m1]\n\t"
+        "v_cmp_lt_f32_e64 %[c2], %[a2], %[m2]\n\t"
+        "v_cmp_lt_f32_e64 %[c3], %[a3], %[m3]\n\t"
+        "v_cndmask_b32_e64 %[t0], 0, %[t0], %[c0]\n\t"
+        "v_addc_co_u32_e64 %[b], vcc, %[b], %[b], %[c0]\n\t"
+        "v_cndmask_b32_e64 %[t1], 0, %[t1], %[c1]\n\t"
+        "v_addc_co_u32_e64 %[b], vcc, %[b], %[b], %[c1]\n\t"
+        "v_cndmask_b32_e64 %[t2], 0, %[t2], %[c2]\n\t"
+        "v_addc_co_u32_e64 %[b], vcc, %[b], %[b], %[c2]\n\t"
+        "v_cndmask_b32_e64 %[t3], 0, %[t3], %[c3]\n\t"
+        "v_addc_co_u32_e64 %[b], vcc, %[b], %[b], %[c3]"
+        : [c0] "=&s"(c0), [c1] "=&s"(c1), [c2] "=&s"(c2), [c3] "=&s"(c3), [t0] "+&v"(t[0]), [t1] "+&v"(t[1]),
+          [t2] "+&v"(t[2]), [t3] "+&v"(t[3]), [b] "+&v"(bits)
+        : [a0] "v"(r2[0]), [a1] "v"(r2[1]), [a2] "v"(r2[2]), [a3] "v"(r2[3]), [m0] "v"(hhu), [m1] "v"(l1),
+          [m2] "v"(l2), [m3] "v"(l3)
+        : "vcc");
+#pragma unroll
+    for (int u = 0; u < 4; u++) acc = __builtin_fmaf(t[u] * t[u], t[u], acc);
+}
+#pragma clang fp contract(fast)
+
+// A coordinate as it is staged, and a particle's own position: a NaN or an
+// infinity becomes a value that no hit can come of (the staged ones stay
+// within 3e38, the own x beyond them), and r2 is never NaN.
+__device__ __forceinline__ float stage_finite(float v) { return __builtin_amdgcn_fmed3f(v, -3.0e38f, 3.0e38f); }
+__device__ __forceinline__ float4 own_finite(float4 p) {
+    if (!(fabsf(p.x) <= 3.0e38f && fabsf(p.y) <= 3.0e38f && fabsf(p.z) <= 3.0e38f))
+        return make_float4(3.4e38f, 0.0f, 0.0f, p.w);
+    return p;
+}
+
+// Part of a stencil row of the density pass from the staged run: cnt
+// candidates from slice index `at`, the first one bit `bit` of the row's mask.
+template <bool MASKS, bool SAME>
+__device__ __forceinline__ void density_row_staged(const float4& p, const DensityStage& st, uint32_t at, uint32_t cnt,
+                                                   uint32_t bit, float h2u, float hhu, float& acc,
+                                                   unsigned long long& mask) {
+    for (;;) {  // a row rarely has more than 32 candidates
+        const uint32_t c = min(cnt, 32u);
+        const float2* xy = st.xy + at;
+        const float* z = st.z + at;
+        uint32_t bits = 0u, k = 0u;
+        for (; k + 4u <= c; k += 4u) density_group<SAME, true>(p, xy + k, z + k, 4u, h2u, hhu, acc, bits);
+        if (k < c) {  // up to three more; what lies past them in the slice is no hit
+            density_group<SAME, false>(p, xy + k, z + k, c - k, h2u, hhu, acc, bits);
+            k += 4u;
+        }
+        // candidate j was shifted in as bit k - 1 - j
+        if (MASKS) mask |= (unsigned long long)(__builtin_bitreverse32(bits) >> (32u - k)) << (bit & 63u);
+        if (cnt <= 32u) break;
+        cnt -= 32u;
+        at += 32u;
+        bit += 32u;
+    }
+}
+
+// The row loop of the density pass for a whole wavefront (every lane present;
+// a lane of an inactive particle, or one past the last particle, takes part
+// with no rows and writes no masks): each row's run staged in the wavefront's
+// LDS slice, the next row's positions loaded into registers while this row
+// is walked.  Same candidates, same order, same sums and masks as the row
+// loop of density_particle.  False when the wavefront has no usable runs
+// (wave_cells): nothing is summed then.
+//
+// Bound by VALU issue: about 4,700 instructions a wavefront, 3,800 of them in
+// the walks (65 groups of four candidates, which its longest lane per row
+// sets); 8,388,608 particles take 702 us against 767 with per-lane lookups
+// row by row and whole positions in LDS, 1,048,576 take 104 against 111.
 template <bool MASKS>
-__device__ __forceinline__ float density_rows_staged(uint32_t i, bool active, const float4& p,
-                                                     const float4* __restrict__ sp,
-                                                     const uint32_t* __restrict__ start,
-                                                     const uint32_t* __restrict__ end, uint32_t n,
-                                                     const fg_common_fluid_params& cp, uint32_t key_base,
-                                                     unsigned long long* __restrict__ masks,
-                                                     float4* __restrict__ stage) {
+__device__ __forceinline__ bool density_rows_staged(uint32_t i, bool active, const float4& p,
+                                                    const float4* __restrict__ sp,
+                                                    const uint32_t* __restrict__ start,
+                                                    const uint32_t* __restrict__ end, uint32_t n,
+                                                    const fg_common_fluid_params& cp, uint32_t key_base,
+                                                    unsigned long long* __restrict__ masks, DensityStage& st,
+                                                    float& sum) {
     const float s = cp.simulation_scale, s2 = s * s;
     const float h = cp.kernel_radius, hh = h * h;
     const float hu = h / s, hhu = hu * hu, h2u = cp.kernel_radius_squared / s2;
     const float cut = hh * 1.0001f;
+    const uint32_t lane = __lane_id();
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(i >> 6);
+    const bool table = MASKS && n >= kRunMinParticles;
     const RowWalker w = make_rows(p, cp);
-    float acc = 0.0f;
-    // The next row's cell bounds are loaded a row ahead, after this row's
-    // staging loads, so they arrive while this row is walked.
-    RowFetch next = active ? row_fetch(w, -1, -1, cut, cp, key_base, start, end) : RowFetch{kEmpty, kEmpty, 0u, false};
-    for (int row = 0; row < 9; row++) {
-        const int dz = row / 3 - 1, dy = row % 3 - 1;
-        const RowFetch f = next;
-        uint32_t rb = 0, re = 0;
-        const bool has = active && row_finish(f, w, dy, dz, cut, cp, key_base, start, end, n, rb, re);
-        uint32_t lo, hi;
-        const bool staged = wave_run(has, rb, re, kStagePos, lo, hi);  // the same on every lane
-        if (staged)
-            for (uint32_t k = __lane_id(); k < hi - lo; k += 64u) stage[k] = sp[lo + k];
-        if (row < 8 && active) next = row_fetch(w, (row + 1) % 3 - 1, (row + 1) / 3 - 1, cut, cp, key_base, start, end);
-        if (staged) wave_lds_sync();
-        unsigned long long msk = 0ull;
-        if (has)
-            msk = staged ? density_row<MASKS, true>(p, stage + (rb - lo), re - rb, h2u, hhu, acc)
-                         : density_row<MASKS, false>(p, sp + rb, re - rb, h2u, hhu, acc);
-        if (MASKS && active) masks[(size_t)row * n + i] = msk;
-        if (staged) wave_lds_sync();  // every lane's reads of this row before the next row's stores
+    uint32_t cell;
+    WaveRuns runs;
+    if (!wave_cells(st.cells, st.temp(), 64u, w, cp, key_base, start, end, n, cell, runs)) {
+        runs.info = kRunGeneric;
+        if (table) store_runs(runs, wave, masks, n);
+        return false;
     }
-    return acc;
+    const bool same = __builtin_amdgcn_readfirstlane(__float_as_uint(h2u) == __float_as_uint(hhu) ? 1u : 0u) != 0u;
+    const float4 own = own_finite(p);
+    uint16_t* offs = MASKS ? nbr_offs(masks, n) + (size_t)9 * 64 * wave + lane : nullptr;
+    uint32_t words = 0u;
+    unsigned long long msk = 0ull, last = 0ull;
+    float acc = 0.0f;
+    float3 n0 = make_float3(0.0f, 0.0f, 0.0f), n1 = n0;
+    auto fetch = [&](int row) {
+        const uint32_t len = runs.word(row);
+        const float4* q = sp + runs.first(row) + lane;
+        if (lane < len) n0 = ld_xyz(q);
+        if (lane + 64u < len) n1 = ld_xyz(q + 64);
+    };
+    auto put = [&](uint32_t k, const float3& q) {
+        st.xy[k] = make_float2(stage_finite(q.x), stage_finite(q.y));
+        st.z[k] = stage_finite(q.z);
+    };
+    fetch(0);
+    for (int row = 0; row < 9; row++) {
+        const uint32_t len = runs.word(row), lo = runs.first(row);  // the same on every lane
+        const LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
+        if (table) {
+            const uint32_t word = run_word(len, r.len);
+            words = (int)lane == row ? word : words;
+        }
+        msk = 0ull;
+        // the lane's candidates among the staged positions [at, at + kStagePos) of the run
+        auto walk = [&](uint32_t at) {
+            const uint32_t a = max(r.off, at), b = min(r.off + r.len, at + kStagePos);
+            if (a < b) {
+                if (same) density_row_staged<MASKS, true>(own, st, a - at, b - a, a - r.off, h2u, hhu, acc, msk);
+                else density_row_staged<MASKS, false>(own, st, a - at, b - a, a - r.off, h2u, hhu, acc, msk);
+            }
+        };
+        for (uint32_t at = 0u;;) {  // (a run rarely fills the slice)
+            const uint32_t cnt = min(len - at, kStagePos);
+            if (at == 0u) {
+                if (lane < cnt) put(lane, n0);
+                if (lane + 64u < cnt) put(lane + 64u, n1);
+                // The last row's mask and this row's offsets are stored
+                // before the next row's loads are issued: loads and stores
+                // are waited for together, and a store issued after the
+                // walk would hold up the next row's positions.
+                if (MASKS && active && row > 0) masks[(size_t)(row - 1) * n + i] = last;
+                if (table) offs[64 * row] = (uint16_t)r.off;
+                if (row < 8) fetch(row + 1);
+            }
+            for (uint32_t k = lane + (at == 0u ? 128u : 0u); k < cnt; k += 64u) put(k, ld_xyz(sp + lo + at + k));
+            wave_lds_sync();
+            walk(at);
+            wave_lds_sync();  // every lane's reads before the next stores
+            at += kStagePos;
+            if (at >= len) break;
+        }
+        last = r.len <= kRowMaskBits ? msk : 0ull;
+    }
+    if (MASKS && active) masks[(size_t)8 * n + i] = last;
+    if (table) {
+        runs.info = words;
+        store_runs(runs, wave, masks, n);
+    }
+    sum = acc;
+    return true;
 }
 
 // Per-lane row table of the flat density schedule, in LDS: first and
@@ -453,6 +792,7 @@ struct FlatRanges {
     uint32_t* rb;  // [9][lanes]
     uint32_t* re;  // [9][lanes]
     uint32_t lanes, lane;
+    WaveCells* cells;  // the wavefront's
     __device__ __forceinline__ uint32_t& b(int r) { return rb[r * lanes + lane]; }
     __device__ __forceinline__ uint32_t& e(int r) { return re[r * lanes + lane]; }
 };
@@ -466,8 +806,9 @@ struct FlatRanges {
 // points): the row loop, where a wavefront waits at every row for its lane
 // with the longest row, and the flat schedule (with a row table), where each
 // lane walks its own candidate stream across rows.  Given an LDS slice
-// (`stage`) and a full wavefront, the row loop reads each row's candidates
-// from LDS (density_rows_staged).
+// (`stage`) and a whole wavefront, the row loop reads each row's candidates
+// from LDS (density_rows_staged).  A whole wavefront may call it with
+// i >= n on its last lanes, which then only take part.
 template <bool MASKS>
 __device__ __forceinline__ void density_particle(uint32_t i, const float4* __restrict__ sp,
                                                  const float4* __restrict__ sv, float2* __restrict__ rho_p, const uint32_t* __restrict__ start,
@@ -475,23 +816,47 @@ __device__ __forceinline__ void density_particle(uint32_t i, const float4* __res
                                                  float m, const fg_common_fluid_params& cp,
                                                  const fg_kernels_cache& kc, uint32_t key_base,
                                                  unsigned long long* __restrict__ masks,
-                                                 FlatRanges* flat = nullptr, float4* __restrict__ stage = nullptr) {
-    const float4 p = sp[i];
+                                                 FlatRanges* flat = nullptr, DensityStage* stage = nullptr) {
+    const bool valid = i < n;
+    const float4 p = sp[min(i, n - 1u)];
     float4* rec = MASKS ? nbr_records(masks, n) : nullptr;
-    const float4 v = MASKS ? sv[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    // The staged row loop needs every lane of the wavefront (the run of each
-    // row is a wavefront reduction); otherwise the rows are read from memory.
-    if (stage != nullptr && flat == nullptr && __ballot(1) == ~0ull) {
-        const bool active = p.w > 0.0f;
-        const float acc = density_rows_staged<MASKS>(i, active, p, sp, start, end, n, cp, key_base, masks, stage);
-        if (active) {
+    // The staged row loop needs every lane of the wavefront (a row's run is
+    // its lanes' together); otherwise the rows are read from memory.
+    const bool whole = __ballot(1) == ~0ull;
+    float sum = 0.0f;
+    if (stage != nullptr && flat == nullptr && whole &&
+        density_rows_staged<MASKS>(i, valid && p.w > 0.0f, p, sp, start, end, n, cp, key_base, masks, *stage, sum)) {
+        if (!valid) return;
+        const float4 v = MASKS ? sv[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (p.w > 0.0f) {
             const float s2 = cp.simulation_scale * cp.simulation_scale;
-            store_density(i, m * kc.kPoly6 * (s2 * s2 * s2) * acc, k, rho0, rho_p, rec, p, v);
+            store_density(i, m * kc.kPoly6 * (s2 * s2 * s2) * sum, k, rho0, rho_p, rec, p, v);
         } else if (MASKS) {
             store_record(i, rho_p[i], p, v, rec);
         }
         return;
     }
+    if (flat && whole && MASKS && n >= kRunMinParticles) {
+        // the runs for a force pass that walks rows
+        const RowWalker w = make_rows(p, cp);
+        const float cut = cp.kernel_radius * cp.kernel_radius * 1.0001f;
+        const uint32_t wave = __builtin_amdgcn_readfirstlane(i >> 6);
+        uint32_t cell, words = kRunGeneric;
+        WaveRuns runs;
+        if (wave_cells(*flat->cells, flat->rb + (flat->lane & ~63u), flat->lanes, w, cp, key_base, start, end, n, cell, runs)) {
+            uint16_t* offs = nbr_offs(masks, n) + (size_t)9 * 64 * wave + __lane_id();
+            for (int row = 0; row < 9; row++) {
+                const LaneRow r = lane_row(*flat->cells, row, cell, valid && p.w > 0.0f, w, cut);
+                offs[64 * row] = (uint16_t)r.off;
+                const uint32_t word = run_word(runs.word(row), r.len);
+                words = (int)__lane_id() == row ? word : words;
+            }
+        }
+        runs.info = words;
+        store_runs(runs, wave, masks, n);
+    }
+    if (!valid) return;
+    const float4 v = MASKS ? sv[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (!(p.w > 0.0f)) {
         // (rho, p) is left as it is; neighbours still read it
         if (MASKS) store_record(i, rho_p[i], p, v, rec);
@@ -520,7 +885,7 @@ __device__ __forceinline__ void density_particle(uint32_t i, const float4* __res
         unsigned long long msk = 0ull;
         for (;;) {
             while (j >= re) {
-                if (MASKS && row >= 0 && re > rb) masks[(size_t)row * n + i] = msk;
+                if (MASKS && row >= 0) masks[(size_t)row * n + i] = msk;
                 if (row == 8) break;
                 row++;
                 rb = flat->b(row);
@@ -542,13 +907,12 @@ __device__ __forceinline__ void density_particle(uint32_t i, const float4* __res
         store_density(i, m * kc.kPoly6 * (s2 * s2 * s2) * acc, k, rho0, rho_p, rec, p, v);
         return;
     }
-#pragma unroll
     for (int row = 0; row < 9; row++) {
         const int dz = row / 3 - 1, dy = row % 3 - 1;
         unsigned long long msk = 0ull;
         uint32_t rb, re;
         if (row_range(w, dy, dz, cut, cp, key_base, start, end, n, rb, re))
-            msk = density_row<MASKS, false>(p, sp + rb, re - rb, h2u, hhu, acc);
+            msk = density_row<MASKS>(p, sp + rb, re - rb, h2u, hhu, acc);
         if (MASKS) masks[(size_t)row * n + i] = msk;
     }
     store_density(i, m * kc.kPoly6 * (s2 * s2 * s2) * acc, k, rho0, rho_p, rec, p, v);
@@ -610,16 +974,13 @@ __device__ __forceinline__ void pair_term_rp(PairAcc& A, uint32_t i, uint32_t j,
 
 // The neighbours of one row from its mask mm (self bit cleared), bit k
 // being record first + k, in ascending order, two per iteration.  Record j
-// is (pa[STRIDE j], pb[STRIDE j]): the interleaved records in memory
-// (STRIDE 2, pb = pa + 1) or the two halves staged apart in LDS (STRIDE 1),
-// where 16-byte reads of consecutive records then fall in distinct banks.
+// is (rec[2 j], rec[2 j + 1]), in memory.
 // The mask is walked as two 32-bit words, low word first (the same
 // ascending order): 32-bit bit scans and clears, and rows of at most 32
 // candidates never enter the second loop.
-template <int STRIDE>
 __device__ __forceinline__ void walk_row_mask(PairAcc& A, unsigned long long mm, uint32_t first,
-                                              const float4* __restrict__ pa, const float4* __restrict__ pb,
-                                              const float4& pos, const float4& vel, float pri, float h, float s) {
+                                              const float4* __restrict__ rec, const float4& pos, const float4& vel,
+                                              float pri, float h, float s) {
     uint32_t word = (uint32_t)mm, base = first;
     for (int half = 0; half < 2; half++) {
         while (word) {
@@ -629,8 +990,8 @@ __device__ __forceinline__ void walk_row_mask(PairAcc& A, unsigned long long mm,
             const uint32_t k2 = two ? (uint32_t)__builtin_ctz(word) : k1;
             word &= word - 1u;  // (0 stays 0)
             const uint32_t j1 = base + k1, j2 = base + k2;
-            const float4 a1 = pa[STRIDE * (size_t)j1], b1 = pb[STRIDE * (size_t)j1];
-            const float4 a2 = pa[STRIDE * (size_t)j2], b2 = pb[STRIDE * (size_t)j2];
+            const float4 a1 = rec[2 * (size_t)j1], b1 = rec[2 * (size_t)j1 + 1];
+            const float4 a2 = rec[2 * (size_t)j2], b2 = rec[2 * (size_t)j2 + 1];
             const float3 q1 = make_float3(a1.x, a1.y, a1.z), q2 = make_float3(a2.x, a2.y, a2.z);
             const float3 v1 = make_float3(b1.x, b1.y, b1.z), v2 = make_float3(b2.x, b2.y, b2.z);
             const float2 d1 = make_float2(a1.w, b1.w), d2 = make_float2(a2.w, b2.w);
@@ -645,6 +1006,24 @@ __device__ __forceinline__ void walk_row_mask(PairAcc& A, unsigned long long mm,
         word = (uint32_t)(mm >> 32);  // then the high word
         base = first + 32u;
         if (!word) break;
+    }
+}
+
+// One word of a row's mask over records staged in LDS (their first halves at
+// st, their second halves at st + kStageRecs, so that 16-byte reads of
+// consecutive records fall in distinct banks), bit k being record first + k,
+// in ascending order, one per iteration: from LDS a pair's latency is covered
+// by the SIMD's other wavefronts, and two pairs per iteration, the second
+// one under a mask of its own, took 24% more cycles per row (6775 against
+// 5466 SIMD cycles for a wavefront's nine rows of 24 neighbours).
+__device__ __forceinline__ void walk_staged_word(PairAcc& A, uint32_t word, uint32_t first,
+                                                 const float4* __restrict__ st, const float4& pos, const float4& vel,
+                                                 float pri, float h, float s) {
+    while (word) {
+        const uint32_t j = first + (uint32_t)__builtin_ctz(word);
+        word &= word - 1u;
+        const float4 a = st[j], b = st[kStageRecs + j];
+        pair_term_masked(A, pos, vel, pri, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w, h, s);
     }
 }
 
@@ -680,7 +1059,7 @@ __device__ __forceinline__ void forces_rowloop(PairAcc& A, uint32_t i, const flo
             unsigned long long mm = mrow;
             // the particle itself is in its own row's mask; it adds nothing
             if (i >= rb && i < re) mm &= ~(1ull << (i - rb));
-            walk_row_mask<2>(A, mm, rb, rec, rec + 1, pos, vel, dpi.y, h, s);
+            walk_row_mask(A, mm, rb, rec, pos, vel, dpi.y, h, s);
         } else {
             for (uint32_t j = rb; j < re; j++)
                 pair_term_rp(A, i, j, pos, vel, dpi.y, ld_xyz(sp + j), ld_xyz(sv + j), rho_p[j], h, s, hhu);
@@ -688,76 +1067,117 @@ __device__ __forceinline__ void forces_rowloop(PairAcc& A, uint32_t i, const flo
     }
 }
 
-// The masked row loop with each row's neighbour records staged in the
-// wavefront's LDS slice `stage` (kStageRecs records: their first halves,
-// then their second halves), for a whole wavefront
-// (every lane present; a lane of an inactive particle takes part with no
-// rows).  Same pairs, same order, same sums as forces_rowloop<true>.
-// AHEAD: the next row's cell bounds and mask are loaded a row ahead, after
-// this row's staging loads, so they arrive while this row is walked (about
-// five more registers; the single-fluid kernel runs it at 7 waves per SIMD).
-template <bool AHEAD>
-__device__ __forceinline__ void forces_rows_staged(PairAcc& A, uint32_t i, bool active, const float4& pos,
-                                                   const float4& vel, float2 dpi, const float4* __restrict__ sp,
-                                                   const float4* __restrict__ sv, const float2* __restrict__ rho_p,
-                                                   const uint32_t* __restrict__ start,
-                                                   const uint32_t* __restrict__ end, uint32_t n,
-                                                   const fg_common_fluid_params& cp, uint32_t key_base,
+// The masked row loop for a whole wavefront (every lane present; a lane of an
+// inactive particle, or one past the last particle, takes part with no rows)
+// from the runs the density pass left: each row's neighbour records staged
+// in the wavefront's LDS slice `stage` (kStageRecs first halves, then their
+// second halves), the next row's records, masks and offsets loaded into
+// registers while this row is walked.  No cell is looked up.  Same pairs,
+// same order, same sums as forces_rowloop<true>.  False when a row of the
+// wavefront has no usable run: nothing is summed then.
+//
+// Bound by VALU issue (3,300 instructions a wavefront) and by the records,
+// which come from past the L2 cache about three times at 8,388,608 particles:
+// 579 us there against 701 with the cells looked up again and a min/max
+// reduction per row; 84 against 98 us at 1,048,576.
+__device__ __forceinline__ bool forces_rows_staged(PairAcc& A, uint32_t i, bool active, const float4& pos,
+                                                   const float4& vel, float pri, uint32_t n,
+                                                   const fg_common_fluid_params& cp,
                                                    const unsigned long long* __restrict__ masks,
                                                    float4* __restrict__ stage) {
-    const float h = cp.kernel_radius, hh = h * h;
-    const float s = cp.simulation_scale;
-    const float hu = h / s, hhu = hu * hu;
-    const float cut = hh * 1.0001f;
-    const RowWalker w = make_rows(pos, cp);
+    const float h = cp.kernel_radius, s = cp.simulation_scale;
+    const uint32_t lane = __lane_id();
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(i >> 6);
     const float4* rec = nbr_records(masks, n);
-    RowFetch next{kEmpty, kEmpty, 0u, false};
-    unsigned long long next_mask = 0ull;
-    if (AHEAD && active) {
-        next = row_fetch(w, -1, -1, cut, cp, key_base, start, end);
-        next_mask = masks[i];
+    const uint16_t* offs = nbr_offs(masks, n) + (size_t)9 * 64 * wave + lane;
+    WaveRuns runs;
+    if (lane < 9u) {
+        const uint32_t* t = nbr_runs(masks, n) + (size_t)kRunWords * wave + lane;
+        runs.lo = t[0];
+        runs.info = t[9];
     }
+    if (__ballot((runs.info & kRunGeneric) != 0u) != 0ull) return false;
+    float4 a0, b0, a1, b1;
+    a0 = b0 = a1 = b1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    unsigned long long next_mask = 0ull;
+    uint32_t next_off = 0u;
+    auto fetch = [&](int row) {
+        const uint32_t len = runs.word(row) & kRunLength;
+        next_mask = active ? masks[(size_t)row * n + i] : 0ull;
+        next_off = offs[64 * row];
+        const float4* q = rec + 2 * ((size_t)runs.first(row) + lane);
+        if (lane < len) {
+            a0 = q[0];
+            b0 = q[1];
+        }
+        if (lane + 64u < len) {
+            a1 = q[128];
+            b1 = q[129];
+        }
+    };
+    fetch(0);
     for (int row = 0; row < 9; row++) {
-        const int dz = row / 3 - 1, dy = row % 3 - 1;
-        unsigned long long mrow = 0ull;
-        uint32_t rb = 0, re = 0;
-        bool has = false;
-        if (AHEAD) {
-            mrow = next_mask;
-            has = active && row_finish(next, w, dy, dz, cut, cp, key_base, start, end, n, rb, re);
-        } else if (active) {
-            mrow = masks[(size_t)row * n + i];
-            asm volatile("" ::"v"(mrow));
-            has = row_range(w, dy, dz, cut, cp, key_base, start, end, n, rb, re);
+        const uint32_t word = runs.word(row), len = word & kRunLength, lo = runs.first(row);  // the same on every lane
+        unsigned long long mm = next_mask;
+        const uint32_t off = next_off;
+        if (lane < len) {
+            stage[lane] = a0;
+            stage[kStageRecs + lane] = b0;
         }
-        uint32_t lo, hi;
-        const bool staged = wave_run_minmax(has, rb, re, kStageRecs, lo, hi);  // the same on every lane
-        if (staged) {
-            for (uint32_t k = __lane_id(); k < hi - lo; k += 64u) {
-                stage[k] = rec[2 * (size_t)(lo + k)];
-                stage[kStageRecs + k] = rec[2 * (size_t)(lo + k) + 1];
+        if (lane + 64u < len) {
+            stage[lane + 64u] = a1;
+            stage[kStageRecs + lane + 64u] = b1;
+        }
+        if (lane + 128u < min(len, kStageRecs)) {
+            const float4* q = rec + 2 * ((size_t)lo + lane + 128u);
+            stage[lane + 128u] = q[0];
+            stage[kStageRecs + lane + 128u] = q[1];
+        }
+        if (row < 8) fetch(row + 1);
+        // the particle itself is in its own cell's row; it adds nothing
+        if (row == 4) mm &= ~(1ull << ((i - lo - off) & 63u));
+        wave_lds_sync();
+        if (len <= kStageRecs) {
+            walk_staged_word(A, (uint32_t)mm, off, stage, pos, vel, pri, h, s);
+            if (word & kRunWide) walk_staged_word(A, (uint32_t)(mm >> 32), off + 32u, stage, pos, vel, pri, h, s);
+            wave_lds_sync();  // every lane's reads before the next stores
+            continue;
+        }
+        // a run that fills the slice more than once: the mask is walked as far
+        // as the records [at, at + kStageRecs) of the run go, then on from there
+        for (uint32_t at = 0u;;) {
+            while (mm) {
+                const uint32_t j = off + (uint32_t)__builtin_ctzll(mm) - at;
+                if (j >= kStageRecs) break;
+                mm &= mm - 1ull;
+                const float4 a = stage[j], b = stage[kStageRecs + j];
+                pair_term_masked(A, pos, vel, pri, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w, h,
+                                 s);
             }
-        }
-        if (AHEAD && row < 8 && active) {
-            next = row_fetch(w, (row + 1) % 3 - 1, (row + 1) / 3 - 1, cut, cp, key_base, start, end);
-            next_mask = masks[(size_t)(row + 1) * n + i];
-        }
-        if (staged) wave_lds_sync();
-        if (has) {
-            if (re - rb <= kRowMaskBits) {
-                unsigned long long mm = mrow;
-                // the particle itself is in its own row's mask; it adds nothing
-                if (i >= rb && i < re) mm &= ~(1ull << (i - rb));
-                if (staged)
-                    walk_row_mask<1>(A, mm, rb - lo, stage, stage + kStageRecs, pos, vel, dpi.y, h, s);
-                else
-                    walk_row_mask<2>(A, mm, rb, rec, rec + 1, pos, vel, dpi.y, h, s);
-            } else {
-                for (uint32_t j = rb; j < re; j++)
-                    pair_term_rp(A, i, j, pos, vel, dpi.y, ld_xyz(sp + j), ld_xyz(sv + j), rho_p[j], h, s, hhu);
+            wave_lds_sync();
+            at += kStageRecs;
+            if (at >= len) break;
+            for (uint32_t k = lane; k < min(len - at, kStageRecs); k += 64u) {
+                const float4* q = rec + 2 * ((size_t)lo + at + k);
+                stage[k] = q[0];
+                stage[kStageRecs + k] = q[1];
             }
+            wave_lds_sync();
         }
-        if (staged) wave_lds_sync();  // every lane's reads of this row before the next row's stores
+    }
+    return true;
+}
+
+// `v`; with LATER, by a pointer that the compiler takes for a new one, so that
+// nothing read through it is read before this point.
+template <bool LATER, class T>
+__device__ __forceinline__ const T& later(const T& v) {
+    if constexpr (LATER) {
+        const T* p = &v;
+        asm volatile("" : "+s"(p));
+        return *p;
+    } else {
+        return v;
     }
 }
 
@@ -782,8 +1202,9 @@ struct FlatRows {
 // in ascending sorted order):
 //  * row loop: the 9 rows in turn; a wavefront waits at every row for its
 //    lane with the most neighbours in that row.  Given an LDS slice
-//    (`stage`) and a full wavefront, each row's records are staged there
-//    first (forces_rows_staged);
+//    (`stage`) and a whole wavefront, each row's records are staged there
+//    first (forces_rows_staged); its last lanes may have i >= n and then
+//    only take part;
 //  * flat (MASKS with a row table): the rows with neighbours are gathered
 //    first, compacted in row order, then each lane walks its own neighbour
 //    stream across them, two neighbours per iteration with their loads
@@ -792,29 +1213,36 @@ struct FlatRows {
 //    most neighbours in that row.  The next row's entry is read from LDS
 //    one row ahead.  A particle with a row longer than kFlatRowBits takes
 //    the row loop.
-template <bool MASKS, bool COUPLED = false, bool DEFER = false, bool AHEAD = false>
+//
+// INDIRECT: cp lies in memory at a wave-uniform address (a batch's scene):
+// what follows the pair sums then reads it through a pointer of its own, or
+// the compiler loads all of it up front and keeps it in vector registers
+// during the pair sums.
+template <bool MASKS, bool COUPLED = false, bool DEFER = false, bool INDIRECT = false>
 __device__ __forceinline__ void forces_particle(uint32_t i, const float4* __restrict__ sp,
                                                 const float4* __restrict__ sv, const float2* __restrict__ rho_p,
                                                 const uint32_t* __restrict__ start, const uint32_t* __restrict__ end,
                                                 float4* __restrict__ vout, float4* __restrict__ pout,
                                                 const uint32_t* __restrict__ id, uint32_t n, float m, float mu,
-                                                const fg_common_fluid_params& cp, const fg_kernels_cache& kc,
+                                                const fg_common_fluid_params& cp0, const fg_kernels_cache& kc0,
                                                 uint32_t key_base, const unsigned long long* __restrict__ masks,
                                                 const Contacts& bc, FlatRows* flat = nullptr,
                                                 const DeferredContact* defer = nullptr,
                                                 float4* __restrict__ stage = nullptr) {
-    const float4 pos = sp[i];
-    const float4 vel = sv[i];
-    const bool active = pos.w > 0.0f;
+    const uint32_t il = min(i, n - 1u);
+    const float4 pos = sp[il];
+    const float4 vel = sv[il];
+    const bool active = i < n && pos.w > 0.0f;
     F3 a = f3(0.0f, 0.0f, 0.0f);
     PairAcc A{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    // The staged row loop needs every lane of the wavefront (the run of
-    // each row is a wavefront reduction); otherwise the rows are read from
-    // memory below.
-    const bool staged_rows = MASKS && stage != nullptr && flat == nullptr && __ballot(1) == ~0ull;
-    if (staged_rows)
-        forces_rows_staged<AHEAD>(A, i, active, pos, vel, active ? rho_p[i] : make_float2(1.0f, 0.0f), sp, sv, rho_p,
-                                  start, end, n, cp, key_base, masks, stage);
+    // The staged row loop needs every lane of the wavefront, as the density
+    // pass did; otherwise the rows are read from memory below.
+    bool staged_rows = false;
+    if (MASKS && stage != nullptr && flat == nullptr && __ballot(1) == ~0ull)
+        staged_rows = forces_rows_staged(A, i, active, pos, vel, rho_p[il].y, n, cp0, masks, stage);
+    const fg_common_fluid_params& cp = later<INDIRECT>(cp0);
+    const fg_kernels_cache& kc = later<INDIRECT>(kc0);
+    if (i >= n) return;
     if (active) {
         const float h = cp.kernel_radius, hh = h * h;
         const float s = cp.simulation_scale;

@@ -223,33 +223,40 @@ struct MixedRow {
 // rho = m kPoly6 s^6 sum (h^2 - r^2)^3 over the same pairs, summed in
 // ascending sorted order within rows in order, compensated.
 //
-// Given an LDS slice (`stage`, kMixedStage pair records then kMixedStage
-// positions) and a full wavefront, each row's run of pair records and
-// positions is staged there first, as in density_rows_staged; every lane
-// then takes part (an inactive particle's lane with no rows).
+// Given an LDS slice (`stage`) and a whole wavefront, each row's run of pair
+// records and positions is staged there first, as in density_rows_staged;
+// every lane then takes part (the lane of an inactive particle, or one past
+// the last particle, with no rows), and the runs are left for the force pass.
 constexpr uint32_t kMixedStage = 128;
+struct MixedStage {
+    uint4 rec[kMixedStage + 4];
+    float4 pos[kMixedStage];
+    WaveCells cells;
+};
+static_assert(offsetof(MixedStage, cells) >= sizeof(uint32_t) * kWaveCellsTemp, "wave_cells' temporary words");
 __device__ __forceinline__ void density_particle_mixed(uint32_t i, const float4* __restrict__ sp,
                                                        const float4* __restrict__ sv, float2* __restrict__ rho_p,
                                                        const uint32_t* __restrict__ start,
                                                        const uint32_t* __restrict__ end, uint32_t n, float k,
                                                        float rho0, float m, const fg_common_fluid_params& cp,
                                                        const fg_kernels_cache& kc,
-                                                       unsigned long long* __restrict__ masks,
-                                                       float4* __restrict__ stage = nullptr) {
-    const float4 p = sp[i];
+                                                       unsigned long long* __restrict__ masks, MixedStage& st) {
+    const bool valid = i < n;
+    const uint32_t il = min(i, n - 1u), lane = __lane_id();
+    const float4 p = sp[il];
     float4* rec = nbr_records(masks, n);
-    const float4 v = sv[i];
-    const bool active = p.w > 0.0f;
-    const bool staged_rows = stage != nullptr && __ballot(1) == ~0ull;
-    if (!active && !staged_rows) {
-        store_record(i, rho_p[i], p, v, rec);
-        return;
-    }
+    const bool active = valid && p.w > 0.0f;
     const float s = cp.simulation_scale, s2 = s * s;
     const float h = cp.kernel_radius, hh = h * h;
     const float hu = h / s, hhu = hu * hu, h2u = cp.kernel_radius_squared / s2;
     const float cut = hh * 1.0001f;
     const RowWalker w = make_rows(p, cp);
+    uint32_t cell, words = kRunGeneric;
+    WaveRuns runs;
+    const bool ok = wave_cells(st.cells, reinterpret_cast<uint32_t*>(st.rec), 64u, w, cp, 0u, start, end, n, cell, runs);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(i >> 6);
+    const bool table = n >= kRunMinParticles;
+    uint16_t* offs = nbr_offs(masks, n) + (size_t)9 * 64 * wave + lane;
     const HalfGeom g = half_geom(cp);
     const float3 o = half_offsets(p, cp, g);
     const uint4* __restrict__ hr = nbr_half(masks, n);
@@ -261,32 +268,49 @@ __device__ __forceinline__ void density_particle_mixed(uint32_t i, const float4*
                h2u,
                0.0f,
                0.0f};
-    uint4* hst = reinterpret_cast<uint4*>(stage);
-    const float4* pst = stage + (kMixedStage + 4u);
 
     for (int row = 0; row < 9; row++) {
         const int dz = row / 3 - 1, dy = row % 3 - 1;
+        const uint32_t len = runs.word(row), lo = runs.first(row);  // the same on every lane
+        const bool staged = ok && len <= kMixedStage;
         uint32_t rb = 0, re = 0;
-        const bool has = active && row_range(w, dy, dz, cut, cp, 0u, start, end, n, rb, re);
-        uint32_t lo = 0, hi = 0;
-        const bool staged = staged_rows && wave_run(has, rb, re, kMixedStage, lo, hi);  // the same on every lane
+        bool has;
+        if (ok) {
+            const LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
+            has = r.len != 0u;
+            rb = lo + r.off;
+            re = rb + r.len;
+            if (table) {
+                offs[64 * row] = (uint16_t)r.off;
+                const uint32_t word = run_word(len, r.len);
+                words = (int)lane == row ? word : words;
+            }
+        } else {
+            has = active && row_range(w, dy, dz, cut, cp, 0u, start, end, n, rb, re);
+        }
         if (staged) {
             // the pair records of the run and the two after it (a quad of
             // candidates reads the records t and t + 2), and the positions
-            for (uint32_t q = __lane_id(); q < hi - lo + 2u; q += 64u) hst[q] = hr[lo + q];
-            for (uint32_t q = __lane_id(); q < hi - lo; q += 64u) stage[kMixedStage + 4u + q] = sp[lo + q];
+            for (uint32_t q = lane; q < len + 2u; q += 64u) st.rec[q] = hr[lo + q];
+            for (uint32_t q = lane; q < len; q += 64u) st.pos[q] = sp[lo + q];
             wave_lds_sync();
         }
         unsigned long long msk = 0ull;
         if (has) {
             const half2v ty = {(_Float16)(o.y - (float)dy * g.wy), (_Float16)(o.y - (float)dy * g.wy)};
             const half2v tz = {(_Float16)(o.z - (float)dz * g.wz), (_Float16)(o.z - (float)dz * g.wz)};
-            msk = staged ? M.row<true>(hst + (rb - lo), pst + (rb - lo), re - rb, ty, tz)
+            msk = staged ? M.row<true>(st.rec + (rb - lo), st.pos + (rb - lo), re - rb, ty, tz)
                          : M.row<false>(hr + rb, sp + rb, re - rb, ty, tz);
         }
         if (active) masks[(size_t)row * n + i] = msk;
         if (staged) wave_lds_sync();  // every lane's reads of this row before the next row's stores
     }
+    if (table) {
+        runs.info = words;
+        store_runs(runs, wave, masks, n);
+    }
+    if (!valid) return;
+    const float4 v = sv[i];
     if (active)
         store_density(i, m * kc.kPoly6 * (s2 * s2 * s2) * (M.sum + M.comp), k, rho0, rho_p, rec, p, v);
     else

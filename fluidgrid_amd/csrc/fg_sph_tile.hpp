@@ -40,19 +40,8 @@ constexpr int kTileRowsMax = 2;
 constexpr int kTileSegs = 9 * kTileRowsMax;
 constexpr int kTileSpanMax = 128;  // cells per segment: two 64-lane chunks
 constexpr uint32_t kTileCap = 1664;  // 2 x 1664 x 16 B of records: three force workgroups per CU
-constexpr uint32_t kListMax = 64;
 constexpr uint16_t kListOverflow = 0xFFFFu;
 
-// Neighbour buffer (fg_neighbor_mask_bytes): 9 row masks per particle, then
-// from 256-byte boundaries the 32-byte neighbour records, a u16 list count
-// per particle and the lists (kListMax u16 per particle, in 16-byte groups).
-__host__ __device__ __forceinline__ size_t nbr_align256(size_t x) { return (x + 255) & ~(size_t)255; }
-__host__ __device__ __forceinline__ size_t nbr_count_offset(uint32_t n) {
-    return nbr_align256(nbr_record_offset(n) + 2 * 16 * (size_t)n);
-}
-__host__ __device__ __forceinline__ size_t nbr_list_offset(uint32_t n) {
-    return nbr_align256(nbr_count_offset(n) + 2 * (size_t)n);
-}
 // After the lists, one 256-byte descriptor per tile (TileDesc), written by
 // the tiled density pass for the force pass.
 constexpr uint32_t kTileDescWords = 64;

@@ -47,7 +47,7 @@ int key_bits_for(uint64_t nb) {
 
 // The persistent launches' work queue of a tuning (counters null: plain launches).
 fg::WorkQueue work_queue(unsigned* counters, const BatchTuning& t) {
-    return fg::WorkQueue{t.queueItems > 0 ? counters : nullptr, (uint32_t)(t.queueItems > 0 ? t.queueItems : 1)};
+    return fg::WorkQueue{t.queueItems > 0 ? counters : nullptr, (uint32_t)(t.queueItems > 0 ? t.queueItems : 1), 0u};
 }
 
 struct StreamScope {
