@@ -27,6 +27,18 @@ namespace fg {
 
 constexpr int kSphThreads = 256;
 
+// Lanes per particle of the reference-arithmetic kernels (k_density_ref,
+// k_forces_ref).  Up to kRefSpreadMax particles eight lanes a particle fill
+// the GPU and keep eight bucket walks in flight; above, one lane a particle
+// already does, and the groups' adding up costs more than it gains.  Measured
+// with the reference's hash (density / forces, us):
+//   24,108 particles   1 lane 51 / 90     8 lanes 15 / 31    16 lanes 15 / 31
+//   108,000            1 lane 60 / 141    8 lanes 48 / 100   16 lanes 49 / 109
+//   250,880            1 lane 98 / 185    8 lanes 125 / 212  16 lanes 131 / 249
+//   1,048,576          1 lane 358 / 593   8 lanes 647 / 970
+constexpr uint32_t kRefLanes = 8;
+constexpr uint32_t kRefSpreadMax = 163840;
+
 // ---------------------------------------------------------------------------
 // Reference-arithmetic kernels
 // ---------------------------------------------------------------------------
@@ -50,120 +62,188 @@ __device__ __forceinline__ bool stencil_bucket(const float4& p, const CellXYZ& c
     }
 }
 
-// K_FluidSim.cu:210-254 with ProcessMassDensityGridD (:46-79)
-template <int MODE>
+// The reference form spreads a particle's 27 buckets over LP lanes: lane sub
+// walks buckets sub, sub + LP, ... of the z, y, x stencil order, each into a
+// sum of its own from zero, and after each round the group adds the round's
+// sums in bucket order.  The 27 walks are chains of dependent loads (bucket
+// range, then its particles); one lane per particle walks them one after
+// another with most of the GPU idle below a few hundred thousand particles.
+// Sums equal to zero are not added: the running sum starts at +0 and so is
+// never -0 under round-to-nearest, and adding +0 or -0 changes no bit.
+//
+// A pair whose squared distance exceeds h^2 (1 + 2^-20) has a distance more
+// than two units in the last place above h, so its rounded square root
+// exceeds h as well: it is rejected without the square root (most of a
+// bucket's particles are).
+//
+// Bound by latency in small fluids and by VALU issue in large ones: a fluid
+// of 24,108 particles with hashed keys takes 15 (density) and 31 us (forces),
+// where one lane a particle, a powf a pair and every particle's terms under
+// one branch took 105 and 109; 1,048,576 particles take 358 and 593 us, then
+// 972 and 1,115.
+__device__ __forceinline__ float ref_cut(float h) { return rn_mul(rn_mul(h, h), 0x1.00001p+0f); }
+
+// x^3 (powf(x, 3.0f) in the reference), rounded once from 64 bits: x * x is
+// exact there.
+__device__ __forceinline__ float ref_cube(float x) {
+    const double d = (double)x;
+    return (float)(d * d * d);
+}
+
+// Adds the group's sums of one round to `total`, in lane order.
+template <uint32_t LP>
+__device__ __forceinline__ void ref_add_round(float& total, float part) {
+    const uint32_t first = __lane_id() & ~(LP - 1u);
+    uint32_t m = (uint32_t)(__ballot(part != 0.0f) >> first) & ((1u << LP) - 1u);
+    while (m) {
+        const int src = (int)first + __ffs((int)m) - 1;
+        m &= m - 1u;
+        total = rn_add(total, __shfl(part, src));
+    }
+}
+template <uint32_t LP>
+__device__ __forceinline__ void ref_add_round(F3& total, F3 part) {
+    const uint32_t first = __lane_id() & ~(LP - 1u);
+    uint32_t m = (uint32_t)(__ballot(part.x != 0.0f || part.y != 0.0f || part.z != 0.0f) >> first) & ((1u << LP) - 1u);
+    while (m) {
+        const int src = (int)first + __ffs((int)m) - 1;
+        m &= m - 1u;
+        total = add(total, f3(__shfl(part.x, src), __shfl(part.y, src), __shfl(part.z, src)));
+    }
+}
+
+// K_FluidSim.cu:210-254 with ProcessMassDensityGridD (:46-79), by groups of LP lanes
+template <int MODE, uint32_t LP>
 __global__ void __launch_bounds__(kSphThreads)
     k_density_ref(const float4* __restrict__ sp, float2* __restrict__ rho_p, const uint32_t* __restrict__ start,
                   const uint32_t* __restrict__ end, uint32_t n, float k, float rho0, float m,
                   fg_common_fluid_params cp, fg_kernels_cache kc) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = t / LP, lane = t % LP;
+    if (i >= n) return;  // the same for every lane of a group
     const float4 p = sp[i];
     if (!(p.w > 0.0f)) return;
     const float s = cp.simulation_scale, h = cp.kernel_radius, h2 = cp.kernel_radius_squared;
-    const float mkp = m * kc.kPoly6;
+    const float mkp = m * kc.kPoly6, cut = ref_cut(h);
     const uint32_t nb = dev_num_buckets(cp);
     CellXYZ c{0, 0, 0};
     if (MODE == FG_KEY_LINEAR) c = linear_cell(p.x, p.y, p.z, cp);
+    const F3 p1 = mul(xyz(p), s);
     float rho = 0.0f;
-    for (int z = -1; z <= 1; z++)
-        for (int y = -1; y <= 1; y++)
-            for (int x = -1; x <= 1; x++) {
-                uint32_t b;
-                if (!stencil_bucket<MODE>(p, c, x, y, z, cp, nb, b)) continue;
-                float part = 0.0f;
-                const uint32_t s0 = start[b];
-                if (s0 != kEmpty) {
-                    const F3 p1 = mul(xyz(p), s);
-                    const uint32_t e = min(end[b], n);
-                    for (uint32_t j = s0; j < e; j++) {
-                        const F3 p2 = mul(xyz(sp[j]), s);
-                        const F3 d = sub(p1, p2);
-                        const float l = len(d);
-                        if (l < h) part = part + mkp * powf(h2 - (l * l), 3.0f);
-                    }
+    for (uint32_t r0 = 0; r0 < 27u; r0 += LP) {
+        const int q = (int)(r0 + lane);
+        float part = 0.0f;
+        uint32_t b;
+        if (q < 27 && stencil_bucket<MODE>(p, c, q % 3 - 1, (q / 3) % 3 - 1, q / 9 - 1, cp, nb, b)) {
+            const uint32_t s0 = start[b], e0 = end[b];
+            const uint32_t e = s0 != kEmpty ? min(e0, n) : 0u;
+            for (uint32_t j0 = s0; j0 < e; j0 += 4u) {
+                float4 cand[4];
+#pragma unroll
+                for (uint32_t u = 0; u < 4u; u++) cand[u] = sp[min(j0 + u, e - 1u)];
+#pragma unroll
+                for (uint32_t u = 0; u < 4u; u++) {
+                    const F3 d = sub(p1, mul(xyz(cand[u]), s));
+                    const float r2 = dot(d, d);
+                    if (j0 + u >= e || r2 > cut) continue;
+                    const float l = rn_sqrt(r2);
+                    if (l < h) part = part + mkp * ref_cube(h2 - (l * l));
                 }
-                rho = rho + part;
             }
-    rho_p[i] = make_float2(fmaxf(1.0f, rho), k * (rho - rho0));
+        }
+        ref_add_round<LP>(rho, part);
+    }
+    if (lane == 0u) rho_p[i] = make_float2(fmaxf(1.0f, rho), k * (rho - rho0));
 }
 
 // Pressure + viscosity between particle i and the particles of one bucket
 // (K_FluidSim.cu:85-172).
-__device__ __forceinline__ F3 bucket_internal_ref(uint32_t i, uint32_t s0, uint32_t e, const float4& pos,
-                                                  const float4& vel, float2 dp1, const float4* __restrict__ sp,
+__device__ __forceinline__ F3 bucket_internal_ref(uint32_t i, uint32_t s0, uint32_t e, const F3& p1, const float4& vel,
+                                                  float2 dp1, const float4* __restrict__ sp,
                                                   const float4* __restrict__ sv, const float2* __restrict__ rho_p,
-                                                  float s, float h, float kSpiky, float kVisc, float mu) {
+                                                  float s, float h, float cut, float kSpiky, float kVisc, float mu) {
     F3 total = f3(0.0f, 0.0f, 0.0f);
-    const F3 p1 = mul(xyz(pos), s);
     const F3 v1 = xyz(vel);
-    for (uint32_t j = s0; j < e; j++) {
-        if (j == i) continue;
-        const F3 p2 = mul(xyz(sp[j]), s);
-        const float2 dp2 = rho_p[j];
-        const F3 v2 = xyz(sv[j]);
-        // SPHCalculatePressureForceD, K_FluidSim.cu:107-120
-        F3 fp = f3(0.0f, 0.0f, 0.0f);
-        {
-            const float pp = (dp1.y + dp2.y) / (dp1.x * dp2.x);
-            F3 diff = sub(p1, p2);
-            const float l = len(diff);
-            if (!(l > h)) {
-                const float r = kSpiky * ((h - l) * (h - l));
-                fp = mul(mul(mul(divs(diff, l), r), pp), -1.0f);
+    for (uint32_t b0 = s0; b0 < e; b0 += 32u) {
+        // the particles that may be within h, then only those: the terms'
+        // seven divisions are worth the second look at them
+        const uint32_t cnt = min(e - b0, 32u);
+        uint32_t near = 0u;
+        for (uint32_t k = 0; k < cnt; k += 4u) {
+            float4 cand[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; u++) cand[u] = sp[b0 + min(k + u, cnt - 1u)];
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; u++) {
+                const F3 d = sub(p1, mul(xyz(cand[u]), s));
+                near |= k + u < cnt && !(dot(d, d) > cut) ? 1u << (k + u) : 0u;
             }
         }
-        total = add(total, fp);
-        // SPHCalculateViscosityForceD, K_FluidSim.cu:85-102
-        F3 fv = f3(0.0f, 0.0f, 0.0f);
-        {
-            const F3 diff = sub(p1, p2);
-            const float l = len(diff);
-            if (!(l > h)) {
-                const float lap = kVisc * (h - l);
-                const float rr = dp1.x * dp2.x;
-                fv = f3(((v2.x - v1.x) / rr) * lap * mu, ((v2.y - v1.y) / rr) * lap * mu,
-                        ((v2.z - v1.z) / rr) * lap * mu);
-            }
+        if (i >= b0 && i - b0 < 32u) near &= ~(1u << (i - b0));
+        while (near) {
+            const uint32_t j = b0 + (uint32_t)__builtin_ctz(near);
+            near &= near - 1u;
+            const float2 dp2 = rho_p[j];
+            const F3 v2 = xyz(sv[j]);
+            const F3 diff = sub(p1, mul(xyz(sp[j]), s));
+            const float l = rn_sqrt(dot(diff, diff));
+            if (l > h) continue;  // both terms are zero
+            // SPHCalculatePressureForceD, K_FluidSim.cu:107-120
+            const float rr = dp1.x * dp2.x;
+            const float pp = (dp1.y + dp2.y) / rr;
+            const float r = kSpiky * ((h - l) * (h - l));
+            total = add(total, mul(mul(mul(divs(diff, l), r), pp), -1.0f));
+            // SPHCalculateViscosityForceD, K_FluidSim.cu:85-102
+            const float lap = kVisc * (h - l);
+            total = add(total, f3(((v2.x - v1.x) / rr) * lap * mu, ((v2.y - v1.y) / rr) * lap * mu,
+                                  ((v2.z - v1.z) / rr) * lap * mu));
         }
-        total = add(total, fv);
     }
     return total;
 }
 
 // K_FluidSim.cu:260-309 (+ fused integrate when pout != nullptr); with
-// COUPLED, K_FluidSim.cu:315-413.
-template <int MODE, bool COUPLED>
+// COUPLED, K_FluidSim.cu:315-413.  By groups of LP lanes, as k_density_ref.
+template <int MODE, bool COUPLED, uint32_t LP>
 __global__ void __launch_bounds__(kSphThreads)
     k_forces_ref(const float4* __restrict__ sp, const float4* __restrict__ sv, const float2* __restrict__ rho_p,
                  const uint32_t* __restrict__ start, const uint32_t* __restrict__ end, float4* __restrict__ vout,
                  float4* __restrict__ pout, const uint32_t* __restrict__ id, uint32_t n, float m, float mu,
                  fg_common_fluid_params cp, fg_kernels_cache kc, Contacts bc) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = t / LP, lane = t % LP;
+    if (i >= n) return;  // the same for every lane of a group
     const float4 pos = sp[i];
     const float4 vel = sv[i];
     F3 a = f3(0.0f, 0.0f, 0.0f);
     if (pos.w > 0.0f) {
         const float2 dp1 = rho_p[i];
         const uint32_t nb = dev_num_buckets(cp);
+        const float s = cp.simulation_scale, h = cp.kernel_radius, cut = ref_cut(h);
         CellXYZ c{0, 0, 0};
         if (MODE == FG_KEY_LINEAR) c = linear_cell(pos.x, pos.y, pos.z, cp);
+        const F3 p1 = mul(xyz(pos), s);
         F3 internal = f3(0.0f, 0.0f, 0.0f);
-        for (int z = -1; z <= 1; z++)
-            for (int y = -1; y <= 1; y++)
-                for (int x = -1; x <= 1; x++) {
-                    uint32_t b;
-                    if (!stencil_bucket<MODE>(pos, c, x, y, z, cp, nb, b)) continue;
-                    const uint32_t s0 = start[b];
-                    if (s0 == kEmpty) continue;
-                    internal = add(internal, bucket_internal_ref(i, s0, min(end[b], n), pos, vel, dp1, sp, sv, rho_p,
-                                                                 cp.simulation_scale, cp.kernel_radius,
-                                                                 kc.kSpikyGradient, kc.kViscosityLaplacian, mu));
-                }
-        a = finish_accel<COUPLED>(internal, m, pos, vel, cp, bc);
+        for (uint32_t r0 = 0; r0 < 27u; r0 += LP) {
+            const int q = (int)(r0 + lane);
+            F3 part = f3(0.0f, 0.0f, 0.0f);
+            uint32_t b;
+            if (q < 27 && stencil_bucket<MODE>(pos, c, q % 3 - 1, (q / 3) % 3 - 1, q / 9 - 1, cp, nb, b)) {
+                const uint32_t s0 = start[b], e0 = end[b];
+                if (s0 != kEmpty)
+                    part = bucket_internal_ref(i, s0, min(e0, n), p1, vel, dp1, sp, sv, rho_p, s, h, cut,
+                                               kc.kSpikyGradient, kc.kViscosityLaplacian, mu);
+            }
+            ref_add_round<LP>(internal, part);
+        }
+        // the body contact (fluid_external) with its cells over the same lanes
+        F3 ext = f3(0.0f, 0.0f, 0.0f);
+        if (COUPLED && bc.coupled) {
+            if (bc.st.enabled) ext = add(ext, contact_cells<LP>(pos, vel, bc.st, lane));
+            if (bc.dyn.enabled) ext = add(ext, contact_cells<LP>(pos, vel, bc.dyn, lane));
+        }
+        if (lane != 0u) return;
+        a = finish_accel_ext(internal, m, pos, vel, cp, COUPLED && bc.coupled, ext);
     }
-    write_back(id[i], n, pos, vel, a, cp, vout, pout);
+    if (lane == 0u) write_back(id[i], n, pos, vel, a, cp, vout, pout);
 }
 
 // K_FluidSim.cu:418-438
@@ -516,11 +596,20 @@ static bool use_fast() { return state().key_mode == FG_KEY_LINEAR && state().mat
         }                                                                                                   \
     } while (0)
 
+// Launch the reference form with kRefLanes lanes or one lane a particle.
+#define FG_REF_LAUNCH(SPREAD, SINGLE, ...)                                                                            \
+    do {                                                                                                              \
+        if (n <= kRefSpreadMax)                                                                                       \
+            hipLaunchKernelGGL(SPREAD, dim3(grid_for((uint64_t)n * kRefLanes, kSphThreads)), dim3(kSphThreads), 0,    \
+                               st.stream, __VA_ARGS__);                                                               \
+        else                                                                                                          \
+            hipLaunchKernelGGL(SINGLE, dim3(grid_for(n, kSphThreads)), dim3(kSphThreads), 0, st.stream, __VA_ARGS__); \
+    } while (0)
+
 int launch_density(float4* sp, float2* rho_p, uint32_t* start, uint32_t* end, uint32_t n, float k, float rho0,
                    float m, unsigned long long* masks = nullptr, const float4* sv = nullptr) {
     if (!stencil_covers_h("density pass")) return FG_ERR_UNSUPPORTED;
     const State& st = state();
-    const dim3 grid(grid_for(n, kSphThreads)), block(kSphThreads);
     const bool mixed = st.precision == FG_PRECISION_MIXED && use_fast() && masks;
     if (mixed && !half_records_for(masks, n)) {
         set_error(FG_ERR_NOT_INITIALIZED, "density pass (mixed precision): no cell pass has written FP16 offsets "
@@ -542,11 +631,11 @@ int launch_density(float4* sp, float2* rho_p, uint32_t* start, uint32_t* end, ui
         FG_SPH_LAUNCH(k_density_fast, false, n, sp, (const float4*)nullptr, rho_p, start, end, n, k, rho0, m, st.common, st.kernels,
                       (unsigned long long*)nullptr);
     else if (st.key_mode == FG_KEY_LINEAR)
-        hipLaunchKernelGGL(k_density_ref<FG_KEY_LINEAR>, grid, block, 0, st.stream, sp, rho_p, start, end, n, k,
-                           rho0, m, st.common, st.kernels);
+        FG_REF_LAUNCH((k_density_ref<FG_KEY_LINEAR, kRefLanes>), (k_density_ref<FG_KEY_LINEAR, 1>), sp, rho_p, start,
+                      end, n, k, rho0, m, st.common, st.kernels);
     else
-        hipLaunchKernelGGL(k_density_ref<FG_KEY_REF_XOR>, grid, block, 0, st.stream, sp, rho_p, start, end, n, k,
-                           rho0, m, st.common, st.kernels);
+        FG_REF_LAUNCH((k_density_ref<FG_KEY_REF_XOR, kRefLanes>), (k_density_ref<FG_KEY_REF_XOR, 1>), sp, rho_p, start,
+                      end, n, k, rho0, m, st.common, st.kernels);
     return check_launch("density") ? FG_OK : fg_peek_error();
 }
 
@@ -558,7 +647,6 @@ int launch_forces(float4* sp, float4* sv, float2* rho_p, uint32_t* start, uint32
     if (bcp) bc = *bcp;
     const bool coupled = bc.coupled != 0;
     const State& st = state();
-    const dim3 grid(grid_for(n, kSphThreads)), block(kSphThreads);
     if (use_fast() && masks && nbr_format_tiled(masks)) {
         if (coupled)
             hipLaunchKernelGGL(k_forces_tile<true>, dim3(grid_for(n, kTileLanes)), dim3(kTileLanes), 0, st.stream, sp,
@@ -615,18 +703,18 @@ int launch_forces(float4* sp, float4* sv, float2* rho_p, uint32_t* start, uint32
                            st.common, st.kernels, mk, bc, runs);
     } else if (st.key_mode == FG_KEY_LINEAR) {
         if (coupled)
-            hipLaunchKernelGGL((k_forces_ref<FG_KEY_LINEAR, true>), grid, block, 0, st.stream, sp, sv, rho_p, start,
-                               end, vout, pout, id, n, m, mu, st.common, st.kernels, bc);
+            FG_REF_LAUNCH((k_forces_ref<FG_KEY_LINEAR, true, kRefLanes>), (k_forces_ref<FG_KEY_LINEAR, true, 1>), sp, sv,
+                          rho_p, start, end, vout, pout, id, n, m, mu, st.common, st.kernels, bc);
         else
-            hipLaunchKernelGGL((k_forces_ref<FG_KEY_LINEAR, false>), grid, block, 0, st.stream, sp, sv, rho_p, start,
-                               end, vout, pout, id, n, m, mu, st.common, st.kernels, bc);
+            FG_REF_LAUNCH((k_forces_ref<FG_KEY_LINEAR, false, kRefLanes>), (k_forces_ref<FG_KEY_LINEAR, false, 1>), sp, sv,
+                          rho_p, start, end, vout, pout, id, n, m, mu, st.common, st.kernels, bc);
     } else {
         if (coupled)
-            hipLaunchKernelGGL((k_forces_ref<FG_KEY_REF_XOR, true>), grid, block, 0, st.stream, sp, sv, rho_p, start,
-                               end, vout, pout, id, n, m, mu, st.common, st.kernels, bc);
+            FG_REF_LAUNCH((k_forces_ref<FG_KEY_REF_XOR, true, kRefLanes>), (k_forces_ref<FG_KEY_REF_XOR, true, 1>), sp, sv,
+                          rho_p, start, end, vout, pout, id, n, m, mu, st.common, st.kernels, bc);
         else
-            hipLaunchKernelGGL((k_forces_ref<FG_KEY_REF_XOR, false>), grid, block, 0, st.stream, sp, sv, rho_p,
-                               start, end, vout, pout, id, n, m, mu, st.common, st.kernels, bc);
+            FG_REF_LAUNCH((k_forces_ref<FG_KEY_REF_XOR, false, kRefLanes>), (k_forces_ref<FG_KEY_REF_XOR, false, 1>), sp, sv,
+                          rho_p, start, end, vout, pout, id, n, m, mu, st.common, st.kernels, bc);
     }
     return check_launch("forces") ? FG_OK : fg_peek_error();
 }
