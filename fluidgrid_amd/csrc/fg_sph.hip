@@ -302,11 +302,14 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
                   Contacts bc, int runs) {
     // one LDS slice of kStageRecs neighbour records per wavefront (staged row loop)
     __shared__ float4 s_stage[MASKS ? (BS / 64) * 2 * kStageRecs : 1];
+    // without masks: a slice of records with their cells
+    __shared__ ForceStage s_tested[MASKS ? 1 : BS / 64];
     const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * BS + threadIdx.x;
     if ((i & ~63u) >= n) return;  // whole wavefronts; lanes past the last particle take part idle
     forces_particle<MASKS, COUPLED>(i, sp, sv, rho_p, start, end, vout, pout, id, n, m, mu, cp, kc, 0u, masks, bc,
                                     nullptr, nullptr,
-                                    MASKS && runs ? s_stage + (threadIdx.x / 64) * 2 * kStageRecs : nullptr);
+                                    MASKS && runs ? s_stage + (threadIdx.x / 64) * 2 * kStageRecs : nullptr,
+                                    MASKS ? nullptr : &s_tested[threadIdx.x / 64]);
 }
 
 // Flat schedule (row table in LDS); same results as k_forces_fast<true, COUPLED>.

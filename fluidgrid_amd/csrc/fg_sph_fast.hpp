@@ -1168,6 +1168,123 @@ __device__ __forceinline__ bool forces_rows_staged(PairAcc& A, uint32_t i, bool 
     return true;
 }
 
+// A wavefront's slice in the force pass without masks: the records of the
+// current part of a run, (x, y), (z, 1/rho) and (vx, vy, vz, p/rho) apart, so
+// that the distance test reads them as the density pass does.
+struct ForceStage {
+    float2 xy[kStageRecs + 4], za[kStageRecs + 4];
+    float4 vb[kStageRecs];
+    WaveCells cells;
+    __device__ __forceinline__ uint32_t* temp() { return reinterpret_cast<uint32_t*>(xy); }
+};
+static_assert(offsetof(ForceStage, cells) >= sizeof(uint32_t) * kWaveCellsTemp, "wave_cells' temporary words");
+
+// The bits of up to 32 staged candidates from slice index `at` that lie
+// within h of p (density_group's hit bits; p and the slice hold no NaN).
+#pragma clang fp contract(off)
+__device__ __forceinline__ uint32_t near_bits(const float4& p, const ForceStage& st, uint32_t at, uint32_t cnt,
+                                              float hhu) {
+    const float2* xy = st.xy + at;
+    const float2* za = st.za + at;
+    uint32_t bits = 0u, k = 0u;
+    for (; k < cnt; k += 4u) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            const float dx = p.x - xy[k + u].x, dy = p.y - xy[k + u].y, dz = p.z - za[k + u].x;
+            const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+            bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(r2 - hhu), 31);
+        }
+    }
+    const uint32_t word = __builtin_bitreverse32(bits) >> (32u - k);
+    return cnt < 32u ? word & ((1u << cnt) - 1u) : word;  // (what lies past them in the slice)
+}
+#pragma clang fp contract(fast)
+
+// The row loop without masks for a whole wavefront (as forces_rows_staged):
+// each row's records are made from the sorted arrays while they are staged,
+// the lanes test their candidates there and then walk those within h.  Same
+// pairs, same order, same sums as forces_rowloop<false>.  False when the
+// wavefront has no usable runs (wave_cells): nothing is summed then.
+//
+// Bound by VALU issue (the test and the walk); 250,047 particles take 48 us,
+// where every candidate's position, velocity and density read from memory
+// and a division per candidate took 97; 1,048,576 take 159, then 344.
+__device__ __forceinline__ bool forces_rows_tested(PairAcc& A, uint32_t i, bool active, const float4& pos,
+                                                   const float4& vel, float pri, const float4* __restrict__ sp,
+                                                   const float4* __restrict__ sv, const float2* __restrict__ rho_p,
+                                                   const uint32_t* __restrict__ start,
+                                                   const uint32_t* __restrict__ end, uint32_t n,
+                                                   const fg_common_fluid_params& cp, uint32_t key_base,
+                                                   ForceStage& st) {
+    const float h = cp.kernel_radius, s = cp.simulation_scale;
+    const float hu = h / s, hhu = hu * hu, cut = h * h * 1.0001f;
+    const uint32_t lane = __lane_id();
+    const RowWalker w = make_rows(pos, cp);
+    uint32_t cell;
+    WaveRuns runs;
+    if (!wave_cells(st.cells, st.temp(), 64u, w, cp, key_base, start, end, n, cell, runs)) return false;
+    const float4 own = own_finite(pos);
+    float3 p0, p1, v0, v1;
+    float2 d0, d1;
+    p0 = p1 = v0 = v1 = make_float3(0.0f, 0.0f, 0.0f);
+    d0 = d1 = make_float2(1.0f, 0.0f);
+    auto load = [&](uint32_t j, float3& p, float3& v, float2& d) {
+        p = ld_xyz(sp + j);
+        v = ld_xyz(sv + j);
+        d = rho_p[j];
+    };
+    auto put = [&](uint32_t k, const float3& p, const float3& v, const float2& d) {
+        const float a = 1.0f / d.x;
+        st.xy[k] = make_float2(stage_finite(p.x), stage_finite(p.y));
+        st.za[k] = make_float2(stage_finite(p.z), a);
+        st.vb[k] = make_float4(v.x, v.y, v.z, d.y * a);
+    };
+    auto fetch = [&](int row) {
+        const uint32_t len = runs.word(row), lo = runs.first(row);
+        if (lane < len) load(lo + lane, p0, v0, d0);
+        if (lane + 64u < len) load(lo + lane + 64u, p1, v1, d1);
+    };
+    fetch(0);
+    for (int row = 0; row < 9; row++) {
+        const uint32_t len = runs.word(row), lo = runs.first(row);  // the same on every lane
+        const LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
+        for (uint32_t at = 0u;;) {  // (a run rarely fills the slice)
+            const uint32_t cnt = min(len - at, kStageRecs);
+            if (at == 0u) {
+                if (lane < cnt) put(lane, p0, v0, d0);
+                if (lane + 64u < cnt) put(lane + 64u, p1, v1, d1);
+                if (row < 8) fetch(row + 1);
+            }
+            for (uint32_t k = lane + (at == 0u ? 128u : 0u); k < cnt; k += 64u) {
+                float3 p, v;
+                float2 d;
+                load(lo + at + k, p, v, d);
+                put(k, p, v, d);
+            }
+            wave_lds_sync();
+            const uint32_t b = min(r.off + r.len, at + kStageRecs);
+            for (uint32_t a = max(r.off, at); a < b; a += 32u) {
+                const uint32_t c = min(b - a, 32u), k0 = a - at;
+                uint32_t word = near_bits(own, st, k0, c, hhu);
+                const uint32_t self = i - (lo + a);  // the particle itself adds nothing
+                if (self < 32u) word &= ~(1u << self);
+                while (word) {
+                    const uint32_t k = k0 + (uint32_t)__builtin_ctz(word);
+                    word &= word - 1u;
+                    const float2 xy = st.xy[k], za = st.za[k];
+                    const float4 vb = st.vb[k];
+                    pair_term_masked(A, pos, vel, pri, make_float3(xy.x, xy.y, za.x), make_float3(vb.x, vb.y, vb.z),
+                                     za.y, vb.w, h, s);
+                }
+            }
+            wave_lds_sync();  // every lane's reads before the next stores
+            at += kStageRecs;
+            if (at >= len) break;
+        }
+    }
+    return true;
+}
+
 // `v`; with LATER, by a pointer that the compiler takes for a new one, so that
 // nothing read through it is read before this point.
 template <bool LATER, class T>
@@ -1228,7 +1345,7 @@ __device__ __forceinline__ void forces_particle(uint32_t i, const float4* __rest
                                                 uint32_t key_base, const unsigned long long* __restrict__ masks,
                                                 const Contacts& bc, FlatRows* flat = nullptr,
                                                 const DeferredContact* defer = nullptr,
-                                                float4* __restrict__ stage = nullptr) {
+                                                float4* __restrict__ stage = nullptr, ForceStage* tested = nullptr) {
     const uint32_t il = min(i, n - 1u);
     const float4 pos = sp[il];
     const float4 vel = sv[il];
@@ -1240,6 +1357,9 @@ __device__ __forceinline__ void forces_particle(uint32_t i, const float4* __rest
     bool staged_rows = false;
     if (MASKS && stage != nullptr && flat == nullptr && __ballot(1) == ~0ull)
         staged_rows = forces_rows_staged(A, i, active, pos, vel, rho_p[il].y, n, cp0, masks, stage);
+    if (!MASKS && tested != nullptr && __ballot(1) == ~0ull)
+        staged_rows = forces_rows_tested(A, i, active, pos, vel, rho_p[il].y, sp, sv, rho_p, start, end, n, cp0,
+                                         key_base, *tested);
     const fg_common_fluid_params& cp = later<INDIRECT>(cp0);
     const fg_kernels_cache& kc = later<INDIRECT>(kc0);
     if (i >= n) return;

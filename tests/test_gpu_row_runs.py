@@ -110,3 +110,34 @@ def test_runs_match_oracle(fglib, orc, which):
                                               nbr.ptr, d["vel"].ptr, None, d["sp"].ptr, s.n, s.fluid.mass,
                                               s.fluid.viscosity), "forces")
     check_velocity(d["vel"].numpy(), v_ref.astype(np.float64), acc, mag, sp, s.common.deltaTimeIntegration)
+
+
+@pytest.mark.parametrize("which", list(CASES))
+def test_launchers_without_masks_give_the_same_bits(fglib, orc, which):
+    """gCalcMassDensity and gSPHCalculateForces, which keep no neighbour
+    buffer, against the passes that do: the same densities and velocities,
+    bit for bit."""
+    s = CASES[which]()
+    L = fglib.load()
+    sk, sp, start, end, spos, svel = grid_cpu(orc, s)
+    fglib.init_params(s.common, s.kernels, s.key_mode, abi.MATH_FAST)
+    d = {k: fglib.DeviceArray.from_numpy(v) for k, v in dict(spos=spos, svel=svel, start=start, end=end, sp=sp).items()}
+    nbr = fglib.DeviceArray((L.fg_neighbor_mask_bytes(s.n),), np.uint8)
+    out = []
+    for masks in (True, False):
+        rp = fglib.DeviceArray.from_numpy(np.zeros((s.n, 2), np.float32))
+        vel = fglib.DeviceArray.from_numpy(s.vel)
+        if masks:
+            fglib.check(L.fg_sph_density_nbr(d["spos"].ptr, d["svel"].ptr, rp.ptr, d["start"].ptr, d["end"].ptr,
+                                             nbr.ptr, s.n, s.fluid.gasConstant, s.fluid.restDensity, s.fluid.mass))
+            fglib.check(L.fg_sph_forces_integrate_nbr(d["spos"].ptr, d["svel"].ptr, rp.ptr, d["start"].ptr,
+                                                      d["end"].ptr, nbr.ptr, vel.ptr, None, d["sp"].ptr, s.n,
+                                                      s.fluid.mass, s.fluid.viscosity))
+        else:
+            L.gCalcMassDensity(d["spos"].ptr, rp.ptr, None, d["start"].ptr, d["end"].ptr, s.n, s.fluid.gasConstant,
+                               s.fluid.restDensity, s.fluid.mass)
+            L.gSPHCalculateForces(d["spos"].ptr, d["svel"].ptr, None, rp.ptr, d["start"].ptr, d["end"].ptr, vel.ptr,
+                                  d["sp"].ptr, s.n, s.fluid.mass, s.fluid.viscosity)
+            fglib.check(None, "launchers")
+        out.append((rp.numpy(), vel.numpy()))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
