@@ -227,18 +227,18 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(6)))
 // Second pass of the deferred form: contact, walls, clamp and integration
 // of the deferred particles (finish_accel<true> and write_back, as
 // forces_particle ends), from the pair sum in dc.acc.  Each deferred
-// particle takes a pair of lanes that walk its stencil cells together
-// (contact_cells): a body grid's walk is a chain of dependent loads (bucket
-// range, then each sphere), and one lane per particle would walk its 27
-// cells one after another.  Of 1, 2, 4, 8 and 16 lanes per particle, 2
-// measured fastest (256 scenes with 479 bodies, 455k deferred particles).
-constexpr uint32_t kContactLanes = 2;
-__global__ void __launch_bounds__(256)
+// particle takes a group of lanes that walk its stencil cells together
+// (contact_cells).  128 scenes with 4 or fewer bodies each: 115 us with two
+// lanes a particle, 98 us so.  Five wavefronts a SIMD (96 registers, 20 bytes
+// of scratch) measured faster than the compiler's four: 98 against 117 us.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
     k_batch_contact_finish(const fg_scene_desc* __restrict__ scenes, uint32_t nscenes,
                            const uint32_t* __restrict__ scene_of, const float4* __restrict__ sp,
                            const float4* __restrict__ sv, float4* __restrict__ vout, float4* __restrict__ pout,
                            const uint32_t* __restrict__ id, uint32_t n, const BatchBodyScene* __restrict__ bodies,
                            DeferredContact dc) {
+    __shared__ ContactWave s_contact[256 / 64];
+    ContactWave& contact = s_contact[threadIdx.x / 64];
     const uint32_t cnt = min(*dc.count, n);
     const uint32_t sub = threadIdx.x % kContactLanes;
     const uint32_t groups = gridDim.x * (blockDim.x / kContactLanes);
@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(256)
             const BodyContact& dyn = bodies[s].dyn;
             const float4 pos = sp[i], vel = sv[i];
             // fluid_external with the dynamic grid only: +0 + its contact sum
-            const F3 ext = dyn.enabled ? add(f3(0.0f, 0.0f, 0.0f), contact_cells<kContactLanes>(pos, vel, dyn, sub))
+            const F3 ext = dyn.enabled ? add(f3(0.0f, 0.0f, 0.0f), contact_cells(pos, vel, dyn, sub, contact))
                                        : f3(0.0f, 0.0f, 0.0f);
             if (sub != 0) return;
             const fg_scene_desc& d = scenes[s];

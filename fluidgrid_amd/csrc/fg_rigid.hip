@@ -21,15 +21,10 @@ GridDesc fluid_grid_desc(const fg_common_fluid_params& cp, fg_float3 cs, uint32_
 
 #pragma clang fp contract(off)
 
-// Lanes per body sphere of the body-force kernels: the stencil cells of a
-// sphere are walked by a group of kBodyLanes lanes (contact_stencil_lanes),
-// so a sphere's 27 chains of dependent loads are in flight together.
-constexpr uint32_t kBodyLanes = 8;
+// The body-force kernels take a group of kContactLanes lanes for each body
+// sphere (contact_stencil_lanes); sub is the lane's index in its group.
 
-// K_RigidBodySim.cu:66-99, for body sphere i, with its stencil walked by LP
-// lanes (sub: the lane's index in its group; LP = 1: one lane, the 27 cell
-// starts loaded together).
-template <uint32_t LP>
+// K_RigidBodySim.cu:66-99, for body sphere i.
 __device__ __forceinline__ void body_sphere_from_fluid(uint32_t i, const float4* __restrict__ rb_pos,
                                                        const float4* __restrict__ rb_vel,
                                                        const float4* __restrict__ rb_cm, float4* __restrict__ out_f,
@@ -39,19 +34,14 @@ __device__ __forceinline__ void body_sphere_from_fluid(uint32_t i, const float4*
                                                        const uint32_t* __restrict__ sph_start,
                                                        const uint32_t* __restrict__ sph_end, uint32_t nsph,
                                                        float sph_radius, const GridDesc& g, int3 relation, float ks,
-                                                       float kd, uint32_t sub = 0) {
+                                                       float kd, uint32_t sub, ContactWave& contact) {
     const float4 pos = rb_pos[i];
     const int b = f2i_sat(pos.w);
     const bool ok = b >= 0 && (uint32_t)b < nbodies;
     const float4 vel = ok ? rb_vel[b] : make_float4(0, 0, 0, 0);
     const float4 cm = ok ? rb_cm[b] : make_float4(0, 0, 0, 0);
-    F3 F;
-    if constexpr (LP == 1)
-        F = contact_stencil<true>(pos, vel, radius, sph_pos, sph_vel, sph_radius, ks, kd, relation, sph_start, sph_end,
-                                  g, false, false, 0, 0.0001f, nsph, nsph);
-    else
-        F = contact_stencil_lanes<LP>(pos, vel, radius, sph_pos, sph_vel, sph_radius, ks, kd, relation, sph_start,
-                                      sph_end, g, false, false, 0, 0.0001f, nsph, nsph, sub);
+    const F3 F = contact_stencil_lanes(pos, vel, radius, sph_pos, sph_vel, sph_radius, ks, kd, relation, sph_start,
+                                       sph_end, g, false, false, 0, 0.0001f, nsph, nsph, sub, contact);
     if (sub != 0) return;
     out_f[i] = make_float4(F.x, F.y, F.z, (float)b);
     const float4 dir = make_float4(pos.x - cm.x, pos.y - cm.y, pos.z - cm.z, pos.w - cm.w);
@@ -68,10 +58,12 @@ __global__ void __launch_bounds__(256)
                              const uint32_t* __restrict__ sph_end, uint32_t nsph, float sph_radius, GridDesc g,
                              int3 relation, float ks, float kd) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t i = t / kBodyLanes;
+    const uint32_t i = t / kContactLanes;
+    __shared__ ContactWave s_contact[256 / 64];
     if (i >= m) return;  // the same for every lane of a group
-    body_sphere_from_fluid<kBodyLanes>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, radius, sph_pos, sph_vel,
-                                       sph_start, sph_end, nsph, sph_radius, g, relation, ks, kd, t % kBodyLanes);
+    body_sphere_from_fluid(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, radius, sph_pos, sph_vel,
+                                       sph_start, sph_end, nsph, sph_radius, g, relation, ks, kd, t % kContactLanes,
+                           s_contact[threadIdx.x / 64]);
 }
 
 __device__ __forceinline__ bool inside_box(const float4& p, const float4& lo, const float4& hi) {
@@ -88,16 +80,15 @@ __device__ __forceinline__ bool inside_box(const float4& p, const float4& lo, co
 // skipped walk would only have added +0.  ACCUM adds the force and torque to
 // what out_f/out_t hold (the fluid's part), else they are written.
 // For body sphere i; the broad phase looks at the bounds of bodies
-// [k0, k1) other than the sphere's own.  The stencils are walked by LP
-// lanes (sub: the lane's index in its group).
-template <bool ACCUM, uint32_t LP>
+// [k0, k1) other than the sphere's own.
+template <bool ACCUM>
 __device__ __forceinline__ void body_sphere_from_bodies(uint32_t i, const float4* __restrict__ rb_pos,
                                                         const float4* __restrict__ rb_vel,
                                                         const float4* __restrict__ rb_cm, float4* __restrict__ out_f,
                                                         float4* __restrict__ out_t, uint32_t nbodies, float radius,
                                                         const BodyContact& dyn, const BodyContact& st,
                                                         const float4* __restrict__ body_bounds, uint32_t k0,
-                                                        uint32_t k1, uint32_t sub) {
+                                                        uint32_t k1, uint32_t sub, ContactWave& contact) {
     const float4 pos = rb_pos[i];
     const int b = f2i_sat(pos.w);
     const bool ok = b >= 0 && (uint32_t)b < nbodies;
@@ -107,22 +98,22 @@ __device__ __forceinline__ void body_sphere_from_bodies(uint32_t i, const float4
     if (dyn.enabled) {
         bool near = body_bounds == nullptr;
         if (!near) {
-            // the group's lanes test the bodies in turn (lane sub: k0 + sub, k0 + sub + LP, ...)
+            // the group's lanes test the bodies in turn (lane sub: k0 + sub, k0 + sub + 8, ...)
             bool hit = false;
-            for (uint32_t k = k0 + sub; !hit && k < k1; k += LP)
+            for (uint32_t k = k0 + sub; !hit && k < k1; k += kContactLanes)
                 if ((int)k != b) hit = inside_box(pos, body_bounds[2 * k], body_bounds[2 * k + 1]);
-            const uint32_t first = __lane_id() & ~(LP - 1u);
-            near = ((__ballot(hit) >> first) & (LP == 32 ? 0xFFFFFFFFull : ((1ull << LP) - 1ull))) != 0ull;
+            const uint32_t first = __lane_id() & ~(kContactLanes - 1u);
+            near = ((__ballot(hit) >> first) & ((1ull << kContactLanes) - 1ull)) != 0ull;
         }
         if (near)
-            F = add(F, contact_stencil_lanes<LP>(pos, vel, radius, dyn.pos, dyn.vel, dyn.body_radius, dyn.ks, dyn.kd,
+            F = add(F, contact_stencil_lanes(pos, vel, radius, dyn.pos, dyn.vel, dyn.body_radius, dyn.ks, dyn.kd,
                                                  dyn.relation, dyn.start, dyn.end, dyn.grid, true, true, b, dyn.eps,
-                                                 dyn.count, dyn.nvel, sub));
+                                                 dyn.count, dyn.nvel, sub, contact));
     }
     if (st.enabled && (st.aabb == nullptr || inside_box(pos, st.aabb[0], st.aabb[1])))
-        F = add(F, contact_stencil_lanes<LP>(pos, vel, radius, st.pos, nullptr, st.body_radius, st.ks, st.kd,
+        F = add(F, contact_stencil_lanes(pos, vel, radius, st.pos, nullptr, st.body_radius, st.ks, st.kd,
                                              st.relation, st.start, st.end, st.grid, false, false, 0, st.eps,
-                                             st.count, 0u, sub));
+                                             st.count, 0u, sub, contact));
     if (sub != 0) return;
     const float4 dir = make_float4(pos.x - cm.x, pos.y - cm.y, pos.z - cm.z, pos.w - cm.w);
     const float4 t = vec3_cross(dir, make_float4(F.x, F.y, F.z, 0.0f));
@@ -143,10 +134,11 @@ __global__ void __launch_bounds__(256)
                               float4* __restrict__ out_t, uint32_t m, uint32_t nbodies, float radius, BodyContact dyn,
                               BodyContact st, const float4* __restrict__ body_bounds, uint32_t nbounds) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t i = t / kBodyLanes;
+    const uint32_t i = t / kContactLanes;
+    __shared__ ContactWave s_contact[256 / 64];
     if (i >= m) return;  // the same for every lane of a group
-    body_sphere_from_bodies<ACCUM, kBodyLanes>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, radius, dyn, st,
-                                               body_bounds, 0u, nbounds, t % kBodyLanes);
+    body_sphere_from_bodies<ACCUM>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, radius, dyn, st,
+                                               body_bounds, 0u, nbounds, t % kContactLanes, s_contact[threadIdx.x / 64]);
 }
 
 // K_RigidBodySim.cu:102-111
@@ -463,7 +455,7 @@ __global__ void __launch_bounds__(256) k_bbody_bounds(const float4* __restrict__
 }
 
 #pragma clang fp contract(off)
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
     k_bbody_from_fluid(const float4* __restrict__ rb_pos, const float4* __restrict__ rb_vel,
                        const float4* __restrict__ rb_cm, float4* __restrict__ out_f, float4* __restrict__ out_t,
                        uint32_t m, uint32_t nbodies, const uint32_t* __restrict__ body_scene,
@@ -471,14 +463,15 @@ __global__ void __launch_bounds__(256)
                        const float4* __restrict__ sph_vel, const uint32_t* __restrict__ sph_start,
                        const uint32_t* __restrict__ sph_end, uint32_t nsph) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t i = t / kBodyLanes;
+    const uint32_t i = t / kContactLanes;
+    __shared__ ContactWave s_contact[256 / 64];
     if (i >= m) return;  // the same for every lane of a group
     const int b = f2i_sat(rb_pos[i].w);
     if (b < 0 || (uint32_t)b >= nbodies) return;
     const BatchBodyScene& d = scenes[body_scene[b]];
-    body_sphere_from_fluid<kBodyLanes>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, d.sphere_radius, sph_pos,
+    body_sphere_from_fluid(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, d.sphere_radius, sph_pos,
                                        sph_vel, sph_start, sph_end, nsph, d.fluid_radius, d.fluid, d.rb_to_fluid, d.ks,
-                                       d.kd, t % kBodyLanes);
+                                       d.kd, t % kContactLanes, s_contact[threadIdx.x / 64]);
 }
 
 // Scenes with one body have no body-body pass (the single-fluid simulator
@@ -489,7 +482,8 @@ __global__ void __launch_bounds__(256)
                         uint32_t m, uint32_t nbodies, const uint32_t* __restrict__ body_scene,
                         const BatchBodyScene* __restrict__ scenes, const float4* __restrict__ body_bounds) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t i = t / kBodyLanes;
+    const uint32_t i = t / kContactLanes;
+    __shared__ ContactWave s_contact[256 / 64];
     if (i >= m) return;  // the same for every lane of a group
     const int b = f2i_sat(rb_pos[i].w);
     if (b < 0 || (uint32_t)b >= nbodies) return;
@@ -501,8 +495,9 @@ __global__ void __launch_bounds__(256)
     dyn.eps = 0.001f;
     dyn.aabb = nullptr;
     const BodyContact st{};
-    body_sphere_from_bodies<true, kBodyLanes>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, d.sphere_radius, dyn,
-                                              st, body_bounds, d.body_begin, d.body_end, t % kBodyLanes);
+    body_sphere_from_bodies<true>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, d.sphere_radius, dyn,
+                                              st, body_bounds, d.body_begin, d.body_end, t % kContactLanes,
+                                  s_contact[threadIdx.x / 64]);
 }
 
 __global__ void k_bintegrate_rb(float4* __restrict__ pos, const float* __restrict__ mass, float4* __restrict__ vel,
@@ -545,10 +540,10 @@ int batch_body_forces(const float4* world, const float4* vel, const float4* cm, 
                       const float4* fluid_pos, const float4* fluid_vel, const uint32_t* fluid_start,
                       const uint32_t* fluid_end, uint32_t nfluid, const float4* body_bounds) {
     if (m == 0) return FG_OK;
-    hipLaunchKernelGGL(k_bbody_from_fluid, dim3(grid_for((uint64_t)m * kBodyLanes, 256)), dim3(256), 0, state().stream, world, vel, cm,
+    hipLaunchKernelGGL(k_bbody_from_fluid, dim3(grid_for((uint64_t)m * kContactLanes, 256)), dim3(256), 0, state().stream, world, vel, cm,
                        out_f, out_t, m, nbodies, body_scene, scenes, fluid_pos, fluid_vel, fluid_start, fluid_end,
                        nfluid);
-    hipLaunchKernelGGL(k_bbody_from_bodies, dim3(grid_for((uint64_t)m * kBodyLanes, 256)), dim3(256), 0, state().stream, world, vel, cm,
+    hipLaunchKernelGGL(k_bbody_from_bodies, dim3(grid_for((uint64_t)m * kContactLanes, 256)), dim3(256), 0, state().stream, world, vel, cm,
                        out_f, out_t, m, nbodies, body_scene, scenes, body_bounds);
     return check_launch("batch_body_forces") ? FG_OK : fg_peek_error();
 }
@@ -733,7 +728,7 @@ int fg_body_forces_from_fluid(fg_float4* spheres, fg_float4* bodyVelocities, fg_
     const State& st = state();
     // The fluid grid is walked with the key function it was built with.
     const GridDesc g = fluid_grid_desc(st.common, fluidCellSize, fluidNumBuckets, st.key_mode);
-    hipLaunchKernelGGL(k_body_forces_from_fluid, dim3(grid_for((uint64_t)numSpheres * kBodyLanes, 256)), dim3(256), 0, st.stream,
+    hipLaunchKernelGGL(k_body_forces_from_fluid, dim3(grid_for((uint64_t)numSpheres * kContactLanes, 256)), dim3(256), 0, st.stream,
                        FG_F4(spheres), FG_F4(bodyVelocities), FG_F4(bodyCM), FG_F4(outForces), FG_F4(outTorques),
                        numSpheres, numBodies, radius, FG_F4(fluidOrderedPositions), FG_F4(fluidOrderedVelocities),
                        fluidGridStart, fluidGridEnd, numFluid, fluidRadius, g,
@@ -781,7 +776,7 @@ void gCalculateRigidBodyForcesFromRB(fg_float4* _in_RBPositions, fg_float4* _in_
     st.grid = body_grid(_in_CellSize, _in_numSRB > 0 ? (uint32_t)_in_SRBHashTableSize : 1u);
     st.count = 0xFFFFFFFFu;
     st.nvel = 0;
-    hipLaunchKernelGGL(k_body_forces_from_bodies<false>, dim3(grid_for((uint64_t)_in_NumParticles * kBodyLanes, 256)), dim3(256), 0,
+    hipLaunchKernelGGL(k_body_forces_from_bodies<false>, dim3(grid_for((uint64_t)_in_NumParticles * kContactLanes, 256)), dim3(256), 0,
                        state().stream, FG_F4(_in_RBPositions), FG_F4(_in_RBVelocites), FG_F4(_in_RBCMPosition),
                        FG_F4(_out_Forces), FG_F4(_out_torque), _in_NumParticles, 0xFFFFFFFFu, _in_Radius, dyn, st,
                        (const float4*)nullptr, 0u);
@@ -820,13 +815,13 @@ int fg_body_forces_from_bodies(const fg_float4* spheres, const fg_float4* bodyVe
     }
     const float4* bb = bodies ? reinterpret_cast<const float4*>(bodyBounds) : nullptr;
     if (accumulate)
-        hipLaunchKernelGGL(k_body_forces_from_bodies<true>, dim3(grid_for((uint64_t)numSpheres * kBodyLanes, 256)), dim3(256), 0,
+        hipLaunchKernelGGL(k_body_forces_from_bodies<true>, dim3(grid_for((uint64_t)numSpheres * kContactLanes, 256)), dim3(256), 0,
                            state().stream, reinterpret_cast<const float4*>(spheres),
                            reinterpret_cast<const float4*>(bodyVelocities), reinterpret_cast<const float4*>(bodyCM),
                            FG_F4(outForces), FG_F4(outTorques), numSpheres, numBodies, radius, dyn, st, bb,
                            numBodies);
     else
-        hipLaunchKernelGGL(k_body_forces_from_bodies<false>, dim3(grid_for((uint64_t)numSpheres * kBodyLanes, 256)), dim3(256), 0,
+        hipLaunchKernelGGL(k_body_forces_from_bodies<false>, dim3(grid_for((uint64_t)numSpheres * kContactLanes, 256)), dim3(256), 0,
                            state().stream, reinterpret_cast<const float4*>(spheres),
                            reinterpret_cast<const float4*>(bodyVelocities), reinterpret_cast<const float4*>(bodyCM),
                            FG_F4(outForces), FG_F4(outTorques), numSpheres, numBodies, radius, dyn, st, bb,

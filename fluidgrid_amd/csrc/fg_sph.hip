@@ -237,8 +237,13 @@ __global__ void __launch_bounds__(kSphThreads)
         // the body contact (fluid_external) with its cells over the same lanes
         F3 ext = f3(0.0f, 0.0f, 0.0f);
         if (COUPLED && bc.coupled) {
-            if (bc.st.enabled) ext = add(ext, contact_cells<LP>(pos, vel, bc.st, lane));
-            if (bc.dyn.enabled) ext = add(ext, contact_cells<LP>(pos, vel, bc.dyn, lane));
+            if constexpr (LP == kContactLanes) {
+                __shared__ ContactWave s_contact[kSphThreads / 64];
+                ContactWave& contact = s_contact[threadIdx.x / 64];
+                if (bc.st.enabled) ext = add(ext, contact_cells(pos, vel, bc.st, lane, contact));
+                if (bc.dyn.enabled) ext = add(ext, contact_cells(pos, vel, bc.dyn, lane, contact));
+            } else
+                ext = fluid_external(pos, vel, bc);
         }
         if (lane != 0u) return;
         a = finish_accel_ext(internal, m, pos, vel, cp, COUPLED && bc.coupled, ext);
@@ -353,23 +358,26 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
 // Second pass of the deferred form: body contact (fluid_external: the
 // static grid, then the dynamic one, summed from zero), walls, clamp and
 // integration of the listed particles from their pair sums.  Each particle
-// takes a pair of lanes that walk its body-grid cells together
-// (contact_cells, bit-identical to the one-lane walk).
-constexpr uint32_t kFinishLanes = 2;
-__global__ void __launch_bounds__(256)
+// takes a group of lanes that walk its body-grid cells together
+// (contact_cells, bit-identical to the one-lane walk).  Six wavefronts a SIMD
+// (80 registers, 16 bytes of scratch): 58 us, the compiler's five 64 us, at
+// 1,048,576 particles of which 112k are listed.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
     k_contact_finish(const float4* __restrict__ sp, const float4* __restrict__ sv, float4* __restrict__ vout,
                      float4* __restrict__ pout, const uint32_t* __restrict__ id, uint32_t n, float m,
                      fg_common_fluid_params cp, Contacts bc, DeferredContact dc) {
+    __shared__ ContactWave s_contact[256 / 64];
+    ContactWave& contact = s_contact[threadIdx.x / 64];
     const uint32_t cnt = min(*dc.count, n);
-    const uint32_t sub = threadIdx.x % kFinishLanes;
-    const uint32_t groups = gridDim.x * (blockDim.x / kFinishLanes);
-    // k is the same on both lanes of a group, so a group is active or idle as a whole
-    for (uint32_t k = (blockIdx.x * blockDim.x + threadIdx.x) / kFinishLanes; k < cnt; k += groups) {
+    const uint32_t sub = threadIdx.x % kContactLanes;
+    const uint32_t groups = gridDim.x * (blockDim.x / kContactLanes);
+    // k is the same on every lane of a group, so a group is active or idle as a whole
+    for (uint32_t k = (blockIdx.x * blockDim.x + threadIdx.x) / kContactLanes; k < cnt; k += groups) {
         const uint32_t i = dc.list[k];
         const float4 pos = sp[i], vel = sv[i];
         F3 e = f3(0.0f, 0.0f, 0.0f);
-        if (bc.st.enabled) e = add(e, contact_cells<kFinishLanes>(pos, vel, bc.st, sub));
-        if (bc.dyn.enabled) e = add(e, contact_cells<kFinishLanes>(pos, vel, bc.dyn, sub));
+        if (bc.st.enabled) e = add(e, contact_cells(pos, vel, bc.st, sub, contact));
+        if (bc.dyn.enabled) e = add(e, contact_cells(pos, vel, bc.dyn, sub, contact));
         if (sub != 0) continue;
         const float4 ia = dc.acc[i];
         const F3 a = finish_accel_ext(f3(ia.x, ia.y, ia.z), m, pos, vel, cp, bc.coupled != 0, e);
@@ -687,8 +695,8 @@ int launch_forces(float4* sp, float4* sv, float2* rho_p, uint32_t* start, uint32
                 default: FG_SPH_LAUNCH_BS(k_forces_deferred<256>, 256, n, sp, sv, rho_p, start, end, vout, pout, id,
                                           n, m, mu, st.common, st.kernels, mk, bc, dc, runs);
             }
-            // up to one lane pair per particle (the count is known only on the device)
-            unsigned blocks = grid_for((uint64_t)n * kFinishLanes, 256);
+            // up to one group of lanes per particle (the count is known only on the device)
+            unsigned blocks = grid_for((uint64_t)n * kContactLanes, 256);
             if (blocks > 8192) blocks = 8192;
             hipLaunchKernelGGL(k_contact_finish, dim3(blocks), dim3(256), 0, st.stream, sp, sv, vout, pout, id, n, m,
                                st.common, bc, dc);

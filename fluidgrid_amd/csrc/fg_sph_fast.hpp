@@ -353,15 +353,6 @@ struct DensityStage {
 };
 static_assert(offsetof(DensityStage, cells) >= sizeof(uint32_t) * kWaveCellsTemp, "wave_cells' temporary words");
 
-// Orders a wavefront's LDS stores before its other lanes' loads (and loads
-// before the next stores): the lanes of one wavefront need no workgroup
-// barrier.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The runs of a wavefront's nine rows: row r's first index and length word
 // (as in the runs table), in lane r.
 struct WaveRuns {
