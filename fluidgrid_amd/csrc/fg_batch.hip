@@ -310,6 +310,30 @@ static bool queue_ok(const WorkQueue& q, const char* who) {
     return true;
 }
 
+// Scene of every particle: the last scene that begins at or before it.
+__global__ void __launch_bounds__(256)
+    k_batch_scene_of(const fg_scene_desc* __restrict__ scenes, uint32_t nscenes, uint32_t* __restrict__ scene_of,
+                     uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    uint32_t lo = 0, hi = nscenes;  // scenes[lo].particleBegin <= i; scenes[hi] begins after i or is past the end
+    while (hi - lo > 1u) {
+        const uint32_t mid = lo + (hi - lo) / 2u;
+        if (scenes[mid].particleBegin <= i)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    scene_of[i] = lo;
+}
+
+int batch_scene_of(const fg_scene_desc* scenes, uint32_t nscenes, uint32_t* scene_of, uint32_t n) {
+    if (n == 0) return FG_OK;
+    hipLaunchKernelGGL(k_batch_scene_of, dim3(grid_for(n, 256)), dim3(256), 0, state().stream, scenes, nscenes,
+                       scene_of, n);
+    return check_launch("batch_scene_of") ? FG_OK : fg_peek_error();
+}
+
 int batch_density(const fg_scene_desc* scenes, uint32_t nscenes, const uint32_t* scene_of, float4* sp,
                   const float4* sv, float2* rho_p, uint32_t* start, uint32_t* end, unsigned long long* masks,
                   uint32_t n, WorkQueue q) {

@@ -42,6 +42,9 @@ struct WorkQueue {
     uint32_t runs;  // (force passes) the neighbour buffer holds the wavefronts' row runs
 };
 
+// Writes the scene of each of n particles.
+int batch_scene_of(const fg_scene_desc* scenes, uint32_t nscenes, uint32_t* scene_of, uint32_t n);
+
 // fg_batch_density_nbr / fg_batch_forces_integrate_nbr, optionally persistent.
 int batch_density(const fg_scene_desc* scenes, uint32_t nscenes, const uint32_t* scene_of, float4* sp,
                   const float4* sv, float2* rho_p, uint32_t* start, uint32_t* end, unsigned long long* masks,

@@ -35,15 +35,14 @@ int fg_bsim_create(unsigned int numScenes, const fg_common_fluid_params* commons
     }
     try {
         batch().reset();
-        std::vector<Simulators::BatchScene> scenes(numScenes);
+        std::vector<Simulators::BatchSceneView> scenes(numScenes);
         size_t off = 0;
         for (unsigned s = 0; s < numScenes; s++) {
             scenes[s].common = Application::abi_cast<Application::CommonFluidParams>(commons[s]);
             scenes[s].fluid = Application::abi_cast<Application::FluidParams>(fluids[s]);
-            const float4* p = reinterpret_cast<const float4*>(positions) + off;
-            const float4* v = reinterpret_cast<const float4*>(velocities) + off;
-            scenes[s].positions.assign(p, p + counts[s]);
-            scenes[s].velocities.assign(v, v + counts[s]);
+            scenes[s].positions = reinterpret_cast<const float4*>(positions) + off;
+            scenes[s].velocities = reinterpret_cast<const float4*>(velocities) + off;
+            scenes[s].count = counts[s];
             off += counts[s];
         }
         batch() = std::make_unique<Simulators::BatchedSimulator>(scenes);

@@ -31,6 +31,16 @@ struct BatchScene {
     std::vector<float4> velocities;
 };
 
+// A scene whose particles stay in the caller's arrays, which are read only
+// while the simulator is constructed.
+struct BatchSceneView {
+    Application::CommonFluidParams common;
+    Application::FluidParams fluid;
+    const float4* positions;
+    const float4* velocities;
+    size_t count;
+};
+
 // Dynamic rigid bodies of one scene: the inputs a single-fluid simulator
 // takes for them (fg_sim_add_bodies).
 struct BatchBodies {
@@ -59,6 +69,7 @@ struct BatchTuning {
 class BatchedSimulator {
 public:
     explicit BatchedSimulator(const std::vector<BatchScene>& scenes);
+    explicit BatchedSimulator(const std::vector<BatchSceneView>& scenes);
     ~BatchedSimulator();
     BatchedSimulator(const BatchedSimulator&) = delete;
     BatchedSimulator& operator=(const BatchedSimulator&) = delete;
