@@ -5,19 +5,18 @@
 // 469, 542).  Ties keep their input order, so the result is the unique stable
 // permutation of the keys.
 //
-// Design (wave64, gfx950): a 256-lane workgroup owns a tile of 2048 or 4096
-// consecutive elements (8 or 16 per lane, by size); each digit pass is three
-// launches,
+// Design (wave64, gfx950): a workgroup owns a tile of 2048 or 4096
+// consecutive elements (2 or 8 per lane, by size); each digit pass is two or
+// three launches,
 //  * upsweep: per-tile digit counts (per-wave LDS histograms; a run of equal
-//    digits in a wavefront is counted once, by its first lane), stored
-//    digit-major;
-//  * scan: one workgroup per digit turns its row of tile counts into
-//    exclusive offsets within the digit and records the digit's total;
+//    digits in a wavefront is counted once, by its first lane);
+//  * scan (many tiles): one workgroup per digit turns its row of tile counts
+//    into exclusive offsets within the digit and records the digit's total;
 //  * downsweep: the tile is ranked stably with wave-wide ballot matching
 //    (peers with an equal digit found bit by bit), its global offsets are
 //    the digit base (an exclusive scan of the totals) plus the tile's offset
-//    within the digit, and it is staged in LDS in digit order and written
-//    out as coalesced runs.
+//    within the digit (of few tiles, summed here from their counts), and it is
+//    staged in LDS in digit order and written out as coalesced runs.
 // No workgroup waits for another (a single-sweep pass with decoupled
 // look-back chains tiles: at 1M keys the chain, not the bytes, set its
 // time).  Digit widths are chosen from the key width (<= 8 bits per pass),
@@ -28,19 +27,30 @@
 
 namespace fg {
 
-constexpr int kSortThreads = 256;
-// Items per lane: 8 (2048-element tiles) up to kSmallTileMaxN keys, where
-// twice as many tiles fill the GPU better and each tile's chain of loads,
-// ranking and stores is shorter; 16 (4096-element tiles) above, where the
-// per-tile counts and their scan would grow.  Measured per sort (22-bit keys
-// at 1M: 63 us against 75; 25-bit at 8M: 230 against 227; 27-bit at 33.5M:
-// 1023 against 849).
-constexpr int kSortItemsSmall = 8;
-constexpr int kSortItemsLarge = 16;
-constexpr uint32_t kSmallTileMaxN = 1u << 22;
-static int sort_items(uint32_t n) { return n <= kSmallTileMaxN ? kSortItemsSmall : kSortItemsLarge; }
+// A pass's workgroup: 2048 keys on 1024 lanes (2 a lane) up to kSmallTileMaxN
+// keys, 4096 on 512 (8 a lane) above.  A lane's keys are ranked one after
+// another through the wavefront's counts, so a short sort, whose workgroups
+// all run at once, takes the time of one chain and wants it short; a long one
+// wants long runs of each digit to write.  Measured per sort (us):
+//   keys (bits)   2048 on 256  on 512  on 1024   4096 on 256  on 512  on 1024
+//   16,000 (16)          20.0    15.2     14.5
+//   1,000,000 (22)       48.8    44.1     44.4          64.0    50.9     48.3
+//   2,000,000 (22)       60.2    57.8     63.5          71.1    59.7     57.6
+//   3,000,000 (22)       73.9    73.2     81.1          78.8    71.0     74.8
+//   33,500,000 (27)     815.5   811.1    858.0         716.4   690.5    693.3
+// (8192 keys on 512 and 1024 lanes at 3,000,000: 87.0 and 94.9.)
+constexpr int kSmallThreads = 1024, kSmallItems = 2;
+constexpr int kLargeThreads = 512, kLargeItems = 8;
+constexpr uint32_t kSmallTileMaxN = 3u << 19;
+// Up to this many tiles (131,072 keys) a pass adds up the tiles' counts of each
+// digit itself, and the launch of the scan is saved (us, with and without the
+// scan: 65,000 keys 20.5 and 16.8; 131,000 20.7 and 20.3; 262,000 21.3 and 27.2).
+constexpr uint32_t kSumMaxTiles = 64;
+static_assert(kSumMaxTiles * kSmallThreads * kSmallItems <= kSmallTileMaxN, "large tiles are scanned");
+constexpr int kSortThreads = 256;  // of the scan
+static bool sort_small(uint32_t n) { return n <= kSmallTileMaxN; }
 static uint32_t sort_tiles(uint32_t n) {
-    const uint32_t tile = (uint32_t)(kSortThreads * sort_items(n));
+    const uint32_t tile = (uint32_t)(sort_small(n) ? kSmallThreads * kSmallItems : kLargeThreads * kLargeItems);
     return (n + tile - 1) / tile;
 }
 constexpr int kSortWaves = kSortThreads / 64;
@@ -119,19 +129,55 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
     return (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
 }
 
+// The value of the lane below, of a wavefront all of whose lanes are active
+// (0 on the first lane): one instruction, where __shfl_up goes through the LDS
+// crossbar.
+__device__ __forceinline__ uint32_t lane_below(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138 /* wave_shr:1 */, 0xF, 0xF, false);
+}
+
+// Inclusive sums of v over the wavefront's lanes, all active: within rows of
+// 16, then row 0 into 1 and 2 into 3, then the lower half into the upper.
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
+    uint32_t x = v;
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111 /* row_shr:1 */, 0xF, 0xF, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142 /* row_bcast:15 */, 0xA, 0xF, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143 /* row_bcast:31 */, 0xC, 0xF, false);
+    return x;
+}
+
+// Adds the wavefront's digits d (of valid lanes) to its counts cnt: a run of
+// equal digits once, by its first lane.
+__device__ __forceinline__ void count_runs(uint32_t d, bool valid, uint32_t* cnt) {
+    const int lane = (int)__lane_id();
+    const uint32_t prev = lane_below(d);
+    const bool head = valid && (lane == 0 || prev != d);
+    const uint64_t heads = __ballot(head) | __ballot(!valid);  // an invalid lane ends the run before it
+    if (head) {
+        const uint64_t after = lane == 63 ? 0ull : (heads >> (lane + 1));
+        const uint32_t len = after ? (uint32_t)__ffsll((long long)after) : (uint32_t)(64 - lane);
+        atomicAdd(&cnt[d], len);
+    }
+}
+
 // Upsweep: digit counts of tile blockIdx.x (ITEMS keys per lane), into
-// counts[d * tiles + tile].
-template <int ITEMS>
-__global__ void __launch_bounds__(kSortThreads) k_sort_upsweep(const uint32_t* __restrict__ keys, uint32_t n,
-                                                               int shift, int bits, uint32_t* __restrict__ counts,
-                                                               uint32_t tiles) {
-    __shared__ uint32_t s_cnt[kSortWaves][kMaxRadix];
+// counts[d * tiles + tile] for the scan, else counts[tile * digits + d], where
+// a pass's lanes read one tile's counts together.
+template <int THREADS, int ITEMS>
+__global__ void __launch_bounds__(THREADS) k_sort_upsweep(const uint32_t* __restrict__ keys, uint32_t n, int shift,
+                                                          int bits, uint32_t* __restrict__ counts, uint32_t tiles,
+                                                          bool scanned) {
+    constexpr int kWaves = THREADS / 64;
+    __shared__ uint32_t s_cnt[kWaves][kMaxRadix];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < kSortWaves * kMaxRadix; i += kSortThreads) (&s_cnt[0][0])[i] = 0;
+    for (int i = tid; i < kWaves * kMaxRadix; i += THREADS) (&s_cnt[0][0])[i] = 0;
     __syncthreads();
     const uint32_t tile = blockIdx.x;
     const uint32_t dmask = (1u << bits) - 1u;
-    const uint32_t wbase = tile * (uint32_t)(kSortThreads * ITEMS) + (uint32_t)wave * 64u * ITEMS;
+    const uint32_t wbase = tile * (uint32_t)(THREADS * ITEMS) + (uint32_t)wave * 64u * ITEMS;
     uint32_t key[ITEMS];
 #pragma unroll
     for (int k = 0; k < ITEMS; k++) {
@@ -142,41 +188,29 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_upsweep(const uint32_t* _
     for (int k = 0; k < ITEMS; k++) {
         const uint32_t idx = wbase + (uint32_t)k * 64u + (uint32_t)lane;
         const bool valid = idx < n;
-        const uint32_t d = valid ? (key[k] >> shift) & dmask : 0xFFFFFFFFu;
-        const uint32_t prev = (uint32_t)__shfl_up((int)d, 1);
-        const bool head = valid && (lane == 0 || prev != d);
-        const uint64_t heads = __ballot(head) | __ballot(!valid);  // an invalid lane ends the run before it
-        if (head) {
-            const uint64_t after = lane == 63 ? 0ull : (heads >> (lane + 1));
-            const uint32_t len = after ? (uint32_t)__ffsll((long long)after) : (uint32_t)(64 - lane);
-            atomicAdd(&s_cnt[wave][d], len);
-        }
+        count_runs(valid ? (key[k] >> shift) & dmask : 0xFFFFFFFFu, valid, s_cnt[wave]);
     }
     __syncthreads();
     const uint32_t radix = 1u << bits;
-    for (uint32_t d = (uint32_t)tid; d < radix; d += kSortThreads) {
+    for (uint32_t d = (uint32_t)tid; d < radix; d += THREADS) {
         uint32_t c = 0;
 #pragma unroll
-        for (int w = 0; w < kSortWaves; w++) c += s_cnt[w][d];
-        counts[(size_t)d * tiles + tile] = c;
+        for (int w = 0; w < kWaves; w++) c += s_cnt[w][d];
+        counts[scanned ? (size_t)d * tiles + tile : (size_t)tile * radix + d] = c;
     }
 }
 
 // Exclusive scan of v over the workgroup's 256 lanes (in lane order);
 // *total receives the sum.  Uses s_w[kSortWaves].
+template <int WAVES>
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_w, uint32_t* total) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)x, o);
-        if (lane >= o) x += y;
-    }
+    const uint32_t x = wave_inclusive_scan(v);
     if (lane == 63) s_w[wave] = x;
     __syncthreads();
     uint32_t before = 0, sum = 0;
 #pragma unroll
-    for (int w = 0; w < kSortWaves; w++) {
+    for (int w = 0; w < WAVES; w++) {
         const uint32_t t = s_w[w];
         before += w < wave ? t : 0u;
         sum += t;
@@ -201,7 +235,7 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_scan(uint32_t* __restrict
 #pragma unroll 4
     for (uint32_t t = t0; t < t1; t++) sum += row[t];
     uint32_t total;
-    uint32_t run = block_exclusive_scan(sum, s_w, &total);
+    uint32_t run = block_exclusive_scan<kSortWaves>(sum, s_w, &total);
     for (uint32_t t = t0; t < t1; t++) {
         const uint32_t c = row[t];
         row[t] = run;
@@ -213,25 +247,25 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_scan(uint32_t* __restrict
 // Downsweep of one digit pass.  Element e of tile T is base + w*64*ITEMS +
 // k*64 + lane, so (wave, item, lane) order is index order and the ranking
 // is stable.
-template <int ITEMS>
-__global__ void __launch_bounds__(kSortThreads) k_sort_pass(const uint32_t* __restrict__ kin,
+template <int THREADS, int ITEMS, bool SCANNED>
+__global__ void __launch_bounds__(THREADS) k_sort_pass(const uint32_t* __restrict__ kin,
                                                             const uint32_t* __restrict__ vin,
                                                             uint32_t* __restrict__ kout,
                                                             uint32_t* __restrict__ vout, uint32_t n, int shift,
                                                             int bits, const uint32_t* __restrict__ counts,
                                                             uint32_t tiles, const uint32_t* __restrict__ totals,
                                                             int values_iota) {
-    constexpr int TILE = kSortThreads * ITEMS;
+    constexpr int TILE = THREADS * ITEMS, kWaves = THREADS / 64;
     __shared__ uint32_t s_keys[TILE];
     __shared__ uint32_t s_vals[TILE];
-    __shared__ uint32_t s_wcnt[kSortWaves][kMaxRadix];
+    __shared__ uint32_t s_wcnt[kWaves][kMaxRadix];
     __shared__ uint32_t s_tstart[kMaxRadix];
     __shared__ uint32_t s_gbase[kMaxRadix];
-    __shared__ uint32_t s_w[kSortWaves];
+    __shared__ uint32_t s_w[kWaves];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t radix = 1u << bits, dmask = radix - 1u;
-    for (int i = tid; i < kSortWaves * kMaxRadix; i += kSortThreads) (&s_wcnt[0][0])[i] = 0;
+    for (int i = tid; i < kWaves * kMaxRadix; i += THREADS) (&s_wcnt[0][0])[i] = 0;
     __syncthreads();
     const uint32_t tile = blockIdx.x;
     const uint32_t base = tile * (uint32_t)TILE;
@@ -248,8 +282,20 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_pass(const uint32_t* __re
     // this tile's offset within each digit and the digit totals, loaded
     // while the tile is ranked
     const uint32_t d_own = (uint32_t)tid;
-    const uint32_t my_off = d_own < radix ? counts[(size_t)d_own * tiles + tile] : 0u;
-    const uint32_t my_total = d_own < radix ? totals[d_own] : 0u;
+    uint32_t my_off = 0, my_total = 0;
+    if constexpr (SCANNED) {
+        if (d_own < radix) {
+            my_off = counts[(size_t)d_own * tiles + tile];
+            my_total = totals[d_own];
+        }
+    } else if (d_own < radix) {
+#pragma unroll 8
+        for (uint32_t t = 0; t < tiles; t++) {
+            const uint32_t c = counts[(size_t)t * radix + d_own];
+            my_off += t < tile ? c : 0u;
+            my_total += c;
+        }
+    }
     const uint64_t lt = lanemask_lt();
 #pragma unroll
     for (int k = 0; k < ITEMS; k++) {
@@ -279,7 +325,7 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_pass(const uint32_t* __re
     uint32_t tile_count = 0;
     if (d_own < radix) {
         uint32_t run = 0;
-        for (int w = 0; w < kSortWaves; w++) {
+        for (int w = 0; w < kWaves; w++) {
             const uint32_t c = s_wcnt[w][d_own];
             s_wcnt[w][d_own] = run;
             run += c;
@@ -287,8 +333,8 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_pass(const uint32_t* __re
         tile_count = run;
     }
     uint32_t unused;
-    const uint32_t tstart = block_exclusive_scan(tile_count, s_w, &unused);
-    const uint32_t dbase = block_exclusive_scan(my_total, s_w, &unused);
+    const uint32_t tstart = block_exclusive_scan<kWaves>(tile_count, s_w, &unused);
+    const uint32_t dbase = block_exclusive_scan<kWaves>(my_total, s_w, &unused);
     if (d_own < radix) {
         s_tstart[d_own] = tstart;
         s_gbase[d_own] = dbase + my_off;
@@ -308,7 +354,7 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_pass(const uint32_t* __re
     }
     __syncthreads();
     const uint32_t count = (n - base) < (uint32_t)TILE ? (n - base) : (uint32_t)TILE;
-    for (uint32_t q = tid; q < count; q += kSortThreads) {
+    for (uint32_t q = tid; q < count; q += THREADS) {
         const uint32_t kk = s_keys[q];
         const uint32_t d = (kk >> shift) & dmask;
         const uint32_t dest = s_gbase[d] + (q - s_tstart[d]);
@@ -383,7 +429,12 @@ static int run_sort(uint32_t* keys, uint32_t* vals, uint32_t n, int keyBits, voi
     uint32_t* t2k = plan.passes >= 3 ? reinterpret_cast<uint32_t*>(w + L.t2k) : nullptr;
     uint32_t* t2v = plan.passes >= 3 ? reinterpret_cast<uint32_t*>(w + L.t2v) : nullptr;
     const uint32_t tiles = sort_tiles(n);
-    const bool small = sort_items(n) == kSortItemsSmall;
+    const bool small = sort_small(n), scanned = tiles > kSumMaxTiles;
+    const int threads = small ? kSmallThreads : kLargeThreads;
+    const auto upsweep = small ? k_sort_upsweep<kSmallThreads, kSmallItems> : k_sort_upsweep<kLargeThreads, kLargeItems>;
+    const auto pass = !scanned ? k_sort_pass<kSmallThreads, kSmallItems, false>
+                      : small  ? k_sort_pass<kSmallThreads, kSmallItems, true>
+                               : k_sort_pass<kLargeThreads, kLargeItems, true>;
 
     const uint32_t* src_k = keys;
     const uint32_t* src_v = vals;
@@ -398,12 +449,12 @@ static int run_sort(uint32_t* keys, uint32_t* vals, uint32_t n, int keyBits, voi
         } else {
             dk = t2k; dv = t2v;
         }
-        hipLaunchKernelGGL(small ? k_sort_upsweep<kSortItemsSmall> : k_sort_upsweep<kSortItemsLarge>, dim3(tiles),
-                           dim3(kSortThreads), 0, st, src_k, n, plan.shift[p], plan.bits[p], counts, tiles);
-        hipLaunchKernelGGL(k_sort_scan, dim3(1u << plan.bits[p]), dim3(kSortThreads), 0, st, counts, tiles, totals);
-        hipLaunchKernelGGL(small ? k_sort_pass<kSortItemsSmall> : k_sort_pass<kSortItemsLarge>, dim3(tiles),
-                           dim3(kSortThreads), 0, st, src_k, src_v, dk, dv, n, plan.shift[p], plan.bits[p], counts,
-                           tiles, totals, (p == 0 && iota) ? 1 : 0);
+        hipLaunchKernelGGL(upsweep, dim3(tiles), dim3(threads), 0, st, src_k, n, plan.shift[p], plan.bits[p],
+                           counts, tiles, scanned);
+        if (scanned)
+            hipLaunchKernelGGL(k_sort_scan, dim3(1u << plan.bits[p]), dim3(kSortThreads), 0, st, counts, tiles, totals);
+        hipLaunchKernelGGL(pass, dim3(tiles), dim3(threads), 0, st, src_k, src_v, dk, dv, n, plan.shift[p],
+                           plan.bits[p], counts, tiles, totals, (p == 0 && iota) ? 1 : 0);
         src_k = dk;
         src_v = dv;
     }
