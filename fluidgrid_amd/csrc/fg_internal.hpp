@@ -152,6 +152,16 @@ __device__ __forceinline__ int32_t f2i_sat(float v) {
     return (int32_t)v;
 }
 
+// Blocks are handed to the eight XCDs round-robin; remapping them so that each
+// XCD walks one contiguous slice of the sorted particles (or keys) keeps what
+// consecutive blocks share, neighbour rows or parts of a line, in the same L2.
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nblocks) {
+    constexpr uint32_t kXcd = 8;
+    const uint32_t per = nblocks / kXcd, rem = nblocks % kXcd;
+    const uint32_t x = b % kXcd, idx = b / kXcd;
+    return x * per + min(x, rem) + idx;
+}
+
 // Correctly rounded IEEE single operations for the reference-arithmetic
 // code.  They are written as plain operators in a region with contraction
 // off, so no multiply is ever fused into a following add, even after

@@ -17,6 +17,9 @@
 //    the digit base (an exclusive scan of the totals) plus the tile's offset
 //    within the digit (of few tiles, summed here from their counts), and it is
 //    staged in LDS in digit order and written out as coalesced runs.
+// Each XCD takes a run of consecutive tiles: they write next to each other
+// within every digit, and its L2 joins their parts of a 128-byte line (a pass
+// over 33,500,000 keys 189 us with the tiles dealt out in turn, 140 us so).
 // No workgroup waits for another (a single-sweep pass with decoupled
 // look-back chains tiles: at 1M keys the chain, not the bytes, set its
 // time).  Digit widths are chosen from the key width (<= 8 bits per pass),
@@ -175,7 +178,7 @@ __global__ void __launch_bounds__(THREADS) k_sort_upsweep(const uint32_t* __rest
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int i = tid; i < kWaves * kMaxRadix; i += THREADS) (&s_cnt[0][0])[i] = 0;
     __syncthreads();
-    const uint32_t tile = blockIdx.x;
+    const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t dmask = (1u << bits) - 1u;
     const uint32_t wbase = tile * (uint32_t)(THREADS * ITEMS) + (uint32_t)wave * 64u * ITEMS;
     uint32_t key[ITEMS];
@@ -267,7 +270,7 @@ __global__ void __launch_bounds__(THREADS) k_sort_pass(const uint32_t* __restric
     const uint32_t radix = 1u << bits, dmask = radix - 1u;
     for (int i = tid; i < kWaves * kMaxRadix; i += THREADS) (&s_wcnt[0][0])[i] = 0;
     __syncthreads();
-    const uint32_t tile = blockIdx.x;
+    const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t base = tile * (uint32_t)TILE;
     const uint32_t wbase = base + (uint32_t)wave * 64u * ITEMS;
 

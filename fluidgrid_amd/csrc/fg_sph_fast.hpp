@@ -217,16 +217,6 @@ __device__ __forceinline__ bool row_range(const RowWalker& w, int dy, int dz, fl
                       end, n, rb, re);
 }
 
-// Blocks are handed to the eight XCDs round-robin; remapping them so that each
-// XCD walks one contiguous slice of the sorted particles keeps the neighbour
-// rows of consecutive blocks in the same L2.
-__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nblocks) {
-    constexpr uint32_t kXcd = 8;
-    const uint32_t per = nblocks / kXcd, rem = nblocks % kXcd;
-    const uint32_t x = b % kXcd, idx = b / kXcd;
-    return x * per + min(x, rem) + idx;
-}
-
 // Neighbour bitmasks: for each of the 9 stencil rows of a particle, bit k of
 // masks[row * n + i] is set when sorted particle rowBegin + k lies within h.
 // Rows longer than 64 particles are not encoded and are re-tested.
