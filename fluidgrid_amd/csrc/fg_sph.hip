@@ -629,7 +629,7 @@ int launch_density(float4* sp, float2* rho_p, uint32_t* start, uint32_t* end, ui
     }
     if (masks && use_fast()) note_nbr_format(masks, n, st.tiled && !mixed);
     if (mixed)
-        FG_SPH_LAUNCH_BS(k_density_mixed<256>, 256, n, sp, sv, rho_p, start, end, n, k, rho0, m, st.common,
+        FG_SPH_LAUNCH_BS(k_density_mixed<64>, 64, n, sp, sv, rho_p, start, end, n, k, rho0, m, st.common,
                          st.kernels, masks);
     else if (use_fast() && masks && st.tiled)
         hipLaunchKernelGGL(k_density_tile, dim3(grid_for(n, kTileLanes)), dim3(kTileLanes), 0, st.stream, sp, sv,

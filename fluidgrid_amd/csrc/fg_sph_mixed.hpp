@@ -105,14 +105,11 @@ __device__ __forceinline__ uint32_t cull_pair(const uint4& r, half2v tx, half2v 
     return __builtin_bit_cast(uint32_t, d);
 }
 
-// Bits 0..3: candidates j..j+3 survive (records j and j+2).
-__device__ __forceinline__ uint32_t cull_quad(const uint4& r0, const uint4& r1, half2v tx, half2v ty, half2v tz,
-                                              half2v per, half2v ncut) {
-    const short2v m0 = __builtin_bit_cast(short2v, cull_pair(r0, tx, ty, tz, per, ncut)) >> (short)15;
-    const short2v m1 = __builtin_bit_cast(short2v, cull_pair(r1, tx, ty, tz, per, ncut)) >> (short)15;
-    const uint32_t x = (__builtin_bit_cast(uint32_t, m0) & 0x00020001u) |
-                       (__builtin_bit_cast(uint32_t, m1) & 0x00080004u);
-    return (x & 0xFu) | (x >> 16);
+// Shifts the survivor bits of a pair record's two candidates into `bits` from
+// below, the first candidate first: the halves' signs.
+__device__ __forceinline__ uint32_t push_pair(uint32_t bits, uint32_t d) {
+    bits = __builtin_amdgcn_alignbit(bits, d << 16, 31);
+    return __builtin_amdgcn_alignbit(bits, d, 31);
 }
 
 // |p - q|^2 with the operations of density4 (the FP32 pass's test).
@@ -125,94 +122,102 @@ __device__ __forceinline__ float poly6_term(float h2u, float r2) {
     return (t * t) * t;
 }
 
-// sum + comp += x (Neumaier's compensated summation).
+// sum + comp += x (Neumaier's compensated summation), for a sum and an x that
+// are not negative: which is larger in magnitude is then one plain compare.  (A
+// term that the rounding of h^2 leaves just below zero is exact in both forms.)
 __device__ __forceinline__ void neumaier_add(float& sum, float& comp, float x) {
     const float t = sum + x;
-    comp += (fabsf(sum) >= fabsf(x)) ? ((sum - t) + x) : ((x - t) + sum);
+    comp += (sum >= x) ? ((sum - t) + x) : ((x - t) + sum);
     sum = t;
 }
 #pragma clang fp contract(fast)
 
+// A wavefront's staged run: the pair records (the two after the run too: a
+// group of candidates t..t+3 reads the records t and t + 2) and the positions,
+// each as 8 and 4 bytes: lanes read at unrelated offsets, and 16-byte reads of
+// that kind take three to four times the LDS cycles of an 8- and a 4-byte one.
+//
+// Bound by VALU issue: 5,770 instructions a wavefront against the FP32 pass's
+// 4,670, and more of them (packed FP16, compares, selects, bit moves) of those
+// that take 4 cycles and more to issue, so a packed pair of candidates costs
+// what two FP32 ones do.  2,097,152 particles: the step 595 us with 16-byte
+// staging in workgroups of 256, rows loaded when they are needed and survivors
+// four at a time, 585 us so.
+constexpr uint32_t kMixedStage = 128;
+struct MixedStage {
+    uint2 hxy[kMixedStage + 2];
+    float2 xy[kMixedStage];
+    uint32_t hz[kMixedStage + 2];
+    float z[kMixedStage];
+    WaveCells cells;
+};
+static_assert(offsetof(MixedStage, cells) >= sizeof(uint32_t) * kWaveCellsTemp, "wave_cells' temporary words");
+
 // One stencil row of the mixed density pass for one particle: the cull of
 // the row's candidates from their FP16 pair records, then the exact FP32
-// test and compensated sum of the survivors.  H and P are the pair records
-// and sorted positions from the row's first candidate, in memory or (LDS)
-// staged.
+// test and compensated sum of the survivors.  `at` is the row's first
+// candidate, in the staged run or (LDS false) among the sorted arrays.
 struct MixedRow {
     float4 p;
     half2v tx, per, ncut;
     float hhu, h2u;
     float sum, comp;
+    const MixedStage& st;
+    const uint4* __restrict__ H;
+    const float4* __restrict__ P;
 
-    // The survivors among candidates P[bits of word], four per iteration
-    // with their loads issued together; returns the bits of those within h
-    // (the FP32 test of density4).
+    // The survivors among the candidates at + (bits of word); returns the bits
+    // of those within h (the FP32 test of density4).
     template <bool LDS>
-    __device__ __forceinline__ uint32_t exact(uint32_t word, const float4* __restrict__ P) {
-        auto ld = [](const float4* q) { return LDS ? ld_xyz_lds(q) : ld_xyz(q); };
+    __device__ __forceinline__ uint32_t exact(uint32_t word, uint32_t at) {
         uint32_t hits = 0u;
         while (word) {
-            const uint32_t k0 = (uint32_t)__builtin_ctz(word);
-            word &= word - 1u;
-            const bool v1 = word != 0u;
-            const uint32_t k1 = v1 ? (uint32_t)__builtin_ctz(word) : k0;
-            word &= word - 1u;
-            const bool v2 = word != 0u;
-            const uint32_t k2 = v2 ? (uint32_t)__builtin_ctz(word) : k0;
-            word &= word - 1u;
-            const bool v3 = word != 0u;
-            const uint32_t k3 = v3 ? (uint32_t)__builtin_ctz(word) : k0;
-            word &= word - 1u;
-            const float3 q0 = ld(P + k0), q1 = ld(P + k1);
-            const float3 q2 = ld(P + k2), q3 = ld(P + k3);
-            const float r0 = exact_r2(p, q0), r1 = exact_r2(p, q1);
-            const float r2 = exact_r2(p, q2), r3 = exact_r2(p, q3);
-            if (r0 < hhu) {
-                neumaier_add(sum, comp, poly6_term(h2u, r0));
-                hits |= 1u << k0;
-            }
-            if (v1 && r1 < hhu) {
-                neumaier_add(sum, comp, poly6_term(h2u, r1));
-                hits |= 1u << k1;
-            }
-            if (v2 && r2 < hhu) {
-                neumaier_add(sum, comp, poly6_term(h2u, r2));
-                hits |= 1u << k2;
-            }
-            if (v3 && r3 < hhu) {
-                neumaier_add(sum, comp, poly6_term(h2u, r3));
-                hits |= 1u << k3;
-            }
+            const uint32_t k = (uint32_t)__builtin_ctz(word), rest = word & (word - 1u);
+            float3 q;
+            if (LDS) {
+                const float2 xy = st.xy[at + k];
+                q = make_float3(xy.x, xy.y, st.z[at + k]);
+            } else
+                q = ld_xyz(P + at + k);
+            const float r2 = exact_r2(p, q);
+            const bool hit = r2 < hhu;
+            neumaier_add(sum, comp, hit ? poly6_term(h2u, r2) : 0.0f);
+            hits |= hit ? word ^ rest : 0u;
+            word = rest;
         }
         return hits;
     }
 
-    // Survivor bits of the cnt (<= 32) candidates from H[0].  (Keeping the
-    // next group's records in flight, eight candidates per iteration, needs
-    // 76 VGPRs and was no faster: the loop is bound by issue, not latency.)
-    __device__ __forceinline__ uint32_t cull_word(const uint4* __restrict__ H, uint32_t cnt, half2v ty,
-                                                  half2v tz) const {
-        uint32_t word = 0u;
-        for (uint32_t t = 0; t < cnt; t += 4) {
-            const uint4 r0 = H[t], r1 = H[t + 2];
-            word |= cull_quad(r0, r1, tx, ty, tz, per, ncut) << t;
+    // Survivor bits of the cnt (<= 32) candidates from `at`.
+    template <bool LDS>
+    __device__ __forceinline__ uint32_t cull_word(uint32_t at, uint32_t cnt, half2v ty, half2v tz) const {
+        uint32_t bits = 0u, t = 0u;
+        for (; t < cnt; t += 4) {
+            uint4 r0, r1;
+            if (LDS) {
+                const uint2 a = st.hxy[at + t], b = st.hxy[at + t + 2];
+                r0 = make_uint4(a.x, a.y, st.hz[at + t], 0u);
+                r1 = make_uint4(b.x, b.y, st.hz[at + t + 2], 0u);
+            } else {
+                r0 = H[at + t];
+                r1 = H[at + t + 2];
+            }
+            bits = push_pair(bits, cull_pair(r0, tx, ty, tz, per, ncut));
+            bits = push_pair(bits, cull_pair(r1, tx, ty, tz, per, ncut));
         }
+        if (t == 0u) return 0u;
+        const uint32_t word = __builtin_bitreverse32(bits) >> (32u - t);  // candidate j was shifted in as bit t - 1 - j
         return cnt < 32u ? word & ((1u << cnt) - 1u) : word;
     }
 
     // The row's mask: 64 candidates at a time; a row longer than 64 is never
     // read through its mask (the force pass re-tests it), which is 0.
     template <bool LDS>
-    __device__ __forceinline__ unsigned long long row(const uint4* __restrict__ H, const float4* __restrict__ P,
-                                                      uint32_t len, half2v ty, half2v tz) {
+    __device__ __forceinline__ unsigned long long row(uint32_t at, uint32_t len, half2v ty, half2v tz) {
         unsigned long long msk = 0ull;
-        for (uint32_t c0 = 0; c0 < len; c0 += 64u) {
-            const uint32_t l = min(len - c0, 64u);
-            const uint32_t w0 = cull_word(H + c0, min(l, 32u), ty, tz);
-            const uint32_t w1 = l > 32u ? cull_word(H + c0 + 32u, l - 32u, ty, tz) : 0u;
-            const uint32_t e0 = exact<LDS>(w0, P + c0);
-            const uint32_t e1 = exact<LDS>(w1, P + c0 + 32u);
-            msk = (unsigned long long)e0 | ((unsigned long long)e1 << 32);
+        for (uint32_t c0 = 0; c0 < len; c0 += 32u) {
+            const uint32_t w = cull_word<LDS>(at + c0, min(len - c0, 32u), ty, tz);
+            msk |= (unsigned long long)exact<LDS>(w, at + c0) << (c0 & 32u);
         }
         return len > kRowMaskBits ? 0ull : msk;
     }
@@ -227,13 +232,6 @@ struct MixedRow {
 // records and positions is staged there first, as in density_rows_staged;
 // every lane then takes part (the lane of an inactive particle, or one past
 // the last particle, with no rows), and the runs are left for the force pass.
-constexpr uint32_t kMixedStage = 128;
-struct MixedStage {
-    uint4 rec[kMixedStage + 4];
-    float4 pos[kMixedStage];
-    WaveCells cells;
-};
-static_assert(offsetof(MixedStage, cells) >= sizeof(uint32_t) * kWaveCellsTemp, "wave_cells' temporary words");
 __device__ __forceinline__ void density_particle_mixed(uint32_t i, const float4* __restrict__ sp,
                                                        const float4* __restrict__ sv, float2* __restrict__ rho_p,
                                                        const uint32_t* __restrict__ start,
@@ -253,7 +251,7 @@ __device__ __forceinline__ void density_particle_mixed(uint32_t i, const float4*
     const RowWalker w = make_rows(p, cp);
     uint32_t cell, words = kRunGeneric;
     WaveRuns runs;
-    const bool ok = wave_cells(st.cells, reinterpret_cast<uint32_t*>(st.rec), 64u, w, cp, 0u, start, end, n, cell, runs);
+    const bool ok = wave_cells(st.cells, reinterpret_cast<uint32_t*>(st.hxy), 64u, w, cp, 0u, start, end, n, cell, runs);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(i >> 6);
     const bool table = n >= kRunMinParticles;
     uint16_t* offs = nbr_offs(masks, n) + (size_t)9 * 64 * wave + lane;
@@ -267,7 +265,30 @@ __device__ __forceinline__ void density_particle_mixed(uint32_t i, const float4*
                hhu,
                h2u,
                0.0f,
-               0.0f};
+               0.0f,
+               st,
+               hr,
+               sp};
+    // the next row's records and positions, loaded while a row is walked
+    uint4 h0 = make_uint4(0u, 0u, 0u, 0u), h1 = h0;
+    float3 p0 = make_float3(0.0f, 0.0f, 0.0f), p1 = p0;
+    auto fetch = [&](int row) {
+        const uint32_t len = runs.word(row), lo = runs.first(row);
+        if (!ok || len > kMixedStage) return;
+        if (lane < len + 2u) h0 = hr[lo + lane];
+        if (lane + 64u < len + 2u) h1 = hr[lo + lane + 64u];
+        if (lane < len) p0 = ld_xyz(sp + lo + lane);
+        if (lane + 64u < len) p1 = ld_xyz(sp + lo + lane + 64u);
+    };
+    auto put = [&](uint32_t q, const uint4& h, const float3& pos, bool candidate) {
+        st.hxy[q] = make_uint2(h.x, h.y);
+        st.hz[q] = h.z;
+        if (candidate) {
+            st.xy[q] = make_float2(pos.x, pos.y);
+            st.z[q] = pos.z;
+        }
+    };
+    fetch(0);
 
     for (int row = 0; row < 9; row++) {
         const int dz = row / 3 - 1, dy = row % 3 - 1;
@@ -289,18 +310,17 @@ __device__ __forceinline__ void density_particle_mixed(uint32_t i, const float4*
             has = active && row_range(w, dy, dz, cut, cp, 0u, start, end, n, rb, re);
         }
         if (staged) {
-            // the pair records of the run and the two after it (a quad of
-            // candidates reads the records t and t + 2), and the positions
-            for (uint32_t q = lane; q < len + 2u; q += 64u) st.rec[q] = hr[lo + q];
-            for (uint32_t q = lane; q < len; q += 64u) st.pos[q] = sp[lo + q];
+            if (lane < len + 2u) put(lane, h0, p0, lane < len);
+            if (lane + 64u < len + 2u) put(lane + 64u, h1, p1, lane + 64u < len);
+            if (lane + 128u < len + 2u) put(lane + 128u, hr[lo + lane + 128u], p0, false);
             wave_lds_sync();
         }
+        if (row < 8) fetch(row + 1);
         unsigned long long msk = 0ull;
         if (has) {
             const half2v ty = {(_Float16)(o.y - (float)dy * g.wy), (_Float16)(o.y - (float)dy * g.wy)};
             const half2v tz = {(_Float16)(o.z - (float)dz * g.wz), (_Float16)(o.z - (float)dz * g.wz)};
-            msk = staged ? M.row<true>(st.rec + (rb - lo), st.pos + (rb - lo), re - rb, ty, tz)
-                         : M.row<false>(hr + rb, sp + rb, re - rb, ty, tz);
+            msk = staged ? M.row<true>(rb - lo, re - rb, ty, tz) : M.row<false>(rb, re - rb, ty, tz);
         }
         if (active) masks[(size_t)row * n + i] = msk;
         if (staged) wave_lds_sync();  // every lane's reads of this row before the next row's stores
