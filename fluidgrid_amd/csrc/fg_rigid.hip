@@ -227,33 +227,41 @@ __global__ void k_integrate_rb(float4* __restrict__ pos, const float* __restrict
 constexpr int kReduceThreads = 256;
 constexpr int kBodySumThreads = 1024;  // 20K spheres: 20 loads per lane, unrolled
 
+// Workgroup (b, 0) sums body b's forces, (b, 1) its torques: one CU reads no more
+// than about 64 bytes a cycle, which is what bounds a body of 20K spheres.
 __global__ void __launch_bounds__(kBodySumThreads)
     k_body_reduce_f64(const float4* __restrict__ f, const float4* __restrict__ t, const uint32_t* __restrict__ offset,
                       uint32_t nbodies, double4* __restrict__ out_f, double4* __restrict__ out_t,
                       float4* __restrict__ acc_f, float4* __restrict__ acc_t) {
-    __shared__ double s[6][kBodySumThreads];
+    __shared__ double s[3][kBodySumThreads];
     const uint32_t b = blockIdx.x;
     if (b >= nbodies) return;
+    const bool torque = blockIdx.y != 0;
+    const float4* __restrict__ in = torque ? t : f;
     const uint32_t lo = offset[b], hi = offset[b + 1];
-    double a[6] = {0, 0, 0, 0, 0, 0};
-#pragma unroll 4
+    double a[3] = {0, 0, 0};
+#pragma unroll 8
     for (uint32_t i = lo + threadIdx.x; i < hi; i += kBodySumThreads) {
-        const float4 fi = f[i], ti = t[i];
-        a[0] += fi.x; a[1] += fi.y; a[2] += fi.z;
-        a[3] += ti.x; a[4] += ti.y; a[5] += ti.z;
+        const float4 v = in[i];
+        a[0] += v.x; a[1] += v.y; a[2] += v.z;
     }
-    for (int k = 0; k < 6; k++) s[k][threadIdx.x] = a[k];
+    for (int k = 0; k < 3; k++) s[k][threadIdx.x] = a[k];
     __syncthreads();
-    for (int w = kBodySumThreads / 2; w > 0; w >>= 1) {
+    for (int w = kBodySumThreads / 2; w >= 64; w >>= 1) {
         if ((int)threadIdx.x < w)
-            for (int k = 0; k < 6; k++) s[k][threadIdx.x] += s[k][threadIdx.x + w];
+            for (int k = 0; k < 3; k++) s[k][threadIdx.x] += s[k][threadIdx.x + w];
         __syncthreads();
     }
+    if (threadIdx.x >= 64) return;
+    for (int k = 0; k < 3; k++) {  // the last six levels in one wavefront
+        a[k] = s[k][threadIdx.x];
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) a[k] += __shfl_down(a[k], w);
+    }
     if (threadIdx.x == 0) {
-        out_f[b] = make_double4(s[0][0], s[1][0], s[2][0], 0.0);
-        out_t[b] = make_double4(s[3][0], s[4][0], s[5][0], 0.0);
-        if (acc_f) acc_f[b] = make_float4((float)s[0][0], (float)s[1][0], (float)s[2][0], 0.0f);
-        if (acc_t) acc_t[b] = make_float4((float)s[3][0], (float)s[4][0], (float)s[5][0], 0.0f);
+        (torque ? out_t : out_f)[b] = make_double4(a[0], a[1], a[2], 0.0);
+        float4* __restrict__ acc = torque ? acc_t : acc_f;
+        if (acc) acc[b] = make_float4((float)a[0], (float)a[1], (float)a[2], 0.0f);
     }
 }
 
@@ -308,29 +316,35 @@ __global__ void __launch_bounds__(kReduceThreads)
 // Bounds of all sphere centres, expanded by `margin`: out[0] = min, out[1] = max.
 __global__ void __launch_bounds__(1024) k_sphere_bounds(const float4* __restrict__ p, uint32_t m, float margin,
                                                         float4* __restrict__ out) {
-    __shared__ float s[6][1024];
+    __shared__ float s[6][1024 / 64];
     float lo[3] = {3.0e38f, 3.0e38f, 3.0e38f}, hi[3] = {-3.0e38f, -3.0e38f, -3.0e38f};
+#pragma unroll 8
     for (uint32_t i = threadIdx.x; i < m; i += 1024) {
         const float4 q = p[i];
         lo[0] = fminf(lo[0], q.x); lo[1] = fminf(lo[1], q.y); lo[2] = fminf(lo[2], q.z);
         hi[0] = fmaxf(hi[0], q.x); hi[1] = fmaxf(hi[1], q.y); hi[2] = fmaxf(hi[2], q.z);
     }
+    const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     for (int k = 0; k < 3; k++) {
-        s[k][threadIdx.x] = lo[k];
-        s[3 + k][threadIdx.x] = hi[k];
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) {
+            lo[k] = fminf(lo[k], __shfl_xor(lo[k], w));
+            hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], w));
+        }
+        if (lane == 0) {
+            s[k][wave] = lo[k];
+            s[3 + k][wave] = hi[k];
+        }
     }
     __syncthreads();
-    for (int w = 512; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int k = 0; k < 3; k++) {
-                s[k][threadIdx.x] = fminf(s[k][threadIdx.x], s[k][threadIdx.x + w]);
-                s[3 + k][threadIdx.x] = fmaxf(s[3 + k][threadIdx.x], s[3 + k][threadIdx.x + w]);
-            }
-        __syncthreads();
-    }
     if (threadIdx.x == 0) {
-        out[0] = make_float4(s[0][0] - margin, s[1][0] - margin, s[2][0] - margin, 0.0f);
-        out[1] = make_float4(s[3][0] + margin, s[4][0] + margin, s[5][0] + margin, 0.0f);
+        for (int w = 1; w < 16; w++)
+            for (int k = 0; k < 3; k++) {
+                lo[k] = fminf(lo[k], s[k][w]);
+                hi[k] = fmaxf(hi[k], s[3 + k][w]);
+            }
+        out[0] = make_float4(lo[0] - margin, lo[1] - margin, lo[2] - margin, 0.0f);
+        out[1] = make_float4(hi[0] + margin, hi[1] + margin, hi[2] + margin, 0.0f);
     }
 }
 
@@ -896,7 +910,7 @@ int fg_body_reduce_f64(const fg_float4* forces, const fg_float4* torques, const 
         set_error(FG_ERR_INVALID_ARGUMENT, "fg_body_reduce_f64: null pointer");
         return FG_ERR_INVALID_ARGUMENT;
     }
-    hipLaunchKernelGGL(k_body_reduce_f64, dim3(numBodies), dim3(kBodySumThreads), 0, state().stream,
+    hipLaunchKernelGGL(k_body_reduce_f64, dim3(numBodies, 2), dim3(kBodySumThreads), 0, state().stream,
                        reinterpret_cast<const float4*>(forces), reinterpret_cast<const float4*>(torques), bodyOffsets,
                        numBodies, reinterpret_cast<double4*>(outForces), reinterpret_cast<double4*>(outTorques),
                        accForces ? FG_F4(accForces) : nullptr, accTorques ? FG_F4(accTorques) : nullptr);
