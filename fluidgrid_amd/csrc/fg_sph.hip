@@ -32,8 +32,8 @@ constexpr int kSphThreads = 256;
 // the GPU and keep eight bucket walks in flight; above, one lane a particle
 // already does, and the groups' adding up costs more than it gains.  Measured
 // with the reference's hash (density / forces, us):
-//   24,108 particles   1 lane 51 / 90     8 lanes 15 / 31    16 lanes 15 / 31
-//   108,000            1 lane 60 / 141    8 lanes 48 / 100   16 lanes 49 / 109
+//   24,108 particles   1 lane 51 / 90     8 lanes 14 / 24    16 lanes 15 / 31
+//   108,000            1 lane 60 / 141    8 lanes 51 / 92    16 lanes 49 / 109
 //   250,880            1 lane 98 / 185    8 lanes 125 / 212  16 lanes 131 / 249
 //   1,048,576          1 lane 358 / 593   8 lanes 647 / 970
 constexpr uint32_t kRefLanes = 8;
@@ -77,7 +77,7 @@ __device__ __forceinline__ bool stencil_bucket(const float4& p, const CellXYZ& c
 // bucket's particles are).
 //
 // Bound by latency in small fluids and by VALU issue in large ones: a fluid
-// of 24,108 particles with hashed keys takes 15 (density) and 31 us (forces),
+// of 24,108 particles with hashed keys takes 14 (density) and 24 us (forces),
 // where one lane a particle, a powf a pair and every particle's terms under
 // one branch took 105 and 109; 1,048,576 particles take 358 and 593 us, then
 // 972 and 1,115.
@@ -155,19 +155,41 @@ __global__ void __launch_bounds__(kSphThreads)
     if (lane == 0u) rho_p[i] = make_float2(fmaxf(1.0f, rho), k * (rho - rho0));
 }
 
-// Pressure + viscosity between particle i and the particles of one bucket
-// (K_FluidSim.cu:85-172).
-__device__ __forceinline__ F3 bucket_internal_ref(uint32_t i, uint32_t s0, uint32_t e, const F3& p1, const float4& vel,
-                                                  float2 dp1, const float4* __restrict__ sp,
-                                                  const float4* __restrict__ sv, const float2* __restrict__ rho_p,
-                                                  float s, float h, float cut, float kSpiky, float kVisc, float mu) {
-    F3 total = f3(0.0f, 0.0f, 0.0f);
-    const F3 v1 = xyz(vel);
-    for (uint32_t b0 = s0; b0 < e; b0 += 32u) {
-        // the particles that may be within h, then only those: the terms'
-        // seven divisions are worth the second look at them
-        const uint32_t cnt = min(e - b0, 32u);
-        uint32_t near = 0u;
+// Each lane's sums of one of its four buckets.
+struct RefPart {
+    float x[64], y[64], z[64];
+};
+
+// What the pair terms of particle i read, and the terms of one neighbour
+// (K_FluidSim.cu:85-172) added to `total`.
+struct RefPair {
+    F3 p1, v1;
+    float2 dp1;
+    const float4* __restrict__ sp;
+    const float4* __restrict__ sv;
+    const float2* __restrict__ rho_p;
+    float s, h, cut, kSpiky, kVisc, mu;
+
+    __device__ __forceinline__ void add_terms(F3& total, uint32_t j) const {
+        const float2 dp2 = rho_p[j];
+        const F3 v2 = xyz(sv[j]);
+        const F3 diff = sub(p1, mul(xyz(sp[j]), s));
+        const float l = rn_sqrt(dot(diff, diff));
+        if (l > h) return;  // both terms are zero
+        // SPHCalculatePressureForceD, K_FluidSim.cu:107-120
+        const float rr = dp1.x * dp2.x;
+        const float pp = (dp1.y + dp2.y) / rr;
+        const float r = kSpiky * ((h - l) * (h - l));
+        total = add(total, mul(mul(mul(divs(diff, l), r), pp), -1.0f));
+        // SPHCalculateViscosityForceD, K_FluidSim.cu:85-102
+        const float lap = kVisc * (h - l);
+        total = add(total, f3(((v2.x - v1.x) / rr) * lap * mu, ((v2.y - v1.y) / rr) * lap * mu,
+                              ((v2.z - v1.z) / rr) * lap * mu));
+    }
+
+    // Bits of the cnt (<= 32) particles from b0 that may be within h.
+    __device__ __forceinline__ uint32_t near(uint32_t b0, uint32_t cnt) const {
+        uint32_t bits = 0u;
         for (uint32_t k = 0; k < cnt; k += 4u) {
             float4 cand[4];
 #pragma unroll
@@ -175,31 +197,23 @@ __device__ __forceinline__ F3 bucket_internal_ref(uint32_t i, uint32_t s0, uint3
 #pragma unroll
             for (uint32_t u = 0; u < 4u; u++) {
                 const F3 d = sub(p1, mul(xyz(cand[u]), s));
-                near |= k + u < cnt && !(dot(d, d) > cut) ? 1u << (k + u) : 0u;
+                bits |= k + u < cnt && !(dot(d, d) > cut) ? 1u << (k + u) : 0u;
             }
         }
-        if (i >= b0 && i - b0 < 32u) near &= ~(1u << (i - b0));
-        while (near) {
-            const uint32_t j = b0 + (uint32_t)__builtin_ctz(near);
-            near &= near - 1u;
-            const float2 dp2 = rho_p[j];
-            const F3 v2 = xyz(sv[j]);
-            const F3 diff = sub(p1, mul(xyz(sp[j]), s));
-            const float l = rn_sqrt(dot(diff, diff));
-            if (l > h) continue;  // both terms are zero
-            // SPHCalculatePressureForceD, K_FluidSim.cu:107-120
-            const float rr = dp1.x * dp2.x;
-            const float pp = (dp1.y + dp2.y) / rr;
-            const float r = kSpiky * ((h - l) * (h - l));
-            total = add(total, mul(mul(mul(divs(diff, l), r), pp), -1.0f));
-            // SPHCalculateViscosityForceD, K_FluidSim.cu:85-102
-            const float lap = kVisc * (h - l);
-            total = add(total, f3(((v2.x - v1.x) / rr) * lap * mu, ((v2.y - v1.y) / rr) * lap * mu,
-                                  ((v2.z - v1.z) / rr) * lap * mu));
-        }
+        return bits;
     }
-    return total;
-}
+
+    // Sum over the particles [s0, e) of a bucket of any length.
+    __device__ __forceinline__ F3 bucket(uint32_t i, uint32_t s0, uint32_t e) const {
+        F3 total = f3(0.0f, 0.0f, 0.0f);
+        for (uint32_t b0 = s0; b0 < e; b0 += 32u) {
+            uint32_t w = near(b0, min(e - b0, 32u));
+            if (i - b0 < 32u) w &= ~(1u << (i - b0));
+            for (; w; w &= w - 1u) add_terms(total, b0 + (uint32_t)__builtin_ctz(w));
+        }
+        return total;
+    }
+};
 
 // K_FluidSim.cu:260-309 (+ fused integrate when pout != nullptr); with
 // COUPLED, K_FluidSim.cu:315-413.  By groups of LP lanes, as k_density_ref.
@@ -217,22 +231,77 @@ __global__ void __launch_bounds__(kSphThreads)
     if (pos.w > 0.0f) {
         const float2 dp1 = rho_p[i];
         const uint32_t nb = dev_num_buckets(cp);
-        const float s = cp.simulation_scale, h = cp.kernel_radius, cut = ref_cut(h);
+        const float s = cp.simulation_scale, h = cp.kernel_radius;
         CellXYZ c{0, 0, 0};
         if (MODE == FG_KEY_LINEAR) c = linear_cell(pos.x, pos.y, pos.z, cp);
-        const F3 p1 = mul(xyz(pos), s);
+        const RefPair pair{mul(xyz(pos), s), xyz(vel), dp1, sp, sv, rho_p, s, h, ref_cut(h), kc.kSpikyGradient,
+                           kc.kViscosityLaplacian, mu};
         F3 internal = f3(0.0f, 0.0f, 0.0f);
-        for (uint32_t r0 = 0; r0 < 27u; r0 += LP) {
-            const int q = (int)(r0 + lane);
-            F3 part = f3(0.0f, 0.0f, 0.0f);
+        for (uint32_t q = 0; LP == 1u && q < 27u; q++) {
             uint32_t b;
-            if (q < 27 && stencil_bucket<MODE>(pos, c, q % 3 - 1, (q / 3) % 3 - 1, q / 9 - 1, cp, nb, b)) {
-                const uint32_t s0 = start[b], e0 = end[b];
-                if (s0 != kEmpty)
-                    part = bucket_internal_ref(i, s0, min(e0, n), p1, vel, dp1, sp, sv, rho_p, s, h, cut,
-                                               kc.kSpikyGradient, kc.kViscosityLaplacian, mu);
+            if (!stencil_bucket<MODE>(pos, c, (int)q % 3 - 1, (int)(q / 3u) % 3 - 1, (int)q / 9 - 1, cp, nb, b)) continue;
+            const uint32_t s0 = start[b], e0 = end[b];
+            if (s0 != kEmpty) ref_add_round<LP>(internal, pair.bucket(i, s0, min(e0, n)));
+        }
+        if constexpr (LP > 1u) {
+            static_assert(LP == 1u || 4u * LP >= 27u, "four buckets a lane hold the stencil");
+            __shared__ RefPart s_part[kSphThreads / 64][4];
+            RefPart* const part = s_part[threadIdx.x / 64];
+            const uint32_t wl = threadIdx.x % 64;
+            // Four buckets a lane: where none holds more than 16 particles,
+            // their particles are tested into one mask and those that may be
+            // within h walked as one list, with a sum for each bucket (a
+            // wavefront waits for the longest list, not four times for the
+            // longest bucket; 24,389 particles 30 us bucket by bucket, 24 us
+            // so; 108,288 100 and 92).  One lane a particle walks bucket by
+            // bucket: as lists of four buckets 1,048,576 particles took 983 us
+            // against 594.
+            uint32_t s0[4], cnt[4];
+            bool large = false;
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; u++) {
+                const int q = (int)(u * LP + lane);
+                s0[u] = cnt[u] = 0u;
+                uint32_t b;
+                if (q < 27 && stencil_bucket<MODE>(pos, c, q % 3 - 1, (q / 3) % 3 - 1, q / 9 - 1, cp, nb, b)) {
+                    s0[u] = start[b];
+                    const uint32_t e = min(end[b], n);
+                    cnt[u] = s0[u] != kEmpty && s0[u] < e ? e - s0[u] : 0u;
+                    large |= cnt[u] > 16u;
+                }
             }
-            ref_add_round<LP>(internal, part);
+            uint64_t near = 0;
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; u++) {
+                part[u].x[wl] = part[u].y[wl] = part[u].z[wl] = 0.0f;
+                if (!large) near |= (uint64_t)pair.near(s0[u], cnt[u]) << (16u * u);
+                if (!large && i - s0[u] < cnt[u]) near &= ~(1ull << (16u * u + (i - s0[u])));
+            }
+            F3 sum = f3(0.0f, 0.0f, 0.0f);
+            uint32_t bucket = 4u;
+            for (; near; near &= near - 1u) {
+                const uint32_t k = (uint32_t)__builtin_ctzll(near), u = k >> 4;
+                if (u != bucket) sum = f3(0.0f, 0.0f, 0.0f);
+                bucket = u;
+                pair.add_terms(sum, (u < 2u ? (u == 0u ? s0[0] : s0[1]) : (u == 2u ? s0[2] : s0[3])) + (k & 15u));
+                part[u].x[wl] = sum.x;
+                part[u].y[wl] = sum.y;
+                part[u].z[wl] = sum.z;
+            }
+            if (large) {
+#pragma unroll 1
+                for (uint32_t u = 0; u < 4u; u++) {
+                    const uint32_t a = u < 2u ? (u == 0u ? s0[0] : s0[1]) : (u == 2u ? s0[2] : s0[3]);
+                    const uint32_t m4 = u < 2u ? (u == 0u ? cnt[0] : cnt[1]) : (u == 2u ? cnt[2] : cnt[3]);
+                    const F3 f = pair.bucket(i, a, a + m4);
+                    part[u].x[wl] = f.x;
+                    part[u].y[wl] = f.y;
+                    part[u].z[wl] = f.z;
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; u++)
+                ref_add_round<LP>(internal, f3(part[u].x[wl], part[u].y[wl], part[u].z[wl]));
         }
         // the body contact (fluid_external) with its cells over the same lanes
         F3 ext = f3(0.0f, 0.0f, 0.0f);
