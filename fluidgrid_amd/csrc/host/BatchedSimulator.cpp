@@ -163,9 +163,8 @@ BatchedSimulator::BatchedSimulator(const std::vector<BatchSceneView>& scenes) {
     hip_check(hipStreamCreateWithFlags(&mBodyStream, hipStreamNonBlocking), "hipStreamCreate");
     {
         StreamScope scope(mStream);
-        fg::batch_scene_of(d_descs, (unsigned)mDescs.size(), d_sceneOf, mN);
+        if (fg::batch_scene_of(d_descs, (unsigned)mDescs.size(), d_sceneOf, mN) != FG_OK) fg_check("BatchedSimulator");
     }
-    fg_check("BatchedSimulator");
     for (auto& e : mEv) hip_check(hipEventCreate(&e), "hipEventCreate");
     for (auto& e : mSync) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
     int blk = 256, bits = 8, fd = 0, ff = 0;
