@@ -42,7 +42,7 @@ struct State {
     bool tiled = false;
     // Coupled masked force pass (row loop): body contact of the particles
     // inside a body grid's bounds deferred to a second kernel that walks each
-    // one's body-grid cells on a pair of lanes (fg_set_contact_defer);
+    // one's body-grid cells on a group of lanes (fg_set_contact_defer);
     // results are identical.
     bool defer_contact = true;
     // Arithmetic of the fused density pass (fg_set_precision): FP32, or FP16

@@ -24,6 +24,7 @@
 // look-back chains tiles: at 1M keys the chain, not the bytes, set its
 // time).  Digit widths are chosen from the key width (<= 8 bits per pass),
 // so 16-bit keys take two passes, 22-bit keys three, 25/27-bit keys four.
+#include <algorithm>
 #include <mutex>
 
 #include "fg_internal.hpp"
@@ -110,7 +111,8 @@ static SortLayout make_layout(uint32_t n, int keyBits) {
     if (keyBits < 1) keyBits = 1;
     if (keyBits > 32) keyBits = 32;
     const int max_passes = plan_passes(keyBits, kMinDigitBits);
-    const size_t tiles = sort_tiles(n);
+    // a workspace for n keys also serves fewer of them, in the smaller tiles
+    const size_t tiles = std::max(sort_tiles(n), sort_tiles(std::min(n, kSmallTileMaxN)));
     size_t o = 0;
     L.counters = o; o = align256(o + sizeof(uint32_t) * (kMaxPasses + 1));
     L.totals = o; o = align256(o + sizeof(uint32_t) * kMaxRadix);

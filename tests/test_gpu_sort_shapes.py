@@ -28,3 +28,12 @@ def test_sizes_match_stable_sort(fglib, n, kind, bits):
     k, v = _sorted(fglib, key, bits)
     assert np.array_equal(v, order)
     assert np.array_equal(k, key[order])
+
+
+def test_workspace_of_more_keys_serves_fewer(fglib):
+    """The workspace size does not fall where the tiles grow."""
+    L = fglib.load()
+    for bits in (8, 16, 22, 32):
+        sizes = [L.fg_sort_workspace_size(n, bits) for n in (1, 2048, 131073, 1572863, 1572864, 1572865, 1580000, 4194304,
+                                                             4194305, 8388608)]
+        assert sizes == sorted(sizes)
