@@ -122,7 +122,7 @@ __global__ void __launch_bounds__(BS)
     __shared__ WaveCells s_cells[FLAT ? BS / 64 : 1];
     __shared__ DensityStage s_stage[FLAT ? 1 : BS / 64];
     DensityStage* stage = FLAT ? nullptr : &s_stage[threadIdx.x / 64];
-    FlatRanges fr{s_rb, s_re, (uint32_t)BS, (uint32_t)threadIdx.x, &s_cells[FLAT ? threadIdx.x / 64 : 0]};
+    WaveCells* cells = &s_cells[FLAT ? threadIdx.x / 64 : 0];
     for_each_particle<BS, PERSIST>(q, n, [&](uint32_t i) {
         for_each_scene(scene_of[i], nscenes, [&](uint32_t s, auto whole) {
             const fg_scene_desc& d = scenes[s];
@@ -130,6 +130,8 @@ __global__ void __launch_bounds__(BS)
                 rho_p[i] = make_float2(__builtin_nanf(""), __builtin_nanf(""));
                 return;
             }
+            // What lanes look up for each other holds within one scene's grid only.
+            FlatRanges fr{s_rb, s_re, (uint32_t)BS, (uint32_t)threadIdx.x, whole ? cells : nullptr};
             density_particle<true>(i, sp, sv, rho_p, start, end, n, d.gasConstant, d.restDensity, d.mass, d.common,
                                    d.kernels, d.keyBase, masks, FLAT ? &fr : nullptr, whole ? stage : nullptr);
         });

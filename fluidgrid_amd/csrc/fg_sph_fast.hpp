@@ -773,7 +773,7 @@ struct FlatRanges {
     uint32_t* rb;  // [9][lanes]
     uint32_t* re;  // [9][lanes]
     uint32_t lanes, lane;
-    WaveCells* cells;  // the wavefront's
+    WaveCells* cells;  // the wavefront's; null unless its particles are all of one grid
     __device__ __forceinline__ uint32_t& b(int r) { return rb[r * lanes + lane]; }
     __device__ __forceinline__ uint32_t& e(int r) { return re[r * lanes + lane]; }
 };
@@ -817,7 +817,7 @@ __device__ __forceinline__ void density_particle(uint32_t i, const float4* __res
         }
         return;
     }
-    if (flat && whole && MASKS && n >= kRunMinParticles) {
+    if (flat && flat->cells && whole && MASKS && n >= kRunMinParticles) {
         // the runs for a force pass that walks rows
         const RowWalker w = make_rows(p, cp);
         const float cut = cp.kernel_radius * cp.kernel_radius * 1.0001f;
