@@ -40,6 +40,11 @@ namespace fg {
 constexpr int kMeshPts = 2;
 constexpr int kMeshWaves = 16;
 static_assert(kMeshWaves >= kMeshPts, "a wavefront for each of a lane's points adds the sums");
+// Workgroups along x: a launch has fewer than 2^32 lanes in each dimension, so
+// a lattice of more groups of points (268,435,456 points; half of that where
+// they lie one to a row) goes on along y.
+constexpr uint64_t kMeshMaxX = 1ull << 21;
+static_assert(kMeshMaxX * 64 * kMeshWaves < (1ull << 32), "lanes along x");
 
 #pragma clang fp contract(off)
 // Lattice point (ix, iy, iz): origin + i * spacing per axis, product and sum
@@ -86,7 +91,9 @@ __global__ void __launch_bounds__(64 * kMeshWaves)
     const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     // the lane's points: kMeshPts neighbours in x, of one row of the lattice
     const uint32_t row_groups = nx / kMeshPts + (nx % kMeshPts != 0);
-    const uint64_t g = (uint64_t)blockIdx.x * 64 + lane, row = g / row_groups;
+    const uint64_t first = ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * 64;
+    if (first >= (uint64_t)row_groups * ny * nz) return;  // past the lattice, the whole workgroup
+    const uint64_t g = first + lane, row = g / row_groups;
     const uint32_t ix = (uint32_t)(g % row_groups) * kMeshPts;
     const float3 p0 = mesh_lattice_point(origin, spacing, ix, (uint32_t)(row % ny), (uint32_t)(row / ny));
     float px[kMeshPts];
@@ -163,8 +170,9 @@ int fg_mesh_winding_lattice(const fg_float3* vertices, unsigned int numVertices,
     }
     const State& st = state();
     const uint64_t groups = (uint64_t)(nx / kMeshPts + (nx % kMeshPts != 0)) * ny * nz;
-    hipLaunchKernelGGL(k_mesh_winding, dim3((unsigned)((groups + 63) / 64)), dim3(64 * kMeshWaves), 0, st.stream, vertices,
-                       numVertices, triangles, numTriangles, origin, spacing, nx, ny, nz, winding);
+    const uint64_t blocks = (groups + 63) / 64, x = blocks < kMeshMaxX ? blocks : kMeshMaxX;
+    hipLaunchKernelGGL(k_mesh_winding, dim3((unsigned)x, (unsigned)((blocks + x - 1) / x)), dim3(64 * kMeshWaves), 0,
+                       st.stream, vertices, numVertices, triangles, numTriangles, origin, spacing, nx, ny, nz, winding);
     return check_launch("fg_mesh_winding_lattice") ? FG_OK : fg_peek_error();
 }
 

@@ -107,8 +107,8 @@ void launch(K kernel, dim3 grid, dim3 block, A... args) {
     gdim = grid;
     bdim = block;
     body = [=] { kernel(args...); };
-    for (uint32_t b = 0; b < grid.x; b++) {
-        bid = dim3(b, 0, 0);
+    for (uint64_t b = 0; b < (uint64_t)grid.x * grid.y; b++) {
+        bid = dim3((uint32_t)(b % grid.x), (uint32_t)(b / grid.x), 0);
         lanes.clear();
         lanes.resize(block.x);
         for (Lane& l : lanes) {
