@@ -14,7 +14,7 @@
 // Every lattice point is independent and reads every triangle, an all-pairs
 // shape.  The wavefronts of a workgroup share 64 * kMeshPts lattice points,
 // kMeshPts neighbours of a row a lane, and a tile of triangles staged in LDS;
-// each takes every kMeshWaves-th triangle of the tile (LDS broadcasts), and the
+// each takes every WAVES-th triangle of the tile (LDS broadcasts), and the
 // wavefronts' sums are added at the end, so a lattice of few points fills the
 // chip too.  The per-point sums are FP64, so adding thousands of terms adds no
 // error of its own.
@@ -22,24 +22,38 @@
 // The work is bound by the instructions of a pair.  For most of them the
 // triangle is small and far: with the triangle's normal n = (b - a) x (c - a)
 // staged beside its corners the numerator is a.n (and free of the
-// cancellation of a.(b x c)), and where it is under 1/8 of the denominator
-// the arc tangent is three terms of its series, 7e-9 of the value at most
-// from the whole (about 40 instructions a pair).  Other pairs, next to the
-// surface, take the numerator from the corners and atan2f.  Square roots and
-// the reciprocal are the 1-ulp instructions.  20,000 triangles on 259,308
+// cancellation of a.(b x c)), and where it is under 1/8 of a denominator of
+// positive terms the arc tangent is three terms of its series, 7e-9 of the
+// value at most from the whole, with 1-ulp roots and reciprocal (about 40
+// instructions a pair).  Other pairs, next to the surface, take exact roots,
+// the numerator from the corners and atan2f.  20,000 triangles on 259,308
 // points: 16.1 ms when every pair took the long way on its own, 4.9 ms so; on
-// 12,716 points 12.0 and 0.75 ms.
+// 12,716 points 12.0 and 0.75 ms.  Mean error against 64 bits on lattices
+// through and around a mesh: 200 triangles 9.3e-9 the long way and 8.3e-9 so,
+// 2,400 triangles 8.2e-9 and 2.4e-9.
+//
+// Of few triangles, large beside the lattice, most wavefronts have a near pair
+// among each triangle's, and the short way before it is work on top: up to
+// kMeshNearTris every pair takes the long way, four wavefronts a workgroup
+// (their sums cost more than the pairs with sixteen).  On 8,000,000 points,
+// both ways of a pair in sixteen wavefronts against the long way in four: 12
+// triangles 483 and 240 us, 32 604 and 577, 64 832 and 1,115, 200 1,716 and
+// 3,411.  The rule lies above where the times cross, where the errors do: the
+// 1-ulp roots of pairs at under 1/8 add up to more than exact ones where there
+// are few others (mean error of a 12-triangle box 3.5e-8 the long way; with
+// 1-ulp roots throughout 5.1e-8).
 #include "fg_internal.hpp"
 
 namespace fg {
 
-// Points a lane and wavefronts a workgroup.  20,000 triangles on 259,308 and
-// on 12,716 points: 2 and 16 4.86 and 0.75 ms; 2 and 8 5.01 and 0.94; 3 and 16
+// Points a lane, and wavefronts a workgroup of many triangles.  20,000 triangles
+// on 259,308 and on 12,716 points: 2 and 16 4.86 and 0.75 ms; 2 and 8 5.01 and 0.94; 3 and 16
 // 5.09 and 1.00; 4 and 16 5.54 and 1.29; one point a lane 10.9 and 0.84 (LDS
 // reads).
 constexpr int kMeshPts = 2;
-constexpr int kMeshWaves = 16;
-static_assert(kMeshWaves >= kMeshPts, "a wavefront for each of a lane's points adds the sums");
+constexpr int kMeshWaves = 16, kMeshNearWaves = 4;
+constexpr uint32_t kMeshNearTris = 128;
+static_assert(kMeshNearWaves >= kMeshPts, "a wavefront for each of a lane's points adds the sums");
 // Workgroups along x: a launch has fewer than 2^32 lanes in each dimension, so
 // a lattice of more groups of points (268,435,456 points; half of that where
 // they lie one to a row) goes on along y.
@@ -54,40 +68,58 @@ __device__ __forceinline__ float3 mesh_lattice_point(fg_float3 o, float s, uint3
 }
 #pragma clang fp contract(fast)
 
-// One triangle's half solid angle seen from (px, py, pz); (v0.w, v1.w, v2.w)
-// is its normal.  The x terms come last in every sum, so points that share
-// py and pz share the rest.
+// One triangle's half solid angle seen from (px, py, pz), the long way.
+__device__ __forceinline__ float half_solid_angle_near(float px, float py, float pz, float4 v0, float4 v1, float4 v2) {
+    const float ax = v0.x - px, ay = v0.y - py, az = v0.z - pz;
+    const float bx = v1.x - px, by = v1.y - py, bz = v1.z - pz;
+    const float cx = v2.x - px, cy = v2.y - py, cz = v2.z - pz;
+    const float la = sqrtf(ax * ax + ay * ay + az * az);
+    const float lb = sqrtf(bx * bx + by * by + bz * bz);
+    const float lc = sqrtf(cx * cx + cy * cy + cz * cz);
+    const float det = ax * (by * cz - bz * cy) + ay * (bz * cx - bx * cz) + az * (bx * cy - by * cx);
+    const float den = la * lb * lc + (ax * bx + ay * by + az * bz) * lc + (bx * cx + by * cy + bz * cz) * la +
+                      (cx * ax + cy * ay + cz * az) * lb;
+    return atan2f(det, den);
+}
+
+// The same, the short way where the triangle is far; (v0.w, v1.w, v2.w) is its
+// normal.  The x terms come last in every sum, so points that share py and pz
+// share the rest.
 __device__ __forceinline__ float half_solid_angle(float px, float py, float pz, float4 v0, float4 v1, float4 v2) {
     const float ax = v0.x - px, ay = v0.y - py, az = v0.z - pz;
     const float bx = v1.x - px, by = v1.y - py, bz = v1.z - pz;
     const float cx = v2.x - px, cy = v2.y - py, cz = v2.z - pz;
-    const float la = __builtin_amdgcn_sqrtf(__fmaf_rn(ax, ax, ay * ay + az * az));
-    const float lb = __builtin_amdgcn_sqrtf(__fmaf_rn(bx, bx, by * by + bz * bz));
-    const float lc = __builtin_amdgcn_sqrtf(__fmaf_rn(cx, cx, cy * cy + cz * cz));
+    const float a2 = __fmaf_rn(ax, ax, ay * ay + az * az), b2 = __fmaf_rn(bx, bx, by * by + bz * bz);
+    const float c2 = __fmaf_rn(cx, cx, cy * cy + cz * cz);
     const float ab = __fmaf_rn(ax, bx, ay * by + az * bz), bc = __fmaf_rn(bx, cx, by * cy + bz * cz);
     const float ca = __fmaf_rn(cx, ax, cy * ay + cz * az);
-    const float den = __fmaf_rn(ca, lb, __fmaf_rn(bc, la, __fmaf_rn(la, lb, ab) * lc));
+    auto denominator = [&](float la, float lb, float lc) {
+        return __fmaf_rn(ca, lb, __fmaf_rn(bc, la, __fmaf_rn(la, lb, ab) * lc));
+    };
+    const float den = denominator(__builtin_amdgcn_sqrtf(a2), __builtin_amdgcn_sqrtf(b2), __builtin_amdgcn_sqrtf(c2));
     const float num = __fmaf_rn(ax, v0.w, ay * v1.w + az * v2.w);
-    // den in [1e-30, 1e30): positive, no NaN, and with a reciprocal in range
-    const uint32_t lo = __float_as_uint(1e-30f), hi = __float_as_uint(1e30f);
-    if (__float_as_uint(den) - lo < hi - lo && fabsf(num) < 0.125f * den) {
+    // A denominator of positive terms, so that a root's ulp is no more of it;
+    // above 1e-30 with each product above 1e-20, and with a reciprocal in range
+    // (a NaN fails the tests).
+    if (fminf(fminf(ab, bc), ca) > 1e-20f && fabsf(num) < 0.125f * den && den < 1e30f) {
         const float t = num * __builtin_amdgcn_rcpf(den), t2 = t * t;
         return t + t * t2 * (t2 * (0.2f - t2 * (1.0f / 7.0f)) - (1.0f / 3.0f));
     }
     const float det = ax * (by * cz - bz * cy) + ay * (bz * cx - bx * cz) + az * (bx * cy - by * cx);
-    return atan2f(det, den);
+    return atan2f(det, denominator(sqrtf(a2), sqrtf(b2), sqrtf(c2)));
 }
 
-__global__ void __launch_bounds__(64 * kMeshWaves)
+template <int WAVES, bool SHORT>
+__global__ void __launch_bounds__(64 * WAVES)
     k_mesh_winding(const fg_float3* __restrict__ verts, uint32_t nverts, const uint32_t* __restrict__ tris,
                    uint32_t ntris, fg_float3 origin, float spacing, uint32_t nx, uint32_t ny, uint32_t nz,
                    float* __restrict__ out) {
-    constexpr int kTile = 64 * kMeshWaves;
+    constexpr int kTile = 64 * WAVES;
     __shared__ union {
         float4 tile[3][kTile];
-        double sum[kMeshWaves][64 * kMeshPts];
+        double sum[WAVES][64 * kMeshPts];
     } s;
-    __shared__ uint32_t s_count[kMeshWaves];
+    __shared__ uint32_t s_count[WAVES];
     const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     // the lane's points: kMeshPts neighbours in x, of one row of the lattice
     const uint32_t row_groups = nx / kMeshPts + (nx % kMeshPts != 0);
@@ -118,7 +150,7 @@ __global__ void __launch_bounds__(64 * kMeshWaves)
         if (lane == 0) s_count[wave] = (uint32_t)__popcll(lanes);
         __syncthreads();
         uint32_t at = (uint32_t)__popcll(lanes & ((1ull << lane) - 1ull)), cnt = 0;
-        for (uint32_t w = 0; w < (uint32_t)kMeshWaves; w++) {
+        for (uint32_t w = 0; w < (uint32_t)WAVES; w++) {
             if (w == wave) at += cnt;
             cnt += s_count[w];
         }
@@ -131,10 +163,12 @@ __global__ void __launch_bounds__(64 * kMeshWaves)
             s.tile[2][at] = make_float4(c.x, c.y, c.z, (float)(ux * wy - uy * wx));
         }
         __syncthreads();
-        for (uint32_t j = wave; j < cnt; j += kMeshWaves) {
+        for (uint32_t j = wave; j < cnt; j += WAVES) {
             const float4 v0 = s.tile[0][j], v1 = s.tile[1][j], v2 = s.tile[2][j];
 #pragma unroll
-            for (int k = 0; k < kMeshPts; k++) acc[k] += (double)half_solid_angle(px[k], p0.y, p0.z, v0, v1, v2);
+            for (int k = 0; k < kMeshPts; k++)
+                acc[k] += (double)(SHORT ? half_solid_angle(px[k], p0.y, p0.z, v0, v1, v2)
+                                         : half_solid_angle_near(px[k], p0.y, p0.z, v0, v1, v2));
         }
     }
     // w = sum(2 atan2) / (4 pi)
@@ -145,7 +179,7 @@ __global__ void __launch_bounds__(64 * kMeshWaves)
     __syncthreads();
     if (wave >= (uint32_t)kMeshPts || row >= (uint64_t)ny * nz || ix + wave >= nx) return;
     double a = 0.0;  // wavefront k adds the sums of every lane's point k
-    for (uint32_t w = 0; w < (uint32_t)kMeshWaves; w++) a += s.sum[w][threadIdx.x];
+    for (uint32_t w = 0; w < (uint32_t)WAVES; w++) a += s.sum[w][threadIdx.x];
     out[row * nx + ix + wave] = (float)(a * kInv2Pi);
 }
 
@@ -171,8 +205,10 @@ int fg_mesh_winding_lattice(const fg_float3* vertices, unsigned int numVertices,
     const State& st = state();
     const uint64_t groups = (uint64_t)(nx / kMeshPts + (nx % kMeshPts != 0)) * ny * nz;
     const uint64_t blocks = (groups + 63) / 64, x = blocks < kMeshMaxX ? blocks : kMeshMaxX;
-    hipLaunchKernelGGL(k_mesh_winding, dim3((unsigned)x, (unsigned)((blocks + x - 1) / x)), dim3(64 * kMeshWaves), 0,
-                       st.stream, vertices, numVertices, triangles, numTriangles, origin, spacing, nx, ny, nz, winding);
+    const bool near = numTriangles <= kMeshNearTris;
+    hipLaunchKernelGGL((near ? k_mesh_winding<kMeshNearWaves, false> : k_mesh_winding<kMeshWaves, true>),
+                       dim3((unsigned)x, (unsigned)((blocks + x - 1) / x)), dim3(64 * (near ? kMeshNearWaves : kMeshWaves)),
+                       0, st.stream, vertices, numVertices, triangles, numTriangles, origin, spacing, nx, ny, nz, winding);
     return check_launch("fg_mesh_winding_lattice") ? FG_OK : fg_peek_error();
 }
 
