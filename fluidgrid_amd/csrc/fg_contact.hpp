@@ -216,7 +216,8 @@ __device__ __forceinline__ F3 contact_stencil_lanes(const float4& sp, const floa
     const float mind = sr + cr + eps;
     const float cut2 = rn_mul(rn_mul(mind, mind), 0x1.00001p+0f);
     const CellXYZ c = g.mode == FG_KEY_LINEAR ? grid_cell(sp.x, sp.y, sp.z, g) : CellXYZ{0, 0, 0};
-    const int nx = 2 * rel.x + 1, ny = 2 * rel.y + 1, cells = nx * ny * (2 * rel.z + 1);
+    // (an axis of negative width leaves no cell)
+    const int nx = 2 * rel.x + 1, ny = 2 * rel.y + 1, cells = (rel.x | rel.y | rel.z) < 0 ? 0 : nx * ny * (2 * rel.z + 1);
     const bool unit = rel.x == 1 && rel.y == 1 && rel.z == 1;
     const bool xor_unit = unit && g.mode == FG_KEY_REF_XOR;
     const float csx = g.cs.x, csy = g.cs.y, csz = g.cs.z;
