@@ -81,11 +81,11 @@ std::vector<BatchSceneView> views_of(const std::vector<BatchScene>& scenes) {
 
 // Uploads one array of every scene behind each other, scenes that also lie
 // behind each other in host memory with one copy.
-void upload_scenes(float4* dst, const std::vector<BatchSceneView>& scenes, const float4* BatchSceneView::*from) {
-    for (size_t s = 0; s < scenes.size();) {
+void upload_scenes(float4* dst, const BatchSceneView* scenes, size_t nscenes, const float4* BatchSceneView::*from) {
+    for (size_t s = 0; s < nscenes;) {
         const float4* const src = scenes[s].*from;
         size_t count = scenes[s].count, e = s + 1;
-        while (e < scenes.size() && scenes[e].*from == src + count) count += scenes[e++].count;
+        while (e < nscenes && scenes[e].*from == src + count) count += scenes[e++].count;
         if (count) hip_check(hipMemcpy(dst, src, sizeof(float4) * count, hipMemcpyHostToDevice), "upload");
         dst += count;
         s = e;
@@ -99,10 +99,10 @@ BatchedSimulator::BatchedSimulator(const std::vector<BatchScene>& scenes) : Batc
 // scene of each particle is written there: host copies of them (two of 95 MB,
 // one grown scene by scene) and of the scene indices were 44 of 59 ms for
 // 128 scenes of 2,957,000 particles in all.
-BatchedSimulator::BatchedSimulator(const std::vector<BatchSceneView>& scenes) {
-    if (scenes.empty()) throw std::invalid_argument("BatchedSimulator: no scenes");
+BatchedSimulator::BatchedSimulator(const BatchSceneView* scenes, size_t count) {
+    if (count == 0) throw std::invalid_argument("BatchedSimulator: no scenes");
     uint64_t n = 0, nb = 0;
-    for (size_t s = 0; s < scenes.size(); s++) {
+    for (size_t s = 0; s < count; s++) {
         const BatchSceneView& sc = scenes[s];
         const auto& cp = sc.common;
         if (cp.bucket_size.x <= 0 || cp.bucket_size.y <= 0 || cp.bucket_size.z <= 0)
@@ -154,8 +154,8 @@ BatchedSimulator::BatchedSimulator(const std::vector<BatchSceneView>& scenes) {
 
     hip_check(hipMemcpy(d_descs, mDescs.data(), sizeof(fg_scene_desc) * mDescs.size(), hipMemcpyHostToDevice),
               "upload");
-    upload_scenes(d_pos, scenes, &BatchSceneView::positions);
-    upload_scenes(d_vel, scenes, &BatchSceneView::velocities);
+    upload_scenes(d_pos, scenes, count, &BatchSceneView::positions);
+    upload_scenes(d_vel, scenes, count, &BatchSceneView::velocities);
     hip_check(hipMemset(d_rho, 0, sizeof(float2) * mN), "memset");
     hip_check(hipMemset(d_end, 0, sizeof(unsigned) * mBuckets), "memset");
     d_queue = dalloc<unsigned>(fg::kQueueSlots * fg::kQueueStride);

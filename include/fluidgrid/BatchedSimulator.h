@@ -10,7 +10,9 @@
 // no host synchronisation and is replayed as a captured HIP graph.
 #pragma once
 
+#include <cstddef>
 #include <stdexcept>
+#include <type_traits>
 #include <vector>
 
 #include "ApplicationData.h"
@@ -69,7 +71,9 @@ struct BatchTuning {
 class BatchedSimulator {
 public:
     explicit BatchedSimulator(const std::vector<BatchScene>& scenes);
-    explicit BatchedSimulator(const std::vector<BatchSceneView>& scenes);
+    // (a template, so that a list in braces is one of BatchScene)
+    template <class Views, class = std::enable_if_t<std::is_same<Views, std::vector<BatchSceneView>>::value>>
+    explicit BatchedSimulator(const Views& scenes) : BatchedSimulator(scenes.data(), scenes.size()) {}
     ~BatchedSimulator();
     BatchedSimulator(const BatchedSimulator&) = delete;
     BatchedSimulator& operator=(const BatchedSimulator&) = delete;
@@ -117,6 +121,7 @@ public:
     hipStream_t stream() const { return mStream; }
 
 private:
+    BatchedSimulator(const BatchSceneView* scenes, size_t count);
     void enqueueStep();
     void enqueueStepOverlapped();
     void enqueueCoupledForces();
