@@ -174,7 +174,7 @@ BatchedSimulator::BatchedSimulator(const BatchSceneView* scenes, size_t count) {
     mTuning.sortDigitBits = bits;
     mTuning.flatDensity = fd != 0;
     mTuning.flatForces = ff != 0;
-    mSceneBodies.resize(scenes.size());
+    mSceneBodies.resize(count);
 }
 
 BatchedSimulator::~BatchedSimulator() {
