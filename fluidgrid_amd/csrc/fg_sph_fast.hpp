@@ -257,19 +257,31 @@ __host__ __device__ __forceinline__ size_t nbr_list_offset(uint32_t n) {
 //   runs[18 w + row]     first sorted index of wavefront w's run in the row
 //   runs[18 w + 9 + row] its length (kRunLength; 0 when no lane has the row),
 //                        with kRunWide when a lane has more than 32
-//                        candidates, and kRunGeneric when the force pass
-//                        cannot use it: a lane has more than 64 candidates,
-//                        or the density pass found no runs
+//                        candidates, kRunLong when one has more than 64,
+//                        which its mask does not hold, and kRunFar, and no
+//                        length, when the run is too long (kRunMax,
+//                        kRunSparse): its lanes read their rows from memory
 //   offs[64 (9 w + row) + lane]  the lane's first candidate, from the run's first
-// A force pass that has them looks up no cells.  Both passes agree on the
+// A force pass that has them looks up cells for such rows only.  Both passes agree on the
 // wavefronts: sorted particles 64 w .. 64 w + 63, all present (the last one
 // padded by inactive lanes in a single fluid).  About 19 bytes per particle,
 // which the list area holds from 64 particles on.
 constexpr uint32_t kRunWords = 18;
 constexpr uint32_t kRunLength = 0xFFFFu;
 constexpr uint32_t kRunMax = 2047u;  // longest run
+// A run above kRunSparse that is also longer than kRunSpread times what any lane
+// may read of it is not staged: a wavefront of a few particles far apart, beside
+// or above a pool, would stage thousands of records for a few neighbours a lane,
+// and the kernel wait for it (32 splashing dam breaks, 729,000 particles:
+// density 86 us, forces 85 us with every run up to kRunMax staged, 76 and 67 so).
+// Where cells are full, long runs are read by most lanes and worth staging, and
+// up to 640 the row costs less staged than looked up again (with 160, forces of
+// 500,000 particles 50 against 47 us, a tenth of them spray).
+constexpr uint32_t kRunSparse = 640u, kRunSpread = 4u;
 constexpr uint32_t kRunWide = 0x10000u;
-constexpr uint32_t kRunGeneric = 0x20000u;
+constexpr uint32_t kRunLong = 0x20000u;
+constexpr uint32_t kRunFar = 0x40000u;
+constexpr uint32_t kRunLookup = 0x80000u;  // (not stored) lanes look their range up: WaveCells does not hold it
 constexpr uint32_t kRunMinParticles = 64;
 __host__ __device__ __forceinline__ size_t nbr_runs_offset(uint32_t n) {
     return nbr_align256(nbr_list_offset(n) + 20 * (size_t)n);
@@ -324,6 +336,7 @@ struct WaveCells {
     uint32_t row[9][64];
     uint32_t key[64], sides[64];  // a cell's key, and kSide* of the grid around it
     uint32_t lo[9], hi[9];        // the rows' runs
+    uint32_t most[9];             // most particles in three cells
 };
 constexpr uint32_t kWaveCellsTemp = 9 * 64;  // words that wave_cells needs besides
 constexpr uint32_t kSideLowY = 1u, kSideHighY = 2u, kSideLowZ = 4u, kSideHighZ = 8u, kSideLeft = 16u,
@@ -357,16 +370,20 @@ struct WaveRuns {
 
 // Fills wc for the wavefront (every lane calls it) and gives each lane the
 // index of its cell there, and the wavefront its runs: row r's run goes from
-// the smallest B0 to the largest end of the row's entries.  False, and
-// nothing of use, when a run is longer than kRunMax or three cells hold more
-// than 127 particles; the caller then reads the rows from memory.
+// the smallest B0 to the largest end of the row's entries.  A row in which
+// three cells hold more than 127 particles has kRunLookup set, its lanes look
+// their ranges up (other_row); one whose run is too long has kRunFar set and no
+// length, and is read from memory.  (1,048,576 particles on cells of 2 h, where
+// one such cell used to send all nine rows of its wavefront to memory: density
+// 580 us so and 330 now, forces 1,190 and 670; on cells of 1.3 h, where some
+// rows are longer than a mask, forces 271 and 157.)
 // `temp`: nine times 64 words of LDS, `stride` words apart, free again afterwards.
 //
 // The nine rows of the cells are looked up by (cell, row) pairs, a pair a
 // lane and two a round: one round of twelve loads for the 64 particles in the
 // bulk of a fluid, where every lane looking up its own nine rows takes 54
 // loads of addresses that mostly coincide.
-__device__ __forceinline__ bool wave_cells(WaveCells& wc, uint32_t* __restrict__ temp, uint32_t stride, const RowWalker& w,
+__device__ __forceinline__ void wave_cells(WaveCells& wc, uint32_t* __restrict__ temp, uint32_t stride, const RowWalker& w,
                                            const fg_common_fluid_params& cp, uint32_t key_base,
                                            const uint32_t* __restrict__ start, const uint32_t* __restrict__ end,
                                            uint32_t n, uint32_t& cell, WaveRuns& runs) {
@@ -386,11 +403,10 @@ __device__ __forceinline__ bool wave_cells(WaveCells& wc, uint32_t* __restrict__
     }
     if (lane < 9u) {
         wc.lo[lane] = kEmpty;
-        wc.hi[lane] = 0u;
+        wc.hi[lane] = wc.most[lane] = 0u;
     }
     wave_lds_sync();
     const uint32_t by = (uint32_t)cp.bucket_size.x, bz = by * (uint32_t)cp.bucket_size.y;
-    bool bad = false;
     for (uint32_t q0 = lane; q0 < pairs; q0 += 128u) {
         uint32_t s[2][3], e[2][3];
         bool valid[2];
@@ -426,7 +442,7 @@ __device__ __forceinline__ bool wave_cells(WaveCells& wc, uint32_t* __restrict__
             uint32_t d = 0u;
             if (valid[u] && b0 < b3) {
                 const uint32_t d1 = s[u][0] != kEmpty ? e0 - b0 : 0u, d2 = s[u][2] != kEmpty ? s[u][2] - b0 : b3 - b0;
-                bad |= b3 - b0 > 127u;
+                atomicMax(&wc.most[row], b3 - b0);
                 d = ((d1 & 127u) << 11) | ((d2 & 127u) << 18) | ((b3 - b0) << 25);
                 atomicMin(&wc.lo[row], b0);
                 atomicMax(&wc.hi[row], b3);
@@ -440,14 +456,13 @@ __device__ __forceinline__ bool wave_cells(WaveCells& wc, uint32_t* __restrict__
         const uint32_t c = q / 9u, row = q - 9u * c, d = temp[stride * row + c];
         wc.row[row][c] = d ? ((wc.row[row][c] - wc.lo[row]) & kRunMax) | d : 0u;
     }
-    uint32_t len = 0u;
     if (lane < 9u && wc.hi[lane] != 0u) {
         runs.lo = wc.lo[lane];
-        len = wc.hi[lane] - runs.lo;
+        const uint32_t len = wc.hi[lane] - runs.lo, most = wc.most[lane];
+        runs.info = len > kRunMax || (len > kRunSparse && len > kRunSpread * most) ? kRunFar
+                                                                           : len | (most > 127u ? kRunLookup : 0u);
     }
-    runs.info = len;
     wave_lds_sync();
-    return __ballot(bad || len > kRunMax) == 0ull;
 }
 
 // A lane's range in a row, from its run's first index: the row's cells after
@@ -467,11 +482,24 @@ __device__ __forceinline__ LaneRow lane_row(const WaveCells& wc, int row, uint32
     return LaneRow{(c & kRunMax) + first, active && gyz < cut && last > first ? last - first : 0u};
 }
 
-// A run's length word, from its length and the lanes' candidates in it.
-__device__ __forceinline__ uint32_t run_word(uint32_t run, uint32_t len) {
-    if (__ballot(len > 32u) != 0ull) run |= kRunWide;
-    if (__ballot(len > kRowMaskBits) != 0ull) run |= kRunGeneric;
-    return run;
+// lane_row of a row that WaveCells does not hold: the range from the cell
+// tables (off is of use within kRunMax only).
+__device__ __forceinline__ LaneRow other_row(int row, bool active, const float4& p, uint32_t lo, float cut,
+                                             const fg_common_fluid_params& cp, uint32_t key_base,
+                                             const uint32_t* __restrict__ start, const uint32_t* __restrict__ end,
+                                             uint32_t n) {
+    uint32_t rb = lo, re = lo;
+    const bool has = active && row_range(make_rows(p, cp), row % 3 - 1, row / 3 - 1, cut, cp, key_base, start, end, n,
+                                         rb, re);
+    return LaneRow{rb - lo, has ? re - rb : 0u};
+}
+
+// A run's length word, from its word of wave_cells and the lanes' candidates in it.
+__device__ __forceinline__ uint32_t run_word(uint32_t word, uint32_t len) {
+    word &= kRunLength | kRunFar;
+    if (__ballot(len > 32u) != 0ull) word |= kRunWide;
+    if (__ballot(len > kRowMaskBits) != 0ull) word |= kRunLong;
+    return word;
 }
 
 // Wavefront w's runs and its lanes' offsets (off(row)), for the force pass.
@@ -672,21 +700,19 @@ __device__ __forceinline__ void density_row_staged(const float4& p, const Densit
 // with no rows and writes no masks): each row's run staged in the wavefront's
 // LDS slice, the next row's positions loaded into registers while this row
 // is walked.  Same candidates, same order, same sums and masks as the row
-// loop of density_particle.  False when the wavefront has no usable runs
-// (wave_cells): nothing is summed then.
+// loop of density_particle.
 //
 // Bound by VALU issue: about 4,700 instructions a wavefront, 3,800 of them in
 // the walks (65 groups of four candidates, which its longest lane per row
 // sets); 8,388,608 particles take 702 us against 767 with per-lane lookups
 // row by row and whole positions in LDS, 1,048,576 take 104 against 111.
 template <bool MASKS>
-__device__ __forceinline__ bool density_rows_staged(uint32_t i, bool active, const float4& p,
+__device__ __forceinline__ float density_rows_staged(uint32_t i, bool active, const float4& p,
                                                     const float4* __restrict__ sp,
                                                     const uint32_t* __restrict__ start,
                                                     const uint32_t* __restrict__ end, uint32_t n,
                                                     const fg_common_fluid_params& cp, uint32_t key_base,
-                                                    unsigned long long* __restrict__ masks, DensityStage& st,
-                                                    float& sum) {
+                                                    unsigned long long* __restrict__ masks, DensityStage& st) {
     const float s = cp.simulation_scale, s2 = s * s;
     const float h = cp.kernel_radius, hh = h * h;
     const float hu = h / s, hhu = hu * hu, h2u = cp.kernel_radius_squared / s2;
@@ -697,11 +723,7 @@ __device__ __forceinline__ bool density_rows_staged(uint32_t i, bool active, con
     const RowWalker w = make_rows(p, cp);
     uint32_t cell;
     WaveRuns runs;
-    if (!wave_cells(st.cells, st.temp(), 64u, w, cp, key_base, start, end, n, cell, runs)) {
-        runs.info = kRunGeneric;
-        if (table) store_runs(runs, wave, masks, n);
-        return false;
-    }
+    wave_cells(st.cells, st.temp(), 64u, w, cp, key_base, start, end, n, cell, runs);
     const bool same = __builtin_amdgcn_readfirstlane(__float_as_uint(h2u) == __float_as_uint(hhu) ? 1u : 0u) != 0u;
     const float4 own = own_finite(p);
     uint16_t* offs = MASKS ? nbr_offs(masks, n) + (size_t)9 * 64 * wave + lane : nullptr;
@@ -710,7 +732,7 @@ __device__ __forceinline__ bool density_rows_staged(uint32_t i, bool active, con
     float acc = 0.0f;
     float3 n0 = make_float3(0.0f, 0.0f, 0.0f), n1 = n0;
     auto fetch = [&](int row) {
-        const uint32_t len = runs.word(row);
+        const uint32_t len = runs.word(row) & kRunLength;
         const float4* q = sp + runs.first(row) + lane;
         if (lane < len) n0 = ld_xyz(q);
         if (lane + 64u < len) n1 = ld_xyz(q + 64);
@@ -721,13 +743,19 @@ __device__ __forceinline__ bool density_rows_staged(uint32_t i, bool active, con
     };
     fetch(0);
     for (int row = 0; row < 9; row++) {
-        const uint32_t len = runs.word(row), lo = runs.first(row);  // the same on every lane
-        const LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
+        const uint32_t info = runs.word(row), len = info & kRunLength, lo = runs.first(row);  // the same on every lane
+        LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
+        if (info & (kRunLookup | kRunFar)) r = other_row(row, active, p, lo, cut, cp, key_base, start, end, n);
         if (table) {
-            const uint32_t word = run_word(len, r.len);
+            const uint32_t word = run_word(info, r.len);
             words = (int)lane == row ? word : words;
         }
         msk = 0ull;
+        const bool whole = r.len <= kRowMaskBits;
+        if (info & kRunFar) {
+            if (r.len) msk = density_row<MASKS>(p, sp + lo + r.off, r.len, h2u, hhu, acc);
+            r.len = 0u;
+        }
         // the lane's candidates among the staged positions [at, at + kStagePos) of the run
         auto walk = [&](uint32_t at) {
             const uint32_t a = max(r.off, at), b = min(r.off + r.len, at + kStagePos);
@@ -756,15 +784,14 @@ __device__ __forceinline__ bool density_rows_staged(uint32_t i, bool active, con
             at += kStagePos;
             if (at >= len) break;
         }
-        last = r.len <= kRowMaskBits ? msk : 0ull;
+        last = whole ? msk : 0ull;
     }
     if (MASKS && active) masks[(size_t)8 * n + i] = last;
     if (table) {
         runs.info = words;
         store_runs(runs, wave, masks, n);
     }
-    sum = acc;
-    return true;
+    return acc;
 }
 
 // Per-lane row table of the flat density schedule, in LDS: first and
@@ -804,9 +831,9 @@ __device__ __forceinline__ void density_particle(uint32_t i, const float4* __res
     // The staged row loop needs every lane of the wavefront (a row's run is
     // its lanes' together); otherwise the rows are read from memory.
     const bool whole = __ballot(1) == ~0ull;
-    float sum = 0.0f;
-    if (stage != nullptr && flat == nullptr && whole &&
-        density_rows_staged<MASKS>(i, valid && p.w > 0.0f, p, sp, start, end, n, cp, key_base, masks, *stage, sum)) {
+    if (stage != nullptr && flat == nullptr && whole) {
+        const float sum =
+            density_rows_staged<MASKS>(i, valid && p.w > 0.0f, p, sp, start, end, n, cp, key_base, masks, *stage);
         if (!valid) return;
         const float4 v = MASKS ? sv[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (p.w > 0.0f) {
@@ -822,16 +849,19 @@ __device__ __forceinline__ void density_particle(uint32_t i, const float4* __res
         const RowWalker w = make_rows(p, cp);
         const float cut = cp.kernel_radius * cp.kernel_radius * 1.0001f;
         const uint32_t wave = __builtin_amdgcn_readfirstlane(i >> 6);
-        uint32_t cell, words = kRunGeneric;
+        uint32_t cell, words = 0u;
         WaveRuns runs;
-        if (wave_cells(*flat->cells, flat->rb + (flat->lane & ~63u), flat->lanes, w, cp, key_base, start, end, n, cell, runs)) {
-            uint16_t* offs = nbr_offs(masks, n) + (size_t)9 * 64 * wave + __lane_id();
-            for (int row = 0; row < 9; row++) {
-                const LaneRow r = lane_row(*flat->cells, row, cell, valid && p.w > 0.0f, w, cut);
-                offs[64 * row] = (uint16_t)r.off;
-                const uint32_t word = run_word(runs.word(row), r.len);
-                words = (int)__lane_id() == row ? word : words;
-            }
+        wave_cells(*flat->cells, flat->rb + (flat->lane & ~63u), flat->lanes, w, cp, key_base, start, end, n, cell, runs);
+        uint16_t* offs = nbr_offs(masks, n) + (size_t)9 * 64 * wave + __lane_id();
+        for (int row = 0; row < 9; row++) {
+            const bool active = valid && p.w > 0.0f;
+            const uint32_t info = runs.word(row);
+            LaneRow r = lane_row(*flat->cells, row, cell, active, w, cut);
+            if (info & (kRunLookup | kRunFar))
+                r = other_row(row, active, p, runs.first(row), cut, cp, key_base, start, end, n);
+            offs[64 * row] = (uint16_t)r.off;
+            const uint32_t word = run_word(info, r.len);
+            words = (int)__lane_id() == row ? word : words;
         }
         runs.info = words;
         store_runs(runs, wave, masks, n);
@@ -1008,6 +1038,23 @@ __device__ __forceinline__ void walk_staged_word(PairAcc& A, uint32_t word, uint
     }
 }
 
+// The pairs of one row of forces_rowloop.
+template <bool MASKS>
+__device__ __forceinline__ void forces_row(PairAcc& A, uint32_t i, const float4& pos, const float4& vel, float pri,
+                                           uint32_t rb, uint32_t re, unsigned long long mrow,
+                                           const float4* __restrict__ rec, const float4* __restrict__ sp,
+                                           const float4* __restrict__ sv, const float2* __restrict__ rho_p, float h,
+                                           float s, float hhu) {
+    if (MASKS && re - rb <= kRowMaskBits) {
+        // the particle itself is in its own row's mask; it adds nothing
+        if (i >= rb && i < re) mrow &= ~(1ull << (i - rb));
+        walk_row_mask(A, mrow, rb, rec, pos, vel, pri, h, s);
+    } else {
+        for (uint32_t j = rb; j < re; j++)
+            pair_term_rp(A, i, j, pos, vel, pri, ld_xyz(sp + j), ld_xyz(sv + j), rho_p[j], h, s, hhu);
+    }
+}
+
 // The row loop of the force pass: the 9 stencil rows in turn, each row's
 // neighbours from its mask (ascending, two per iteration) or, without a mask
 // or for a row longer than 64 candidates, by re-testing every candidate.
@@ -1036,15 +1083,7 @@ __device__ __forceinline__ void forces_rowloop(PairAcc& A, uint32_t i, const flo
         }
         uint32_t rb, re;
         if (!row_range(w, dy, dz, cut, cp, key_base, start, end, n, rb, re)) continue;
-        if (MASKS && re - rb <= kRowMaskBits) {
-            unsigned long long mm = mrow;
-            // the particle itself is in its own row's mask; it adds nothing
-            if (i >= rb && i < re) mm &= ~(1ull << (i - rb));
-            walk_row_mask(A, mm, rb, rec, pos, vel, dpi.y, h, s);
-        } else {
-            for (uint32_t j = rb; j < re; j++)
-                pair_term_rp(A, i, j, pos, vel, dpi.y, ld_xyz(sp + j), ld_xyz(sv + j), rho_p[j], h, s, hhu);
-        }
+        forces_row<MASKS>(A, i, pos, vel, dpi.y, rb, re, mrow, rec, sp, sv, rho_p, h, s, hhu);
     }
 }
 
@@ -1053,31 +1092,34 @@ __device__ __forceinline__ void forces_rowloop(PairAcc& A, uint32_t i, const flo
 // from the runs the density pass left: each row's neighbour records staged
 // in the wavefront's LDS slice `stage` (kStageRecs first halves, then their
 // second halves), the next row's records, masks and offsets loaded into
-// registers while this row is walked.  No cell is looked up.  Same pairs,
-// same order, same sums as forces_rowloop<true>.  False when a row of the
-// wavefront has no usable run: nothing is summed then.
+// registers while this row is walked.  Cells are looked up only for a row in
+// which a lane has more candidates than its mask holds (it tests them where
+// they are staged) and for one without a run.  Same pairs, same order, same
+// sums as forces_rowloop<true>.
 //
 // Bound by VALU issue (3,300 instructions a wavefront) and by the records,
 // which come from past the L2 cache about three times at 8,388,608 particles:
 // 579 us there against 701 with the cells looked up again and a min/max
 // reduction per row; 84 against 98 us at 1,048,576.
-__device__ __forceinline__ bool forces_rows_staged(PairAcc& A, uint32_t i, bool active, const float4& pos,
-                                                   const float4& vel, float pri, uint32_t n,
-                                                   const fg_common_fluid_params& cp,
+//
+// OTHER: with rows that lanes look up (kRunLong, kRunFar), a loop of its own,
+// without loads ahead, so that the usual one keeps its registers (in one loop
+// 1,048,576 particles took 178 us against 80).
+template <bool OTHER>
+__device__ __forceinline__ void forces_rows_staged(const WaveRuns& runs, PairAcc& A, uint32_t i, bool active, const float4& pos,
+                                                   const float4& vel, float pri, const float4* __restrict__ sp,
+                                                   const float4* __restrict__ sv, const float2* __restrict__ rho_p,
+                                                   const uint32_t* __restrict__ start,
+                                                   const uint32_t* __restrict__ end, uint32_t n,
+                                                   const fg_common_fluid_params& cp, uint32_t key_base,
                                                    const unsigned long long* __restrict__ masks,
                                                    float4* __restrict__ stage) {
     const float h = cp.kernel_radius, s = cp.simulation_scale;
+    const float hu = h / s, hhu = hu * hu;
     const uint32_t lane = __lane_id();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(i >> 6);
     const float4* rec = nbr_records(masks, n);
     const uint16_t* offs = nbr_offs(masks, n) + (size_t)9 * 64 * wave + lane;
-    WaveRuns runs;
-    if (lane < 9u) {
-        const uint32_t* t = nbr_runs(masks, n) + (size_t)kRunWords * wave + lane;
-        runs.lo = t[0];
-        runs.info = t[9];
-    }
-    if (__ballot((runs.info & kRunGeneric) != 0u) != 0ull) return false;
     float4 a0, b0, a1, b1;
     a0 = b0 = a1 = b1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     unsigned long long next_mask = 0ull;
@@ -1096,36 +1138,67 @@ __device__ __forceinline__ bool forces_rows_staged(PairAcc& A, uint32_t i, bool 
             b1 = q[129];
         }
     };
-    fetch(0);
+    if (!OTHER) fetch(0);
     for (int row = 0; row < 9; row++) {
         const uint32_t word = runs.word(row), len = word & kRunLength, lo = runs.first(row);  // the same on every lane
-        unsigned long long mm = next_mask;
-        const uint32_t off = next_off;
-        if (lane < len) {
+        LaneRow r{0u, 0u};
+        if (OTHER && (word & (kRunLong | kRunFar)))
+            r = other_row(row, active, pos, lo, h * h * 1.0001f, cp, key_base, start, end, n);
+        unsigned long long mm = OTHER ? (active ? masks[(size_t)row * n + i] : 0ull) : next_mask;
+        const uint32_t off = OTHER ? offs[64 * row] : next_off;
+        if (!OTHER && lane < len) {
             stage[lane] = a0;
             stage[kStageRecs + lane] = b0;
         }
-        if (lane + 64u < len) {
+        if (!OTHER && lane + 64u < len) {
             stage[lane + 64u] = a1;
             stage[kStageRecs + lane + 64u] = b1;
         }
-        if (lane + 128u < min(len, kStageRecs)) {
+        if (!OTHER && lane + 128u < min(len, kStageRecs)) {
             const float4* q = rec + 2 * ((size_t)lo + lane + 128u);
             stage[lane + 128u] = q[0];
             stage[kStageRecs + lane + 128u] = q[1];
         }
-        if (row < 8) fetch(row + 1);
+        for (uint32_t k = lane; OTHER && k < min(len, kStageRecs); k += 64u) {
+            const float4* q = rec + 2 * ((size_t)lo + k);
+            stage[k] = q[0];
+            stage[kStageRecs + k] = q[1];
+        }
+        if (!OTHER && row < 8) fetch(row + 1);
+        LaneRow test{0u, 0u};  // the lane's candidates where its mask does not hold them
+        if (OTHER && (word & (kRunLong | kRunFar))) {
+            if (word & kRunFar) {  // from memory, one by one: two at a time need more registers than the loop has
+                const uint32_t rb = lo + r.off;
+                if (r.len > kRowMaskBits) mm = 0ull;
+                for (uint32_t k = 0u; k < r.len; k++) {
+                    if (r.len <= kRowMaskBits) {
+                        if (mm == 0ull) break;
+                        k = (uint32_t)__builtin_ctzll(mm);
+                        mm &= mm - 1ull;
+                    }
+                    const float4 a = rec[2 * (size_t)(rb + k)], b = rec[2 * (size_t)(rb + k) + 1];
+                    pair_term(A, i, rb + k, pos, vel, pri, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w,
+                              b.w, h, s, hhu);
+                }
+                continue;
+            }
+            if (r.len > kRowMaskBits) {
+                test = r;
+                mm = 0ull;
+            }
+        }
         // the particle itself is in its own cell's row; it adds nothing
         if (row == 4) mm &= ~(1ull << ((i - lo - off) & 63u));
         wave_lds_sync();
-        if (len <= kStageRecs) {
+        if (len <= kStageRecs && !(OTHER && (word & kRunLong))) {
             walk_staged_word(A, (uint32_t)mm, off, stage, pos, vel, pri, h, s);
             if (word & kRunWide) walk_staged_word(A, (uint32_t)(mm >> 32), off + 32u, stage, pos, vel, pri, h, s);
             wave_lds_sync();  // every lane's reads before the next stores
             continue;
         }
-        // a run that fills the slice more than once: the mask is walked as far
-        // as the records [at, at + kStageRecs) of the run go, then on from there
+        // A run that fills the slice more than once: the mask is walked as far
+        // as the records [at, at + kStageRecs) of the run go, then on from there,
+        // and so are the candidates to test.
         for (uint32_t at = 0u;;) {
             while (mm) {
                 const uint32_t j = off + (uint32_t)__builtin_ctzll(mm) - at;
@@ -1134,6 +1207,12 @@ __device__ __forceinline__ bool forces_rows_staged(PairAcc& A, uint32_t i, bool 
                 const float4 a = stage[j], b = stage[kStageRecs + j];
                 pair_term_masked(A, pos, vel, pri, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w, h,
                                  s);
+            }
+            const uint32_t last = min(test.off + test.len, at + kStageRecs);
+            for (uint32_t k = max(test.off, at); OTHER && k < last; k++) {
+                const float4 a = stage[k - at], b = stage[kStageRecs + k - at];
+                pair_term(A, i, lo + k, pos, vel, pri, make_float3(a.x, a.y, a.z), make_float3(b.x, b.y, b.z), a.w, b.w,
+                          h, s, hhu);
             }
             wave_lds_sync();
             at += kStageRecs;
@@ -1146,7 +1225,6 @@ __device__ __forceinline__ bool forces_rows_staged(PairAcc& A, uint32_t i, bool 
             wave_lds_sync();
         }
     }
-    return true;
 }
 
 // A wavefront's slice in the force pass without masks: the records of the
@@ -1184,13 +1262,14 @@ __device__ __forceinline__ uint32_t near_bits(const float4& p, const ForceStage&
 // The row loop without masks for a whole wavefront (as forces_rows_staged):
 // each row's records are made from the sorted arrays while they are staged,
 // the lanes test their candidates there and then walk those within h.  Same
-// pairs, same order, same sums as forces_rowloop<false>.  False when the
-// wavefront has no usable runs (wave_cells): nothing is summed then.
+// pairs, same order, same sums as forces_rowloop<false>.
 //
 // Bound by VALU issue (the test and the walk); 250,047 particles take 48 us,
 // where every candidate's position, velocity and density read from memory
 // and a division per candidate took 97; 1,048,576 take 159, then 344.
-__device__ __forceinline__ bool forces_rows_tested(PairAcc& A, uint32_t i, bool active, const float4& pos,
+template <bool OTHER>
+__device__ __forceinline__ void forces_rows_tested(const WaveRuns& runs, const RowWalker& w, uint32_t cell, PairAcc& A,
+                                                   uint32_t i, bool active, const float4& pos,
                                                    const float4& vel, float pri, const float4* __restrict__ sp,
                                                    const float4* __restrict__ sv, const float2* __restrict__ rho_p,
                                                    const uint32_t* __restrict__ start,
@@ -1200,10 +1279,6 @@ __device__ __forceinline__ bool forces_rows_tested(PairAcc& A, uint32_t i, bool 
     const float h = cp.kernel_radius, s = cp.simulation_scale;
     const float hu = h / s, hhu = hu * hu, cut = h * h * 1.0001f;
     const uint32_t lane = __lane_id();
-    const RowWalker w = make_rows(pos, cp);
-    uint32_t cell;
-    WaveRuns runs;
-    if (!wave_cells(st.cells, st.temp(), 64u, w, cp, key_base, start, end, n, cell, runs)) return false;
     const float4 own = own_finite(pos);
     float3 p0, p1, v0, v1;
     float2 d0, d1;
@@ -1221,14 +1296,22 @@ __device__ __forceinline__ bool forces_rows_tested(PairAcc& A, uint32_t i, bool 
         st.vb[k] = make_float4(v.x, v.y, v.z, d.y * a);
     };
     auto fetch = [&](int row) {
-        const uint32_t len = runs.word(row), lo = runs.first(row);
+        const uint32_t len = runs.word(row) & kRunLength, lo = runs.first(row);
         if (lane < len) load(lo + lane, p0, v0, d0);
         if (lane + 64u < len) load(lo + lane + 64u, p1, v1, d1);
     };
     fetch(0);
     for (int row = 0; row < 9; row++) {
-        const uint32_t len = runs.word(row), lo = runs.first(row);  // the same on every lane
-        const LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
+        const uint32_t info = runs.word(row), len = info & kRunLength, lo = runs.first(row);  // the same on every lane
+        LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
+        if (OTHER && (info & (kRunLookup | kRunFar)))
+            r = other_row(row, active, pos, lo, cut, cp, key_base, start, end, n);
+        if (OTHER && (info & kRunFar)) {
+            if (r.len)
+                forces_row<false>(A, i, pos, vel, pri, lo + r.off, lo + r.off + r.len, 0ull, nullptr, sp, sv, rho_p, h, s,
+                                  hhu);
+            r.len = 0u;
+        }
         for (uint32_t at = 0u;;) {  // (a run rarely fills the slice)
             const uint32_t cnt = min(len - at, kStageRecs);
             if (at == 0u) {
@@ -1263,7 +1346,6 @@ __device__ __forceinline__ bool forces_rows_tested(PairAcc& A, uint32_t i, bool 
             if (at >= len) break;
         }
     }
-    return true;
 }
 
 // `v`; with LATER, by a pointer that the compiler takes for a new one, so that
@@ -1336,11 +1418,37 @@ __device__ __forceinline__ void forces_particle(uint32_t i, const float4* __rest
     // The staged row loop needs every lane of the wavefront, as the density
     // pass did; otherwise the rows are read from memory below.
     bool staged_rows = false;
-    if (MASKS && stage != nullptr && flat == nullptr && __ballot(1) == ~0ull)
-        staged_rows = forces_rows_staged(A, i, active, pos, vel, rho_p[il].y, n, cp0, masks, stage);
-    if (!MASKS && tested != nullptr && __ballot(1) == ~0ull)
-        staged_rows = forces_rows_tested(A, i, active, pos, vel, rho_p[il].y, sp, sv, rho_p, start, end, n, cp0,
-                                         key_base, *tested);
+    if (MASKS && stage != nullptr && flat == nullptr && __ballot(1) == ~0ull) {
+        const float pri = rho_p[il].y;
+        const uint32_t lane = __lane_id();
+        WaveRuns runs;
+        if (lane < 9u) {
+            const uint32_t* t = nbr_runs(masks, n) + (size_t)kRunWords * __builtin_amdgcn_readfirstlane(i >> 6) + lane;
+            runs.lo = t[0];
+            runs.info = t[9];
+        }
+        if (__ballot((runs.info & (kRunLong | kRunFar)) != 0u) == 0ull)
+            forces_rows_staged<false>(runs, A, i, active, pos, vel, pri, sp, sv, rho_p, start, end, n, cp0, key_base,
+                                      masks, stage);
+        else
+            forces_rows_staged<true>(runs, A, i, active, pos, vel, pri, sp, sv, rho_p, start, end, n, cp0, key_base,
+                                     masks, stage);
+        staged_rows = true;
+    }
+    if (!MASKS && tested != nullptr && __ballot(1) == ~0ull) {
+        const float pri = rho_p[il].y;
+        const RowWalker w = make_rows(pos, cp0);
+        uint32_t cell;
+        WaveRuns runs;
+        wave_cells(tested->cells, tested->temp(), 64u, w, cp0, key_base, start, end, n, cell, runs);
+        if (__builtin_expect(__ballot((runs.info & (kRunLookup | kRunFar)) != 0u) == 0ull, 1))
+            forces_rows_tested<false>(runs, w, cell, A, i, active, pos, vel, pri, sp, sv, rho_p, start, end, n, cp0, key_base,
+                                      *tested);
+        else
+            forces_rows_tested<true>(runs, w, cell, A, i, active, pos, vel, pri, sp, sv, rho_p, start, end, n, cp0, key_base,
+                                     *tested);
+        staged_rows = true;
+    }
     const fg_common_fluid_params& cp = later<INDIRECT>(cp0);
     const fg_kernels_cache& kc = later<INDIRECT>(kc0);
     if (i >= n) return;

@@ -249,9 +249,9 @@ __device__ __forceinline__ void density_particle_mixed(uint32_t i, const float4*
     const float hu = h / s, hhu = hu * hu, h2u = cp.kernel_radius_squared / s2;
     const float cut = hh * 1.0001f;
     const RowWalker w = make_rows(p, cp);
-    uint32_t cell, words = kRunGeneric;
+    uint32_t cell, words = 0u;
     WaveRuns runs;
-    const bool ok = wave_cells(st.cells, reinterpret_cast<uint32_t*>(st.hxy), 64u, w, cp, 0u, start, end, n, cell, runs);
+    wave_cells(st.cells, reinterpret_cast<uint32_t*>(st.hxy), 64u, w, cp, 0u, start, end, n, cell, runs);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(i >> 6);
     const bool table = n >= kRunMinParticles;
     uint16_t* offs = nbr_offs(masks, n) + (size_t)9 * 64 * wave + lane;
@@ -273,8 +273,8 @@ __device__ __forceinline__ void density_particle_mixed(uint32_t i, const float4*
     uint4 h0 = make_uint4(0u, 0u, 0u, 0u), h1 = h0;
     float3 p0 = make_float3(0.0f, 0.0f, 0.0f), p1 = p0;
     auto fetch = [&](int row) {
-        const uint32_t len = runs.word(row), lo = runs.first(row);
-        if (!ok || len > kMixedStage) return;
+        const uint32_t len = runs.word(row) & kRunLength, lo = runs.first(row);
+        if (len > kMixedStage) return;
         if (lane < len + 2u) h0 = hr[lo + lane];
         if (lane + 64u < len + 2u) h1 = hr[lo + lane + 64u];
         if (lane < len) p0 = ld_xyz(sp + lo + lane);
@@ -292,22 +292,16 @@ __device__ __forceinline__ void density_particle_mixed(uint32_t i, const float4*
 
     for (int row = 0; row < 9; row++) {
         const int dz = row / 3 - 1, dy = row % 3 - 1;
-        const uint32_t len = runs.word(row), lo = runs.first(row);  // the same on every lane
-        const bool staged = ok && len <= kMixedStage;
-        uint32_t rb = 0, re = 0;
-        bool has;
-        if (ok) {
-            const LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
-            has = r.len != 0u;
-            rb = lo + r.off;
-            re = rb + r.len;
-            if (table) {
-                offs[64 * row] = (uint16_t)r.off;
-                const uint32_t word = run_word(len, r.len);
-                words = (int)lane == row ? word : words;
-            }
-        } else {
-            has = active && row_range(w, dy, dz, cut, cp, 0u, start, end, n, rb, re);
+        const uint32_t info = runs.word(row), len = info & kRunLength, lo = runs.first(row);  // the same on every lane
+        const bool staged = len <= kMixedStage && !(info & kRunFar);
+        LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
+        if (info & (kRunLookup | kRunFar)) r = other_row(row, active, p, lo, cut, cp, 0u, start, end, n);
+        const bool has = r.len != 0u;
+        const uint32_t rb = lo + r.off, re = rb + r.len;
+        if (table) {
+            offs[64 * row] = (uint16_t)r.off;
+            const uint32_t word = run_word(info, r.len);
+            words = (int)lane == row ? word : words;
         }
         if (staged) {
             if (lane < len + 2u) put(lane, h0, p0, lane < len);

@@ -26,6 +26,7 @@
 #define __shared__ static
 #undef __launch_bounds__
 #define __launch_bounds__(...)
+#define amdgpu_waves_per_eu(...) unused
 #undef threadIdx
 #undef blockIdx
 #undef blockDim
