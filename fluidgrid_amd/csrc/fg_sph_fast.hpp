@@ -603,7 +603,7 @@ __device__ __forceinline__ unsigned long long density_row(const float4& p, const
 // first.  Candidates from `rest` on are no hits.
 //
 // SAME: h2u and hhu are the same value (always so at simulation scale 1), and
-// no r2 is NaN (stage_finite, own_finite).  Then h2u - r2 is positive exactly
+// no r2 is NaN (stage_number).  Then h2u - r2 is positive exactly
 // for the hits, the sum takes its positive part, and the hit bit is the sign
 // of r2 - hhu: 11 instructions a candidate.
 // Otherwise the compares, selects and shifts are written out: as selects of 0
@@ -660,14 +660,19 @@ __device__ __forceinline__ void density_group(const float4& p, const float2* __r
 }
 #pragma clang fp contract(fast)
 
-// A coordinate as it is staged, and a particle's own position: a NaN or an
-// infinity becomes a value that no hit can come of (the staged ones stay
-// within 3e38, the own x beyond them), and r2 is never NaN.
-__device__ __forceinline__ float stage_finite(float v) { return __builtin_amdgcn_fmed3f(v, -3.0e38f, 3.0e38f); }
-__device__ __forceinline__ float4 own_finite(float4 p) {
-    if (!(fabsf(p.x) <= 3.0e38f && fabsf(p.y) <= 3.0e38f && fabsf(p.z) <= 3.0e38f))
-        return make_float4(3.4e38f, 0.0f, 0.0f, p.w);
-    return p;
+// A coordinate as it is staged: a NaN becomes an infinity.  A particle whose
+// own position is finite (the others have no hits, and walk nothing) then gets
+// an infinite r2 from one that is not, never a NaN, and no hit.  (Written out:
+// of the builtin with these bounds the compiler makes two instructions, 1% of
+// the density pass.  A median of a NaN is the minimum of the other two, or of a
+// signalling one the last.)
+__device__ __forceinline__ float stage_number(float v) {
+    float r = v;
+    asm("v_med3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(-__builtin_inff()), "v"(__builtin_inff()));
+    return r;
+}
+__device__ __forceinline__ bool finite_position(const float4& p) {
+    return fabsf(p.x) < __builtin_inff() && fabsf(p.y) < __builtin_inff() && fabsf(p.z) < __builtin_inff();
 }
 
 // Part of a stencil row of the density pass from the staged run: cnt
@@ -725,7 +730,7 @@ __device__ __forceinline__ float density_rows_staged(uint32_t i, bool active, co
     WaveRuns runs;
     wave_cells(st.cells, st.temp(), 64u, w, cp, key_base, start, end, n, cell, runs);
     const bool same = __builtin_amdgcn_readfirstlane(__float_as_uint(h2u) == __float_as_uint(hhu) ? 1u : 0u) != 0u;
-    const float4 own = own_finite(p);
+    const bool walks = active && finite_position(p);
     uint16_t* offs = MASKS ? nbr_offs(masks, n) + (size_t)9 * 64 * wave + lane : nullptr;
     uint32_t words = 0u;
     unsigned long long msk = 0ull, last = 0ull;
@@ -738,14 +743,14 @@ __device__ __forceinline__ float density_rows_staged(uint32_t i, bool active, co
         if (lane + 64u < len) n1 = ld_xyz(q + 64);
     };
     auto put = [&](uint32_t k, const float3& q) {
-        st.xy[k] = make_float2(stage_finite(q.x), stage_finite(q.y));
-        st.z[k] = stage_finite(q.z);
+        st.xy[k] = make_float2(stage_number(q.x), stage_number(q.y));
+        st.z[k] = stage_number(q.z);
     };
     fetch(0);
     for (int row = 0; row < 9; row++) {
         const uint32_t info = runs.word(row), len = info & kRunLength, lo = runs.first(row);  // the same on every lane
-        LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
-        if (info & (kRunLookup | kRunFar)) r = other_row(row, active, p, lo, cut, cp, key_base, start, end, n);
+        LaneRow r = lane_row(st.cells, row, cell, walks, w, cut);
+        if (info & (kRunLookup | kRunFar)) r = other_row(row, walks, p, lo, cut, cp, key_base, start, end, n);
         if (table) {
             const uint32_t word = run_word(info, r.len);
             words = (int)lane == row ? word : words;
@@ -760,8 +765,8 @@ __device__ __forceinline__ float density_rows_staged(uint32_t i, bool active, co
         auto walk = [&](uint32_t at) {
             const uint32_t a = max(r.off, at), b = min(r.off + r.len, at + kStagePos);
             if (a < b) {
-                if (same) density_row_staged<MASKS, true>(own, st, a - at, b - a, a - r.off, h2u, hhu, acc, msk);
-                else density_row_staged<MASKS, false>(own, st, a - at, b - a, a - r.off, h2u, hhu, acc, msk);
+                if (same) density_row_staged<MASKS, true>(p, st, a - at, b - a, a - r.off, h2u, hhu, acc, msk);
+                else density_row_staged<MASKS, false>(p, st, a - at, b - a, a - r.off, h2u, hhu, acc, msk);
             }
         };
         for (uint32_t at = 0u;;) {  // (a run rarely fills the slice)
@@ -1279,7 +1284,7 @@ __device__ __forceinline__ void forces_rows_tested(const WaveRuns& runs, const R
     const float h = cp.kernel_radius, s = cp.simulation_scale;
     const float hu = h / s, hhu = hu * hu, cut = h * h * 1.0001f;
     const uint32_t lane = __lane_id();
-    const float4 own = own_finite(pos);
+    const bool walks = active && finite_position(pos);
     float3 p0, p1, v0, v1;
     float2 d0, d1;
     p0 = p1 = v0 = v1 = make_float3(0.0f, 0.0f, 0.0f);
@@ -1291,8 +1296,8 @@ __device__ __forceinline__ void forces_rows_tested(const WaveRuns& runs, const R
     };
     auto put = [&](uint32_t k, const float3& p, const float3& v, const float2& d) {
         const float a = 1.0f / d.x;
-        st.xy[k] = make_float2(stage_finite(p.x), stage_finite(p.y));
-        st.za[k] = make_float2(stage_finite(p.z), a);
+        st.xy[k] = make_float2(stage_number(p.x), stage_number(p.y));
+        st.za[k] = make_float2(stage_number(p.z), a);
         st.vb[k] = make_float4(v.x, v.y, v.z, d.y * a);
     };
     auto fetch = [&](int row) {
@@ -1303,9 +1308,9 @@ __device__ __forceinline__ void forces_rows_tested(const WaveRuns& runs, const R
     fetch(0);
     for (int row = 0; row < 9; row++) {
         const uint32_t info = runs.word(row), len = info & kRunLength, lo = runs.first(row);  // the same on every lane
-        LaneRow r = lane_row(st.cells, row, cell, active, w, cut);
+        LaneRow r = lane_row(st.cells, row, cell, walks, w, cut);
         if (OTHER && (info & (kRunLookup | kRunFar)))
-            r = other_row(row, active, pos, lo, cut, cp, key_base, start, end, n);
+            r = other_row(row, walks, pos, lo, cut, cp, key_base, start, end, n);
         if (OTHER && (info & kRunFar)) {
             if (r.len)
                 forces_row<false>(A, i, pos, vel, pri, lo + r.off, lo + r.off + r.len, 0ull, nullptr, sp, sv, rho_p, h, s,
@@ -1329,7 +1334,7 @@ __device__ __forceinline__ void forces_rows_tested(const WaveRuns& runs, const R
             const uint32_t b = min(r.off + r.len, at + kStageRecs);
             for (uint32_t a = max(r.off, at); a < b; a += 32u) {
                 const uint32_t c = min(b - a, 32u), k0 = a - at;
-                uint32_t word = near_bits(own, st, k0, c, hhu);
+                uint32_t word = near_bits(pos, st, k0, c, hhu);
                 const uint32_t self = i - (lo + a);  // the particle itself adds nothing
                 if (self < 32u) word &= ~(1u << self);
                 while (word) {

@@ -1,10 +1,10 @@
 """Rows that the density and force passes cannot stage as usual: more than 64
 candidates a lane (no mask), more than 127 particles in three cells (ranges
-looked up), and runs that are long for what the lanes read of them or longer
-than the longest (read from memory), next to ordinary ones in a wavefront.
-The flat schedules, which stage nothing, and the launchers without a neighbour
-buffer give the same bits; densities and velocities are the FP32 oracle's with
-the tolerances of test_gpu_sph.py."""
+looked up), runs that are long for what the lanes read of them or longer than
+the longest (read from memory), next to ordinary ones in a wavefront, and
+particles at non-finite positions.  The flat schedules, which stage nothing,
+and the launchers without a neighbour buffer give the same bits; densities and
+velocities are the FP32 oracle's with the tolerances of test_gpu_sph.py."""
 import numpy as np
 import pytest
 
@@ -36,6 +36,15 @@ def _pool_and_line(count):
     return _scene(np.concatenate([_block(count, (0.0, 0.05, 0.05), (0.999, 0.1, 0.1)), line, _block(300, 0.2, 0.999, 3)]))
 
 
+def _not_finite():
+    s = _scene(_block(3000, 0.1, 0.6))
+    rng = np.random.default_rng(5)
+    for value in (np.nan, np.inf, -np.inf, 3.2e38, -1e30):
+        for axis in range(3):
+            s.pos[rng.integers(0, s.n, 4), axis] = value
+    return s
+
+
 CASES = {
     "three_cells_64": lambda: _three_cells(64),
     "three_cells_65": lambda: _three_cells(65),
@@ -50,6 +59,7 @@ CASES = {
     "run_700": lambda: _pool_and_line(700),
     "run_2040": lambda: _pool_and_line(2040),
     "run_2060": lambda: _pool_and_line(2060),
+    "not_finite": _not_finite,
 }
 
 
@@ -86,6 +96,8 @@ def test_schedules_and_oracle(fglib, orc, which):
     rp, vel = run(0, 0)
     for other in (run(1, 1), run(1, 0), run(0, 1), run(0, 0, False)):
         assert np.array_equal(other[0], rp) and np.array_equal(other[1], vel)
+    if which == "not_finite":
+        return
     rp, vel = rp.view(np.float32), vel.view(np.float32)
     check_density(rp, orc.density(spos, start, end, s.fluid, s.common, s.kernels, s.key_mode), s)
     v_ref, acc, _ = orc.forces(spos, svel, rp, start, end, sp, s.fluid, s.common, s.kernels, s.key_mode,
