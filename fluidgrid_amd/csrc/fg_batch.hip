@@ -117,12 +117,9 @@ __global__ void __launch_bounds__(BS)
                     const float4* __restrict__ sp, const float4* __restrict__ sv, float2* __restrict__ rho_p,
                     const uint32_t* __restrict__ start, const uint32_t* __restrict__ end,
                     unsigned long long* __restrict__ masks, uint32_t n, WorkQueue q) {
-    __shared__ uint32_t s_rb[FLAT ? 9 * BS : 1];
-    __shared__ uint32_t s_re[FLAT ? 9 * BS : 1];
-    __shared__ WaveCells s_cells[FLAT ? BS / 64 : 1];
+    __shared__ FlatWave s_flat[FLAT ? BS / 64 : 1];
     __shared__ DensityStage s_stage[FLAT ? 1 : BS / 64];
     DensityStage* stage = FLAT ? nullptr : &s_stage[threadIdx.x / 64];
-    WaveCells* cells = &s_cells[FLAT ? threadIdx.x / 64 : 0];
     for_each_particle<BS, PERSIST>(q, n, [&](uint32_t i) {
         for_each_scene(scene_of[i], nscenes, [&](uint32_t s, auto whole) {
             const fg_scene_desc& d = scenes[s];
@@ -131,7 +128,7 @@ __global__ void __launch_bounds__(BS)
                 return;
             }
             // What lanes look up for each other holds within one scene's grid only.
-            FlatRanges fr{s_rb, s_re, (uint32_t)BS, (uint32_t)threadIdx.x, whole ? cells : nullptr};
+            const FlatRanges fr{&s_flat[FLAT ? threadIdx.x / 64 : 0], whole};
             density_particle<true>(i, sp, sv, rho_p, start, end, n, d.gasConstant, d.restDensity, d.mass, d.common,
                                    d.kernels, d.keyBase, masks, FLAT ? &fr : nullptr, whole ? stage : nullptr);
         });

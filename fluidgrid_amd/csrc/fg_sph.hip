@@ -358,12 +358,10 @@ __global__ void __launch_bounds__(BS)
                    const uint32_t* __restrict__ start,
                    const uint32_t* __restrict__ end, uint32_t n, float k, float rho0, float m,
                    fg_common_fluid_params cp, fg_kernels_cache kc, unsigned long long* __restrict__ masks) {
-    __shared__ uint32_t s_rb[9 * BS];
-    __shared__ uint32_t s_re[9 * BS];
-    __shared__ WaveCells s_cells[BS / 64];
+    __shared__ FlatWave s_flat[BS / 64];
     const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * BS + threadIdx.x;
     if ((i & ~63u) >= n) return;
-    FlatRanges fr{s_rb, s_re, (uint32_t)BS, (uint32_t)threadIdx.x, &s_cells[threadIdx.x / 64]};
+    const FlatRanges fr{&s_flat[threadIdx.x / 64], true};
     density_particle<MASKS>(i, sp, sv, rho_p, start, end, n, k, rho0, m, cp, kc, 0u, masks, &fr);
 }
 
