@@ -105,3 +105,35 @@ def test_schedules_and_oracle(fglib, orc, which):
     _, _, mag = orc.forces(spos, svel, rp.astype(np.float64), start, end, sp, s.fluid, s.common, s.kernels,
                            s.key_mode, f64=True, want_mag=True)
     check_velocity(vel, v_ref.astype(np.float64), acc, mag, sp, s.common.deltaTimeIntegration)
+
+
+@pytest.mark.parametrize("which", [k for k in CASES if k != "not_finite"])
+def test_mixed_precision_masks(fglib, orc, which):
+    """The mixed-precision density pass on the same rows: the FP32 pass's masks
+    bit for bit, and its densities within 4e-6: the roundings (2^-24 each) of
+    the FP32 pass's plain sum, of up to some thousand terms in random order,
+    whose square root they grow with; the compensated sum's are below them."""
+    s = CASES[which]()
+    L = fglib.load()
+    sk, sp, start, end, spos, _ = grid_cpu(orc, s)
+    fglib.init_params(s.common, s.kernels, s.key_mode, abi.MATH_FAST)
+    d = {k: fglib.DeviceArray.from_numpy(v) for k, v in dict(key=sk, sp=sp, pos=s.pos, vel=s.vel).items()}
+    nb = s.num_buckets
+    out = []
+    for precision in (abi.PRECISION_FP32, abi.PRECISION_MIXED):
+        fglib.check(L.fg_set_precision(precision))
+        try:
+            g = {k: fglib.DeviceArray((nb,), np.uint32) for k in ("start", "end")}
+            o = {k: fglib.DeviceArray((s.n, 4), np.float32) for k in ("pos", "vel")}
+            rp = fglib.DeviceArray.from_numpy(np.zeros((s.n, 2), np.float32))
+            nbr = fglib.DeviceArray((L.fg_neighbor_mask_bytes(s.n),), np.uint8)
+            fglib.check(L.fg_cell_offsets_pos_vel(g["start"].ptr, g["end"].ptr, d["key"].ptr, d["sp"].ptr, d["pos"].ptr,
+                                                  o["pos"].ptr, d["vel"].ptr, o["vel"].ptr, s.n, nb, 1, nbr.ptr))
+            fglib.check(L.fg_sph_density_nbr(o["pos"].ptr, o["vel"].ptr, rp.ptr, g["start"].ptr, g["end"].ptr, nbr.ptr,
+                                             s.n, s.fluid.gasConstant, s.fluid.restDensity, s.fluid.mass))
+            assert np.array_equal(o["pos"].numpy(), spos)
+            out.append((rp.numpy()[:, 0], fglib.download_raw(nbr.ptr, (9, s.n), np.uint64)))
+        finally:
+            L.fg_set_precision(abi.PRECISION_FP32)
+    assert np.array_equal(out[0][1], out[1][1])
+    assert np.all(np.abs(out[0][0] - out[1][0]) <= 4e-6 * out[0][0])
