@@ -31,8 +31,8 @@
 
 namespace fg {
 
-// A pass's workgroup: 2048 keys on 1024 lanes (2 a lane) up to kSmallTileMaxN
-// keys, 4096 on 512 (8 a lane) above.  A lane's keys are ranked one after
+// A pass's workgroup: 2048 keys on 1024 lanes (2 a lane) up to kShortMaxN keys,
+// on 512 (4 a lane) up to kSmallTileMaxN, 4096 on 512 (8 a lane) above.  A lane's keys are ranked one after
 // another through the wavefront's counts, so a short sort, whose workgroups
 // all run at once, takes the time of one chain and wants it short; a long one
 // wants long runs of each digit to write.  Measured per sort (us):
@@ -42,15 +42,21 @@ namespace fg {
 //   2,000,000 (22)       60.2    57.8     63.5          71.1    59.7     57.6
 //   3,000,000 (22)       73.9    73.2     81.1          78.8    71.0     74.8
 //   33,500,000 (27)     815.5   811.1    858.0         716.4   690.5    693.3
-// (8192 keys on 512 and 1024 lanes at 3,000,000: 87.0 and 94.9.)
+// (8192 keys on 512 and 1024 lanes at 3,000,000: 87.0 and 94.9.)  In a graph, 22
+// bits, 2048 keys on 512 and 1024 lanes: 400,000 keys 39.7 and 39.7, 800,000
+// 49.6 and 49.7, 1,200,000 55.3 and 64.1, 1,572,864 55.7 and 64.7 (a CU holds
+// two workgroups of 1024 lanes: past 512 workgroups the last wait for a place).
 constexpr int kSmallThreads = 1024, kSmallItems = 2;
+constexpr int kMidThreads = 512, kMidItems = 4;
+constexpr uint32_t kShortMaxN = 3u << 18;
+static_assert(kSmallThreads * kSmallItems == kMidThreads * kMidItems, "the same tiles");
 constexpr int kLargeThreads = 512, kLargeItems = 8;
 constexpr uint32_t kSmallTileMaxN = 3u << 19;
 // Up to this many tiles (131,072 keys) a pass adds up the tiles' counts of each
 // digit itself, and the launch of the scan is saved (us, with and without the
 // scan: 65,000 keys 20.5 and 16.8; 131,000 20.7 and 20.3; 262,000 21.3 and 27.2).
 constexpr uint32_t kSumMaxTiles = 64;
-static_assert(kSumMaxTiles * kSmallThreads * kSmallItems <= kSmallTileMaxN, "large tiles are scanned");
+static_assert(kSumMaxTiles * kSmallThreads * kSmallItems <= kShortMaxN, "the other shapes are scanned");
 constexpr int kSortThreads = 256;  // of the scan
 static bool sort_small(uint32_t n) { return n <= kSmallTileMaxN; }
 static uint32_t sort_tiles(uint32_t n) {
@@ -205,8 +211,8 @@ __global__ void __launch_bounds__(THREADS) k_sort_upsweep(const uint32_t* __rest
     }
 }
 
-// Exclusive scan of v over the workgroup's 256 lanes (in lane order);
-// *total receives the sum.  Uses s_w[kSortWaves].
+// Exclusive scan of v over the lanes of the workgroup's WAVES wavefronts (in
+// lane order); *total receives the sum.  Uses s_w[WAVES].
 template <int WAVES>
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_w, uint32_t* total) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -434,12 +440,15 @@ static int run_sort(uint32_t* keys, uint32_t* vals, uint32_t n, int keyBits, voi
     uint32_t* t2k = plan.passes >= 3 ? reinterpret_cast<uint32_t*>(w + L.t2k) : nullptr;
     uint32_t* t2v = plan.passes >= 3 ? reinterpret_cast<uint32_t*>(w + L.t2v) : nullptr;
     const uint32_t tiles = sort_tiles(n);
-    const bool small = sort_small(n), scanned = tiles > kSumMaxTiles;
-    const int threads = small ? kSmallThreads : kLargeThreads;
-    const auto upsweep = small ? k_sort_upsweep<kSmallThreads, kSmallItems> : k_sort_upsweep<kLargeThreads, kLargeItems>;
-    const auto pass = !scanned ? k_sort_pass<kSmallThreads, kSmallItems, false>
-                      : small  ? k_sort_pass<kSmallThreads, kSmallItems, true>
-                               : k_sort_pass<kLargeThreads, kLargeItems, true>;
+    const bool shortest = n <= kShortMaxN, small = sort_small(n), scanned = tiles > kSumMaxTiles;
+    const int threads = shortest ? kSmallThreads : small ? kMidThreads : kLargeThreads;
+    const auto upsweep = shortest ? k_sort_upsweep<kSmallThreads, kSmallItems>
+                         : small  ? k_sort_upsweep<kMidThreads, kMidItems>
+                                  : k_sort_upsweep<kLargeThreads, kLargeItems>;
+    const auto pass = !scanned   ? k_sort_pass<kSmallThreads, kSmallItems, false>
+                      : shortest ? k_sort_pass<kSmallThreads, kSmallItems, true>
+                      : small    ? k_sort_pass<kMidThreads, kMidItems, true>
+                                 : k_sort_pass<kLargeThreads, kLargeItems, true>;
 
     const uint32_t* src_k = keys;
     const uint32_t* src_v = vals;
