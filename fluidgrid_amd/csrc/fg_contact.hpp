@@ -344,6 +344,44 @@ __device__ __forceinline__ F3 contact_stencil_lanes(const float4& sp, const floa
     return f3(__shfl(total, (int)first), __shfl(total, (int)first + 1), __shfl(total, (int)first + 2));
 }
 
+// contact_stencil_lanes with a cell a lane: lane sub walks cells sub, sub + 8,
+// ... of the z, y, x stencil order by itself, each into a sum of its own from
+// zero, and after each round of eight the group adds the round's sums in cell
+// order, without those of zeros.  The same bits.  For a wide stencil, most of
+// whose cells are out of reach: a cell of eight spheres costs a lane of its own
+// less than a pass of the whole group.
+__device__ __forceinline__ F3 contact_stencil_apart(const float4& sp, const float4& sv, float sr,
+                                                    const float4* __restrict__ cpos, const float4* __restrict__ cvel,
+                                                    float cr, float ks, float kd, int3 rel,
+                                                    const uint32_t* __restrict__ start,
+                                                    const uint32_t* __restrict__ end, const GridDesc& g, float eps,
+                                                    uint32_t limit, uint32_t vlimit, uint32_t sub) {
+    F3 F = f3(0.0f, 0.0f, 0.0f);
+    const CellXYZ c = g.mode == FG_KEY_LINEAR ? grid_cell(sp.x, sp.y, sp.z, g) : CellXYZ{0, 0, 0};
+    const int nx = 2 * rel.x + 1, ny = 2 * rel.y + 1, cells = (rel.x | rel.y | rel.z) < 0 ? 0 : nx * ny * (2 * rel.z + 1);
+    const uint32_t first = __lane_id() & ~(kContactLanes - 1u);
+    for (int r0 = 0; r0 < cells; r0 += (int)kContactLanes) {
+        const int k = r0 + (int)sub;
+        F3 part = f3(0.0f, 0.0f, 0.0f);
+        if (k < cells) {
+            const uint32_t key = contact_key(sp, c, k % nx - rel.x, (k / nx) % ny - rel.y, k / (nx * ny) - rel.z, g);
+            if (key != kEmpty) {
+                const uint32_t s0 = start[key], e = end[key];
+                part = contact_range(sp, sv, sr, cr, cpos, cvel, s0, s0 != kEmpty ? e : 0u, ks, kd, false, false, 0, eps,
+                                     limit, vlimit);
+            }
+        }
+        const uint64_t nonzero = __ballot(part.x != 0.0f || part.y != 0.0f || part.z != 0.0f);
+        uint32_t m = (uint32_t)(nonzero >> first) & ((1u << kContactLanes) - 1u);
+        while (m) {
+            const int src = (int)first + __ffs((int)m) - 1;
+            m &= m - 1u;
+            F = add(F, f3(__shfl(part.x, src), __shfl(part.y, src), __shfl(part.z, src)));
+        }
+    }
+    return F;
+}
+
 // fluid_body_contact by a group of lanes (contact_stencil_lanes).
 __device__ __forceinline__ F3 contact_cells(const float4& pos, const float4& vel, const BodyContact& bc, uint32_t sub,
                                             ContactWave& W) {

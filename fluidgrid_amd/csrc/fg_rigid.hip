@@ -24,7 +24,8 @@ GridDesc fluid_grid_desc(const fg_common_fluid_params& cp, fg_float3 cs, uint32_
 // The body-force kernels take a group of kContactLanes lanes for each body
 // sphere (contact_stencil_lanes); sub is the lane's index in its group.
 
-// K_RigidBodySim.cu:66-99, for body sphere i.
+// K_RigidBodySim.cu:66-99, for body sphere i.  APART: contact_stencil_apart.
+template <bool APART>
 __device__ __forceinline__ void body_sphere_from_fluid(uint32_t i, const float4* __restrict__ rb_pos,
                                                        const float4* __restrict__ rb_vel,
                                                        const float4* __restrict__ rb_cm, float4* __restrict__ out_f,
@@ -40,8 +41,10 @@ __device__ __forceinline__ void body_sphere_from_fluid(uint32_t i, const float4*
     const bool ok = b >= 0 && (uint32_t)b < nbodies;
     const float4 vel = ok ? rb_vel[b] : make_float4(0, 0, 0, 0);
     const float4 cm = ok ? rb_cm[b] : make_float4(0, 0, 0, 0);
-    const F3 F = contact_stencil_lanes(pos, vel, radius, sph_pos, sph_vel, sph_radius, ks, kd, relation, sph_start,
-                                       sph_end, g, false, false, 0, 0.0001f, nsph, nsph, sub, contact);
+    const F3 F = APART ? contact_stencil_apart(pos, vel, radius, sph_pos, sph_vel, sph_radius, ks, kd, relation, sph_start,
+                                               sph_end, g, 0.0001f, nsph, nsph, sub)
+                       : contact_stencil_lanes(pos, vel, radius, sph_pos, sph_vel, sph_radius, ks, kd, relation, sph_start,
+                                               sph_end, g, false, false, 0, 0.0001f, nsph, nsph, sub, contact);
     if (sub != 0) return;
     out_f[i] = make_float4(F.x, F.y, F.z, (float)b);
     const float4 dir = make_float4(pos.x - cm.x, pos.y - cm.y, pos.z - cm.z, pos.w - cm.w);
@@ -50,6 +53,7 @@ __device__ __forceinline__ void body_sphere_from_fluid(uint32_t i, const float4*
     out_t[i] = t;
 }
 
+template <bool APART>
 __global__ void __launch_bounds__(256)
     k_body_forces_from_fluid(const float4* __restrict__ rb_pos, const float4* __restrict__ rb_vel,
                              const float4* __restrict__ rb_cm, float4* __restrict__ out_f, float4* __restrict__ out_t,
@@ -61,9 +65,9 @@ __global__ void __launch_bounds__(256)
     const uint32_t i = t / kContactLanes;
     __shared__ ContactWave s_contact[256 / 64];
     if (i >= m) return;  // the same for every lane of a group
-    body_sphere_from_fluid(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, radius, sph_pos, sph_vel,
-                                       sph_start, sph_end, nsph, sph_radius, g, relation, ks, kd, t % kContactLanes,
-                           s_contact[threadIdx.x / 64]);
+    body_sphere_from_fluid<APART>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, radius, sph_pos, sph_vel, sph_start,
+                                  sph_end, nsph, sph_radius, g, relation, ks, kd, t % kContactLanes,
+                                  s_contact[threadIdx.x / 64]);
 }
 
 __device__ __forceinline__ bool inside_box(const float4& p, const float4& lo, const float4& hi) {
@@ -107,13 +111,13 @@ __device__ __forceinline__ void body_sphere_from_bodies(uint32_t i, const float4
         }
         if (near)
             F = add(F, contact_stencil_lanes(pos, vel, radius, dyn.pos, dyn.vel, dyn.body_radius, dyn.ks, dyn.kd,
-                                                 dyn.relation, dyn.start, dyn.end, dyn.grid, true, true, b, dyn.eps,
-                                                 dyn.count, dyn.nvel, sub, contact));
+                                             dyn.relation, dyn.start, dyn.end, dyn.grid, true, true, b, dyn.eps,
+                                             dyn.count, dyn.nvel, sub, contact));
     }
     if (st.enabled && (st.aabb == nullptr || inside_box(pos, st.aabb[0], st.aabb[1])))
-        F = add(F, contact_stencil_lanes(pos, vel, radius, st.pos, nullptr, st.body_radius, st.ks, st.kd,
-                                             st.relation, st.start, st.end, st.grid, false, false, 0, st.eps,
-                                             st.count, 0u, sub, contact));
+        F = add(F, contact_stencil_lanes(pos, vel, radius, st.pos, nullptr, st.body_radius, st.ks, st.kd, st.relation,
+                                         st.start, st.end, st.grid, false, false, 0, st.eps, st.count, 0u, sub,
+                                         contact));
     if (sub != 0) return;
     const float4 dir = make_float4(pos.x - cm.x, pos.y - cm.y, pos.z - cm.z, pos.w - cm.w);
     const float4 t = vec3_cross(dir, make_float4(F.x, F.y, F.z, 0.0f));
@@ -137,8 +141,8 @@ __global__ void __launch_bounds__(256)
     const uint32_t i = t / kContactLanes;
     __shared__ ContactWave s_contact[256 / 64];
     if (i >= m) return;  // the same for every lane of a group
-    body_sphere_from_bodies<ACCUM>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, radius, dyn, st,
-                                               body_bounds, 0u, nbounds, t % kContactLanes, s_contact[threadIdx.x / 64]);
+    body_sphere_from_bodies<ACCUM>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, radius, dyn, st, body_bounds, 0u,
+                                   nbounds, t % kContactLanes, s_contact[threadIdx.x / 64]);
 }
 
 // K_RigidBodySim.cu:102-111
@@ -490,9 +494,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
     const int b = f2i_sat(rb_pos[i].w);
     if (b < 0 || (uint32_t)b >= nbodies) return;
     const BatchBodyScene& d = scenes[body_scene[b]];
-    body_sphere_from_fluid(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, d.sphere_radius, sph_pos,
-                                       sph_vel, sph_start, sph_end, nsph, d.fluid_radius, d.fluid, d.rb_to_fluid, d.ks,
-                                       d.kd, t % kContactLanes, s_contact[threadIdx.x / 64]);
+    body_sphere_from_fluid<false>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, d.sphere_radius, sph_pos, sph_vel,
+                                  sph_start, sph_end, nsph, d.fluid_radius, d.fluid, d.rb_to_fluid, d.ks, d.kd,
+                                  t % kContactLanes, s_contact[threadIdx.x / 64]);
 }
 
 // Scenes with one body have no body-body pass (the single-fluid simulator
@@ -516,9 +520,8 @@ __global__ void __launch_bounds__(256)
     dyn.eps = 0.001f;
     dyn.aabb = nullptr;
     const BodyContact st{};
-    body_sphere_from_bodies<true>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, d.sphere_radius, dyn,
-                                              st, body_bounds, d.body_begin, d.body_end, t % kContactLanes,
-                                  s_contact[threadIdx.x / 64]);
+    body_sphere_from_bodies<true>(i, rb_pos, rb_vel, rb_cm, out_f, out_t, nbodies, d.sphere_radius, dyn, st, body_bounds,
+                                  d.body_begin, d.body_end, t % kContactLanes, s_contact[threadIdx.x / 64]);
 }
 
 __global__ void k_bintegrate_rb(float4* __restrict__ pos, const float* __restrict__ mass, float4* __restrict__ vel,
@@ -749,7 +752,15 @@ int fg_body_forces_from_fluid(fg_float4* spheres, fg_float4* bodyVelocities, fg_
     const State& st = state();
     // The fluid grid is walked with the key function it was built with.
     const GridDesc g = fluid_grid_desc(st.common, fluidCellSize, fluidNumBuckets, st.key_mode);
-    hipLaunchKernelGGL(k_body_forces_from_fluid, dim3(grid_for((uint64_t)numSpheres * kContactLanes, 256)), dim3(256), 0, st.stream,
+    // Wide stencils with a cell a lane.  LINEAR keys, 19,936 body spheres in
+    // 1M particles: 125 cells 62.4 -> 50.0 us, 343 cells 160 -> 107; 45 cells
+    // 28.2 -> 27.7 and 28.0 -> 30.0 by the axis, so those stay with the group.
+    // XOR keys, where colliding cells fill more of a group's passes: 125 cells
+    // 109.5 -> 116.8, 343 cells 298.5 -> 280.
+    const double cells = (2.0 * relation.x + 1.0) * (2.0 * relation.y + 1.0) * (2.0 * relation.z + 1.0);
+    const bool apart = cells > (st.key_mode == FG_KEY_LINEAR ? 45.0 : 125.0);
+    hipLaunchKernelGGL((apart ? k_body_forces_from_fluid<true> : k_body_forces_from_fluid<false>),
+                       dim3(grid_for((uint64_t)numSpheres * kContactLanes, 256)), dim3(256), 0, st.stream,
                        FG_F4(spheres), FG_F4(bodyVelocities), FG_F4(bodyCM), FG_F4(outForces), FG_F4(outTorques),
                        numSpheres, numBodies, radius, FG_F4(fluidOrderedPositions), FG_F4(fluidOrderedVelocities),
                        fluidGridStart, fluidGridEnd, numFluid, fluidRadius, g,
