@@ -83,8 +83,9 @@ __device__ __forceinline__ bool stencil_bucket(const float4& p, const CellXYZ& c
 // 972 and 1,115.
 __device__ __forceinline__ float ref_cut(float h) { return rn_mul(rn_mul(h, h), 0x1.00001p+0f); }
 
-// x^3 (powf(x, 3.0f) in the reference), rounded once from 64 bits: x * x is
-// exact there.
+// x^3 (powf(x, 3.0f) in the reference) by way of 64 bits: x * x is exact
+// there, the cube is rounded to 53 bits and then to 24, just over half a unit
+// in the last place.
 __device__ __forceinline__ float ref_cube(float x) {
     const double d = (double)x;
     return (float)(d * d * d);
@@ -406,8 +407,9 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(8)))
 // The coupled masked force pass with body contact deferred: a particle
 // inside a body grid's expanded bounds stores its pair sum and joins a list
 // (forces_particle with DEFER); the others finish here without the contact
-// walk, which leaves the wavefronts that never meet a body free of it.  Row
-// loop with row-ahead loads, as k_forces_fast<true, true>.
+// walk, which leaves the wavefronts that never meet a body free of it.  The
+// row loop is that of k_forces_fast<true, true>: each row's records staged in
+// LDS a row ahead, at the runs that the density pass left (with `runs`).
 template <int BS>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
     k_forces_deferred(const float4* __restrict__ sp, const float4* __restrict__ sv, const float2* __restrict__ rho_p,

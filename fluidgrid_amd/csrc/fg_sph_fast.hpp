@@ -503,7 +503,7 @@ __device__ __forceinline__ uint32_t run_word(uint32_t word, uint32_t len) {
     return word;
 }
 
-// Wavefront w's runs and its lanes' offsets (off(row)), for the force pass.
+// Wavefront w's runs (first index and word of each row), for the force pass.
 __device__ __forceinline__ void store_runs(const WaveRuns& runs, uint32_t w, unsigned long long* masks, uint32_t n) {
     if (__lane_id() < 9u) {
         uint32_t* t = nbr_runs(masks, n) + (size_t)kRunWords * w + __lane_id();
@@ -553,12 +553,6 @@ __device__ __forceinline__ void store_density(uint32_t i, float rho, float k, fl
     if (rec) store_record(i, rp, p, v, rec);
 }
 #pragma clang fp contract(fast)
-
-// xyz of a position staged in LDS (a 16-byte read; w unused).
-__device__ __forceinline__ float3 ld_xyz_lds(const float4* p) {
-    const float4 q = *p;
-    return make_float3(q.x, q.y, q.z);
-}
 
 // One stencil row of the density pass: the len candidates pp[0, len) of the
 // sorted positions, in groups of four in sorted order (a short last group
@@ -708,10 +702,12 @@ __device__ __forceinline__ void density_row_staged(const float4& p, const Densit
 // is walked.  Same candidates, same order, same sums and masks as the row
 // loop of density_particle.
 //
-// Bound by VALU issue: about 4,700 instructions a wavefront, 3,800 of them in
-// the walks (65 groups of four candidates, which its longest lane per row
-// sets); 8,388,608 particles take 702 us against 767 with per-lane lookups
-// row by row and whole positions in LDS, 1,048,576 take 104 against 111.
+// Bound by VALU issue: 4,724 instructions a wavefront, 3,800 of them in the
+// walks (65 groups of four candidates, which its longest lane per row sets);
+// 30% of a wavefront's time is waiting.  8,388,608 particles take 0.83 ms
+// against 0.87 with per-lane lookups row by row and whole positions in LDS,
+// 1,048,576 at the start of a dam break 99.8 us against 98.5, and on cells of
+// 2 h 330 against 467.
 template <bool MASKS>
 __device__ __forceinline__ float density_rows_staged(uint32_t i, bool active, const float4& p,
                                                     const float4* __restrict__ sp,
@@ -1144,10 +1140,11 @@ __device__ __forceinline__ void forces_rowloop(PairAcc& A, uint32_t i, const flo
 // they are staged) and for one without a run.  Same pairs, same order, same
 // sums as forces_rowloop<true>.
 //
-// Bound by VALU issue (3,300 instructions a wavefront) and by the records,
-// which come from past the L2 cache about three times at 8,388,608 particles:
-// 579 us there against 701 with the cells looked up again and a min/max
-// reduction per row; 84 against 98 us at 1,048,576.
+// Bound by VALU issue (3,342 instructions a wavefront) and by the records,
+// which come from past the L2 cache about three times at 8,388,608 particles
+// (45% of a wavefront's time is waiting): 0.61 ms there against 0.76 with the
+// cells looked up again and a min/max reduction per row; 80 against 94 us at
+// 1,048,576.
 //
 // OTHER: with rows that lanes look up (kRunLong, kRunFar), a loop of its own,
 // without loads ahead, so that the usual one keeps its registers (in one loop
