@@ -1141,7 +1141,7 @@ __device__ __forceinline__ void forces_rowloop(PairAcc& A, uint32_t i, const flo
 // sums as forces_rowloop<true>.
 //
 // Bound by VALU issue (3,342 instructions a wavefront) and by the records,
-// which come from past the L2 cache about three times at 8,388,608 particles
+// which come from past the L2 cache three to four times at 8,388,608 particles
 // (45% of a wavefront's time is waiting): 0.61 ms there against 0.76 with the
 // cells looked up again and a min/max reduction per row; 80 against 94 us at
 // 1,048,576.
